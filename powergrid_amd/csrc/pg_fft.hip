@@ -13,11 +13,14 @@
 //   adjoint: [IFFT_x (keep the Nx cropped outputs)]        -> T   (3-D: IFFT_z first)
 //            [IFFT_y + crop + deapod + WoH + sum_l + conj(S)] -> image
 // Power-of-two lengths 16..1024 use the register-resident two-level FFT of
-// pg_fftreg.h (one LDS exchange per line); other lengths whose prime factors
-// are at most 13 use a mixed radix-4/2/3/5/7/11/13 Stockham FFT staged in LDS.
+// pg_fftreg.h (one LDS exchange per line), the other lengths listed in
+// pg_fftmix.h (up to 480, gridos 2) the same with register DFTs of any factor
+// up to 28; what remains of the lengths whose prime factors are at most 13
+// uses a mixed radix-4/2/3/5/7/11/13 Stockham FFT staged in LDS.
 #include "pg_internal.h"
 #include "pg_gnufft.h"
 #include "pg_fftreg.h"
+#include "pg_fftmix.h"
 
 namespace {
 
@@ -1456,7 +1459,8 @@ void adj_post_reg_n(const pg::Gnufft& G, const float2* tbuf, const pgk::WeightAr
     default: CALL(1024); break; \
     }
 
-// strided line FFT: register kernel for power-of-two lengths, Stockham otherwise
+// strided line FFT: register kernels for powers of two and the lengths of
+// pg_fftmix.h, Stockham otherwise
 template <int SIGN>
 void line_fft_any(const float2* src, float2* dst, long long inner_n, long long src_os,
                   long long dst_os, int nin, int in_off, int nout, int out_off, unsigned outer,
@@ -1469,6 +1473,8 @@ void line_fft_any(const float2* src, float2* dst, long long inner_n, long long s
 #undef PG_CALL_LINE
         return;
     }
+    if (pgm::line(SIGN, src, dst, inner_n, src_os, dst_os, nin, in_off, nout, out_off, outer, p, s))
+        return;
     const int rpw = pick_rpw(p.n);
     const size_t lds = sizeof(float2) * 2 * rpw * (p.n + 1);
     hipLaunchKernelGGL(k_line_fft<SIGN>, dim3((unsigned)((inner_n + rpw - 1) / rpw), outer),
@@ -1597,6 +1603,8 @@ void launch_fwd_prep_fft(const pg::Gnufft& G, const float2* img, long long img_c
 #define PG_CALL_COL(NN) fwd_col_reg_n<NN>(G, img, img_cstride, w, B, L, tbuf, s)
         PG_REG_SWITCH(g.Gy, PG_CALL_COL)
 #undef PG_CALL_COL
+    } else if (pgm::col_ok(g.Gy, g.Ny, g.offY)) {
+        pgm::fwd_col(img, img_cstride, w.S, w.Wo, G.dap, ncol, B, L, G.py, tbuf, s);
     } else {
         const int cpw = pick_cpw(g.Gy, g.Ny);
         const size_t lds1 = sizeof(float2) * 2 * cpw * (g.Gy + 1);
@@ -1706,9 +1714,13 @@ void launch_adj_fft_post(const pg::Gnufft& G, float2* grids, float2* tbuf, float
 #undef PG_CALL_POST
         return;
     }
+    const int ncol = g.Nx * g.Nz;
+    if (pgm::col_ok(g.Gy, g.Ny, g.offY)) {
+        pgm::adj_post(tbuf, w.S, w.WoH, G.dap, ncol, nc, L, G.py, out, out_cstride, s);
+        return;
+    }
     const int cpw = pick_cpw(g.Gy, g.Ny);
     const size_t lds1 = sizeof(float2) * 2 * cpw * (g.Gy + 1);
-    const int ncol = g.Nx * g.Nz;
     hipLaunchKernelGGL(k_adj_colfft_post, dim3((ncol + cpw - 1) / cpw, nc), dim3(256), lds1, s,
                        tbuf, w.S, w.WoH, G.dfx, G.dfy, G.dfz, G.inv_osd, g.Nx, g.Ny, g.Nz, g.offY, L,
                        cpw, pg::fft_args(G.py), out, out_cstride);
