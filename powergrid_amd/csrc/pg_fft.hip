@@ -1415,15 +1415,18 @@ void line_reg_n(const float2* src, float2* dst, long long inner_n, long long src
 {
     constexpr int R1 = pgf::Split<N>::R1, R2 = pgf::Split<N>::R2;
     constexpr int LPB = line_lpb<R1, R2>();
-    const dim3 grid((unsigned)((inner_n + LPB - 1) / LPB), outer), block(LPB * R2);
-    if (2 * nin == N && in_off % N == 3 * N / 4)
-        hipLaunchKernelGGL((k_line_reg<R1, R2, SIGN, true>), grid, block, 0, s, src, dst, inner_n,
-                           src_os, dst_os, nin, in_off % N, nout, out_off % N,
-                           (const float2*)p.tw);
-    else
-        hipLaunchKernelGGL((k_line_reg<R1, R2, SIGN, false>), grid, block, 0, s, src, dst, inner_n,
-                           src_os, dst_os, nin, in_off % N, nout, out_off % N,
-                           (const float2*)p.tw);
+    const bool half = 2 * nin == N && in_off % N == 3 * N / 4;
+    pg::grid_y_runs(outer, [&](long long o, unsigned n) {
+        const dim3 grid((unsigned)((inner_n + LPB - 1) / LPB), n), block(LPB * R2);
+        if (half)
+            hipLaunchKernelGGL((k_line_reg<R1, R2, SIGN, true>), grid, block, 0, s,
+                               src + o * src_os, dst + o * dst_os, inner_n, src_os, dst_os, nin,
+                               in_off % N, nout, out_off % N, (const float2*)p.tw);
+        else
+            hipLaunchKernelGGL((k_line_reg<R1, R2, SIGN, false>), grid, block, 0, s,
+                               src + o * src_os, dst + o * dst_os, inner_n, src_os, dst_os, nin,
+                               in_off % N, nout, out_off % N, (const float2*)p.tw);
+    });
 }
 
 template <int N>
@@ -1494,16 +1497,17 @@ void fwd_col_planes_n(const pg::Gnufft& G, const float2* planes, int Bp, float2*
     const int waves = (g.Nx + lpw - 1) / lpw;
     const int wpb = (waves * (long long)Bp >= 1024) ? 4 : 1;
     const bool half = 2 * g.Ny == N && (g.offY + N / 2) % N == 3 * N / 4;
-    const dim3 grid((waves + wpb - 1) / wpb, Bp), block(64 * wpb);
     const long long nxy = (long long)g.Nx * g.Ny;
-    if (half)
-        hipLaunchKernelGGL((k_fwd_col_reg<R1, R2, 4, true>), grid, block, 0, s, planes, nxy,
-                           (const float2*)nullptr, (const float2*)nullptr, (const float*)nullptr,
-                           g.Nx, g.Ny, 1, g.offY, 1, (const float2*)G.py.tw, T);
-    else
-        hipLaunchKernelGGL((k_fwd_col_reg<R1, R2, 4, false>), grid, block, 0, s, planes, nxy,
-                           (const float2*)nullptr, (const float2*)nullptr, (const float*)nullptr,
-                           g.Nx, g.Ny, 1, g.offY, 1, (const float2*)G.py.tw, T);
+    pg::grid_y_runs(Bp, [&](long long o, unsigned n) {
+        const dim3 grid((waves + wpb - 1) / wpb, n), block(64 * wpb);
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, block, 0, s, planes + o * nxy, nxy,
+                               (const float2*)nullptr, (const float2*)nullptr,
+                               (const float*)nullptr, g.Nx, g.Ny, 1, g.offY, 1,
+                               (const float2*)G.py.tw, T + o * g.Nx * N);
+        };
+        half ? launch(k_fwd_col_reg<R1, R2, 4, true>) : launch(k_fwd_col_reg<R1, R2, 4, false>);
+    });
 }
 
 template <int N>
@@ -1512,9 +1516,12 @@ void col_ifft_crop_n(const pg::Gnufft& G, const float2* T, int Bp, float2* plane
     constexpr int R1 = pgf::Split<N>::R1, R2 = pgf::Split<N>::R2;
     const pg::Geometry& g = G.geo;
     const int lpw = 64 / R2;
-    const dim3 grid((g.Nx + 4 * lpw - 1) / (4 * lpw), Bp), block(256);
-    hipLaunchKernelGGL((k_col_ifft_crop<R1, R2>), grid, block, 0, s, T, g.Nx, g.Ny, g.offY,
-                       (const float2*)G.py.tw, planes, (long long)g.Nx * g.Ny);
+    const long long nxy = (long long)g.Nx * g.Ny;
+    pg::grid_y_runs(Bp, [&](long long o, unsigned n) {
+        hipLaunchKernelGGL((k_col_ifft_crop<R1, R2>), dim3((g.Nx + 4 * lpw - 1) / (4 * lpw), n),
+                           dim3(256), 0, s, T + o * g.Nx * N, g.Nx, g.Ny, g.offY,
+                           (const float2*)G.py.tw, planes + o * nxy, nxy);
+    });
 }
 
 }  // namespace
@@ -1532,7 +1539,7 @@ void launch_fwd_prep_fft(const pg::Gnufft& G, const float2* img, long long img_c
         // z-class planes: the z stage (maps, phases, deapodization, z FFT and
         // z taps) into B*nzc image-sized planes (tbuf2), their y FFT (tbuf)
         // and x FFT (grids, plane (k*B + b))
-        PG_REQUIRE(zclass_active(G, B) && reg_len(g.Gy), PG_ERR_STATE,
+        PG_REQUIRE(zclass_active(G, B), PG_ERR_STATE,
                    "no z-class planes for this batch");
         const int Bp = B * G.nzc;
         const int nxy = g.Nx * g.Ny;
@@ -1591,9 +1598,13 @@ void launch_fwd_prep_fft(const pg::Gnufft& G, const float2* img, long long img_c
                                tbuf2);
         }
 #undef PG_ZSF
+        if (reg_len(g.Gy)) {
 #define PG_CALL_COLP(NN) fwd_col_planes_n<NN>(G, tbuf2, Bp, tbuf, s)
-        PG_REG_SWITCH(g.Gy, PG_CALL_COLP)
+            PG_REG_SWITCH(g.Gy, PG_CALL_COLP)
 #undef PG_CALL_COLP
+        } else {
+            pgm::fwd_col(tbuf2, nxy, nullptr, nullptr, nullptr, g.Nx, Bp, 1, G.py, tbuf, s);
+        }
         line_fft_any<-1>(tbuf, grids, (long long)g.Gy, (long long)g.Nx * g.Gy,
                          (long long)g.Gx * g.Gy, g.Nx, (g.offX + g.Gx / 2) % g.Gx, g.Gx, g.Gx / 2,
                          (unsigned)Bp, G.px, s);
@@ -1635,7 +1646,7 @@ void launch_adj_fft_post(const pg::Gnufft& G, float2* grids, float2* tbuf, float
         // z-class planes: x IFFT of every plane keeping the Nx cropped
         // columns (tbuf), y IFFT and crop (tbuf2: B*nzc image-sized planes),
         // then the z stage into the coils' partial images
-        PG_REQUIRE(zclass_active(G, B) && reg_len(g.Gy), PG_ERR_STATE,
+        PG_REQUIRE(zclass_active(G, B), PG_ERR_STATE,
                    "no z-class planes for this batch");
         const int Bp = B * G.nzc;
         const int nxy = g.Nx * g.Ny;
@@ -1666,8 +1677,8 @@ void launch_adj_fft_post(const pg::Gnufft& G, float2* grids, float2* tbuf, float
 #undef PG_YZM
             return;
         }
-        if (g_zfuse.load(std::memory_order_relaxed) && half && g.Ny >= 64 && g.Ny <= 256 &&
-            g.Nz <= 32 * zgroups && fused_lds <= 64 * 1024) {
+        if (reg_len(g.Gy) && g_zfuse.load(std::memory_order_relaxed) && half && g.Ny >= 64 &&
+            g.Ny <= 256 && g.Nz <= 32 * zgroups && fused_lds <= 64 * 1024) {
             // y IFFT, crop and the z stage in one kernel
             const int zw = (g.Nz + zgroups - 1) / zgroups;
             const unsigned nb = (unsigned)((long long)nc * g.Nx);
@@ -1689,9 +1700,13 @@ void launch_adj_fft_post(const pg::Gnufft& G, float2* grids, float2* tbuf, float
 #undef PG_YZA
             return;
         }
+        if (reg_len(g.Gy)) {
 #define PG_CALL_CROP(NN) col_ifft_crop_n<NN>(G, tbuf, Bp, tbuf2, s)
-        PG_REG_SWITCH(g.Gy, PG_CALL_CROP)
+            PG_REG_SWITCH(g.Gy, PG_CALL_CROP)
 #undef PG_CALL_CROP
+        } else {
+            pgm::adj_post(tbuf, nullptr, nullptr, nullptr, g.Nx, Bp, 1, G.py, tbuf2, nxy, s);
+        }
         const int zg = (g.Nz + 7) / 8;
         const size_t lds = sizeof(float2) * (size_t)G.nzc * g.Nz;
         hipLaunchKernelGGL(k_zstage_adj, dim3((nxy + 63) / 64, nc), dim3(64 * zg), lds, s, tbuf2,

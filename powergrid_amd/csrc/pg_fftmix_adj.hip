@@ -118,9 +118,13 @@ void launch(const float2* T, const float2* S, const float2* WoH, const float* da
     const int rounds = (L + NL - 1) / NL;
     const int ng = (L + rounds - 1) / rounds;
     const int npc = std::max(1, std::min(NL / ng, 128 / (ng * TL)));
-    hipLaunchKernelGGL((k_adj_post_mix<R1, R2>), dim3((ncol + npc - 1) / npc, nc),
-                       dim3(TL * npc * ng), 0, s, T, S, WoH, dap, ncol, L, npc, ng, tw, out,
-                       out_cstride);
+    // (planes of a stack: there may be more than a grid dimension holds)
+    pg::grid_y_runs(nc, [&](long long o, unsigned n) {
+        hipLaunchKernelGGL((k_adj_post_mix<R1, R2>), dim3((ncol + npc - 1) / npc, n),
+                           dim3(TL * npc * ng), 0, s, T + o * L * ncol * (R1 * R2),
+                           S ? S + o * ncol * (R1 * R2 / 2) : S, WoH, dap, ncol, L, npc, ng, tw,
+                           out + o * out_cstride, out_cstride);
+    });
 }
 
 }  // namespace

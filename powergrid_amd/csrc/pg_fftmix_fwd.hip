@@ -87,6 +87,15 @@ void launch(const float2* img, long long img_cstride, const float2* S, const flo
     // fewer columns per block where the launch would leave compute units idle
     int lpb = col_lpb<R1, R2>();
     while (lpb > 2 && (long long)((ncol + lpb - 1) / lpb) * B < 512) lpb = (lpb + 1) / 2;
+    if (L == 1 && !S) {
+        // (planes of a stack: there may be more than a grid dimension holds)
+        pg::grid_y_runs(B, [&](long long o, unsigned n) {
+            hipLaunchKernelGGL((k_fwd_col_mix<R1, R2>), dim3((ncol + lpb - 1) / lpb, n),
+                               dim3(TL * lpb), 0, s, img + o * img_cstride, img_cstride, S, Wo, dap,
+                               ncol, L, tw, T + o * ncol * (R1 * R2));
+        });
+        return;
+    }
     hipLaunchKernelGGL((k_fwd_col_mix<R1, R2>), dim3((ncol + lpb - 1) / lpb, B), dim3(TL * lpb), 0,
                        s, img, img_cstride, S, Wo, dap, ncol, L, tw, T);
 }

@@ -66,10 +66,12 @@ void launch(const float2* src, float2* dst, long long inner_n, long long src_os,
             unsigned outer, const float2* tw, hipStream_t s)
 {
     constexpr int LPB = lpb<R1 * R2>();
-    hipLaunchKernelGGL((k_line_mix<R1, R2, SIGN>),
-                       dim3((unsigned)((inner_n + LPB - 1) / LPB), outer),
-                       dim3(pgm::line_threads<R1, R2>() * LPB), 0, s, src, dst, inner_n, src_os,
-                       dst_os, tw);
+    pg::grid_y_runs(outer, [&](long long o, unsigned n) {
+        hipLaunchKernelGGL((k_line_mix<R1, R2, SIGN>),
+                           dim3((unsigned)((inner_n + LPB - 1) / LPB), n),
+                           dim3(pgm::line_threads<R1, R2>() * LPB), 0, s, src + o * src_os,
+                           dst + o * dst_os, inner_n, src_os, dst_os, tw);
+    });
 }
 
 }  // namespace

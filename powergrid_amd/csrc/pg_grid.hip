@@ -1586,7 +1586,7 @@ int spread_row_floats(const pg::Gnufft& G, int nc, int L, const float* AA, const
 
 bool zclass_active(const pg::Gnufft& G, int B)
 {
-    return G.nzc > 0 && B >= 16 && (long long)B * G.nzc <= 65535;
+    return G.nzc > 0 && B >= 16 && (long long)B * G.nzc < (1LL << 31);
 }
 
 bool interp_lds_possible(const pg::Gnufft& G, int L, bool aa)

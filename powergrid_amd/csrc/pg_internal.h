@@ -95,6 +95,15 @@ constexpr int kSpreadTZ = 4;   // tile extent along z (3-D)
 
 struct Gnufft;
 
+// launch(first, count) over [0, n) in runs that fit one grid dimension (y, z)
+constexpr unsigned kMaxGridY = 65535;
+template <class F>
+inline void grid_y_runs(long long n, F launch)
+{
+    for (long long o = 0; o < n; o += kMaxGridY)
+        launch(o, (unsigned)(n - o < kMaxGridY ? n - o : kMaxGridY));
+}
+
 }  // namespace pg
 
 // --------------------------------------------------- kernel launchers ----

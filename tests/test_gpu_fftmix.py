@@ -53,3 +53,29 @@ def test_every_length(orc, n):
 @pytest.mark.parametrize("N,Nz", [(12, 10), (18, 14), (20, 6), (26, 8)])
 def test_three_dimensions(orc, N, Nz):
     _check(orc, N, Nz, 83, 3, 2, N)
+
+
+# image sizes of both kinds of y FFT, Nz up to and past the matrix-core z
+# stage's 32; the last has more planes (512 coils x 16 segments x 10) than one
+# grid dimension holds
+@pytest.mark.parametrize("N,Nz,nc,L", [(12, 8, 8, 2), (20, 36, 4, 4), (8, 10, 5, 4),
+                                       (10, 10, 512, 16)])
+def test_stack_planes(orc, N, Nz, nc, L):
+    import powergrid_amd as P
+    rng = np.random.default_rng(N)
+    m = 7
+    kx, ky = (rng.uniform(-N / 2, N / 2 - 1e-2, m * Nz).astype(np.float32) for _ in range(2))
+    kz = np.repeat(np.arange(Nz) - Nz / 2.0, m).astype(np.float32)
+    M, n = m * Nz, N * N * Nz
+    t = np.linspace(1e-3, 9e-3, M).astype(np.float32)
+    fm = rng.uniform(-300, 300, n).astype(np.float32)
+    sens = (rng.standard_normal((nc, n)) + 1j * rng.standard_normal((nc, n))).astype(np.complex64)
+    x = (rng.standard_normal(n) + 1j * rng.standard_normal(n)).astype(np.complex64)
+    y = (rng.standard_normal(nc * M) + 1j * rng.standard_normal(nc * M)).astype(np.complex64)
+    Gg = P.Gnufft(M, 2.0, N, N, Nz, kx, ky, kz)
+    assert P.zclasses(Gg) == Nz
+    A = P.SENSE(P.TimeSegmentation(Gg, fm, t, M, n, L), sens, M, n, nc)
+    G = orc.Gnufft(M, 2.0, N, N, Nz, kx, ky, kz, prec="d")
+    O = orc.SENSE(orc.TimeSegmentation(G, fm, t, M, n, L), sens.astype(complex).ravel(), M, n, nc)
+    assert _rel(A * x, O * x.astype(complex)) < TOL
+    assert _rel(A / y, O / y.astype(complex)) < TOL
