@@ -283,7 +283,11 @@ void Gnufft::ensure_batch(int B)
     dev_free(vals);
     vals = dev_alloc<float2>((size_t)M * B);
     dev_free(partial);
-    if (n_slots > 0) partial = dev_alloc<float2>((size_t)((B + 63) / 64) * n_slots * 16 * 64);
+    // 2-D patches: 16 points in chunks of 64 grids; 3-D patches: 64 points in
+    // chunks of 32
+    if (n_slots > 0)
+        partial = dev_alloc<float2>(n_items3 > 0 ? (size_t)((B + 31) / 32) * n_slots * 64 * 32
+                                                 : (size_t)((B + 63) / 64) * n_slots * 16 * 64);
     cap_batch = B;
 }
 
@@ -308,8 +312,11 @@ void Gnufft::release()
     dev_free(irec);
     dev_free(irec4);
     dev_free(ent_w);
-    dev_free(tile_off);
-    dev_free(tile_idx);
+    dev_free(items3);
+    dev_free(entries3);
+    dev_free(wpad3);
+    dev_free(iitems3);
+    dev_free(irec3);
     dev_free(zmat);
     dev_free(dapxy);
     dev_free(zcls);
@@ -828,7 +835,6 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                 for (std::thread& x : th) x.join();
                 G.entries = dev_copy(ent.data(), ent.size());
                 G.ent_w = dev_copy(ew.data(), ew.size());
-                G.tile_entries = cnt[npall];
             }
         }
         // XCD groups: the patches in (plane, Hilbert) order over the npx x npy
@@ -986,41 +992,182 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
         G.witems = dev_copy(witems.data(), witems.size());
         G.bgs = dev_copy(bgs.data(), bgs.size());
     }
-    if (D == 3) {
-        // the full 3-D grid (small batches, or no z classes): samples whose
-        // window meets each 8x8x4 tile
-        const int TX = 8, TY = 8, TZ = 4;
-        G.ntx = (g.Gx + TX - 1) / TX;
-        G.nty = (g.Gy + TY - 1) / TY;
-        G.ntz = (g.Gz + TZ - 1) / TZ;
-        const long long ntiles = (long long)G.ntx * G.nty * G.ntz;
-        std::vector<long long> cnt(ntiles + 1, 0);
-        for (int pass = 0; pass < 2 && G.nzc == 0; ++pass) {
+    if (D == 3 && G.nzc == 0) {
+        // the full 3-D grid: the entries (samples whose window meets it) of
+        // each 4x4x4 patch, in sample order.  Each host thread counts and
+        // fills the patches of a run of z layers.
+        const int npx = g.Gx / 4, npy = g.Gy / 4, npz = g.Gz / 4;
+        const long long np = (long long)npx * npy * npz;
+        PG_REQUIRE(np < (1ll << 31), PG_ERR_UNSUPPORTED, "too many patches");
+        std::vector<long long> cnt(np + 1, 0);
+        std::vector<int2> ent;
+        for (int pass = 0; pass < 2; ++pass) {
             std::vector<long long> pos;
-            std::vector<int> idx;
             if (pass == 1) {
-                for (long long t = 0; t < ntiles; ++t) cnt[t + 1] += cnt[t];
-                PG_REQUIRE(cnt[ntiles] < (1ll << 31), PG_ERR_UNSUPPORTED, "too many tile entries");
+                for (long long q = 0; q < np; ++q) cnt[q + 1] += cnt[q];
+                PG_REQUIRE(cnt[np] < (1ll << 31), PG_ERR_UNSUPPORTED, "too many patch entries");
                 pos.assign(cnt.begin(), cnt.end() - 1);
-                idx.resize(std::max<long long>(1, cnt[ntiles]));
+                ent.resize(std::max<long long>(1, cnt[np]));
             }
-            for (size_t i = 0; i < M; ++i) {
-                if (empty(i)) continue;
-                for (int tz = vlo[2 * M + i] / TZ; tz <= vhi[2 * M + i] / TZ; ++tz)
-                    for (int ty = vlo[M + i] / TY; ty <= vhi[M + i] / TY; ++ty)
-                        for (int tx = vlo[i] / TX; tx <= vhi[i] / TX; ++tx) {
-                            const long long t = ((long long)tz * G.nty + ty) * G.ntx + tx;
-                            if (pass == 0) cnt[t + 1]++;
-                            else idx[pos[t]++] = (int)i;
-                        }
-            }
-            if (pass == 1) {
-                G.tile_entries = cnt[ntiles];
-                std::vector<int> off(cnt.begin(), cnt.end());
-                G.tile_off = dev_copy(off.data(), off.size());
-                G.tile_idx = dev_copy(idx.data(), idx.size());
-            }
+            host_parallel((size_t)npz, M >= 4096 ? 1 : npz, [&](size_t zb, size_t ze) {
+                for (size_t i = 0; i < M; ++i) {
+                    const int z0 = std::max((int)zb, vlo[2 * M + i] / 4);
+                    const int z1 = std::min((int)ze - 1, vhi[2 * M + i] / 4);
+                    if (z1 < z0 || empty(i)) continue;
+                    for (int z = z0; z <= z1; ++z)
+                        for (int y = vlo[M + i] / 4; y <= vhi[M + i] / 4; ++y)
+                            for (int x = vlo[i] / 4; x <= vhi[i] / 4; ++x) {
+                                const long long q = ((long long)z * npy + y) * npx + x;
+                                if (pass == 0) {
+                                    cnt[q + 1]++;
+                                    continue;
+                                }
+                                // (each in 0 .. NT + 2: the window meets the patch)
+                                ent[pos[q]++] =
+                                    make_int2((int)i, (4 * x - lo[i] + 3) |
+                                                          (4 * y - lo[M + i] + 3) << 10 |
+                                                          (4 * z - lo[2 * M + i] + 3) << 20);
+                            }
+                }
+            });
         }
+        // blocks of four patches that follow each other along y (128
+        // contiguous bytes of every grid row), and blocks of four parts of
+        // heavier patches
+        struct Blk {
+            uint64_t key;
+            int work;  // its entries
+            int4 w[4];
+        };
+        std::vector<Blk> blk;
+        std::vector<int4> comb, parts;
+        int nslots = 0;
+        auto morton = [](int x, int y, int z) {
+            uint64_t k = 0;
+            for (int b = 0; b < 20; ++b)
+                k |= (uint64_t)(x >> b & 1) << 3 * b | (uint64_t)(y >> b & 1) << (3 * b + 1) |
+                     (uint64_t)(z >> b & 1) << (3 * b + 2);
+            return k;
+        };
+        auto patch_key = [&](int q) {
+            return morton(q % npx, q / npx % npy / 4, q / npx / npy);
+        };
+        for (int z = 0; z < npz; ++z)
+            for (int x = 0; x < npx; ++x)
+                for (int y = 0; y < npy; y += 4) {
+                    Blk b;
+                    b.key = morton(x, y / 4, z);
+                    b.work = 0;
+                    bool any = false;
+                    for (int w = 0; w < 4; ++w) {
+                        b.w[w] = make_int4(-1, 0, 0, -1);
+                        if (y + w >= npy) continue;
+                        const int q = (int)(((long long)z * npy + y + w) * npx + x);
+                        const int e0 = (int)cnt[q], n = (int)(cnt[q + 1] - cnt[q]);
+                        if (n > kP3Entries) {
+                            const int np_ = (n + kP3Entries - 1) / kP3Entries;
+                            comb.push_back(make_int4(q, nslots, np_, 0));
+                            for (int k = 0; k < np_; ++k)
+                                parts.push_back(make_int4(q, e0 + (int)((long long)n * k / np_),
+                                                          e0 + (int)((long long)n * (k + 1) / np_),
+                                                          nslots + k));
+                            nslots += np_;
+                            continue;
+                        }
+                        b.w[w] = make_int4(q, e0, e0 + n, -1);
+                        b.work += n;
+                        any = true;
+                    }
+                    if (any) blk.push_back(b);
+                }
+        for (size_t k = 0; k < parts.size(); k += 4) {
+            Blk b;
+            b.key = patch_key(parts[k].x);
+            b.work = 4 * kP3Entries;
+            for (size_t w = 0; w < 4; ++w)
+                b.w[w] = k + w < parts.size() ? parts[k + w] : make_int4(-1, 0, 0, -1);
+            blk.push_back(b);
+        }
+        // blocks along a Morton curve over (x, y / 4, z), cut into runs of
+        // equal work, run r at the block ids congruent to r mod 8: the samples
+        // that neighbouring patches share are read into one XCD's L2 (half the
+        // HBM reads of an order by length).  A block's write of its patches
+        // weighs as much as some 320 entries.
+        std::stable_sort(blk.begin(), blk.end(),
+                         [](const Blk& u, const Blk& v) { return u.key < v.key; });
+        const int kRuns = 64;
+        double total = 0, run = 0;
+        for (const Blk& b : blk) total += b.work + 320;
+        std::vector<std::vector<size_t>> runs(8);
+        for (size_t k = 0; k < blk.size(); ++k) {
+            const double w = blk[k].work + 320;
+            runs[(int)((run + 0.5 * w) * kRuns / total) % 8].push_back(k);
+            run += w;
+        }
+        size_t longest = 0;
+        for (auto& r : runs) longest = std::max(longest, r.size());
+        std::vector<int4> items(32 * longest, make_int4(-1, 0, 0, -1));
+        for (size_t g = 0; g < 8; ++g)
+            for (size_t k = 0; k < runs[g].size(); ++k)
+                std::copy(blk[runs[g][k]].w, blk[runs[g][k]].w + 4, &items[4 * (8 * k + g)]);
+        G.n_items3 = (int)items.size();
+        G.items3 = dev_copy(items.data(), items.size());
+        G.entries3 = dev_copy(ent.data(), ent.size());
+        G.n_comb = (int)comb.size();
+        G.n_slots = nslots;
+        if (!comb.empty()) G.comb = dev_copy(comb.data(), comb.size());
+        if (NT <= 8) {
+            // the interpolation's work items; the tiles of a layer in y, x order
+            const int padl = NT / 2;
+            const int Gd[3] = {g.Gx, g.Gy, g.Gz};
+            int nt[3];
+            for (int d = 0; d < 3; ++d) nt[d] = (Gd[d] + padl + 7) / 8;
+            G.ipadl = padl;
+            G.itx = nt[0];
+            G.ity = nt[1];
+            const int ntl = nt[0] * nt[1] * nt[2];
+            std::vector<int> key(M), at((size_t)ntl + 1, 0);
+            std::vector<int4> rec(M), one(M);
+            host_parallel(M, 8192, [&](size_t b, size_t e) {
+                for (size_t i = b; i < e; ++i) {
+                    int t[3], o = 0, sh = 0;
+                    const bool none = empty(i);
+                    for (int d = 0; d < 3; ++d) {
+                        const int l0 = none ? 0 : std::max(lo[(size_t)d * M + i], -padl);
+                        const int drop = none ? NT : l0 - lo[(size_t)d * M + i];
+                        t[d] = (l0 + padl) / 8;
+                        o |= (l0 + padl - 8 * t[d]) << 8 * d;
+                        sh |= std::min(drop, NT) << 8 * d;
+                    }
+                    key[i] = (t[2] * nt[1] + t[1]) * nt[0] + t[0];
+                    one[i] = make_int4((int)i, o, sh, 0);
+                }
+            });
+            for (size_t i = 0; i < M; ++i) {
+                PG_REQUIRE(key[i] >= 0 && key[i] < ntl, PG_ERR_ARG, "interp binning");
+                ++at[key[i] + 1];
+            }
+            for (int q = 0; q < ntl; ++q) at[q + 1] += at[q];
+            std::vector<int> pos(at.begin(), at.end() - 1);
+            for (size_t i = 0; i < M; ++i) rec[pos[key[i]]++] = one[i];
+            std::vector<std::pair<uint64_t, int>> tiles;
+            for (int q = 0; q < ntl; ++q)
+                if (at[q + 1] > at[q])
+                    tiles.push_back({morton(q % nt[0], q / nt[0] % nt[1], q / nt[0] / nt[1]), q});
+            std::sort(tiles.begin(), tiles.end());
+            std::vector<int4> its;
+            for (const auto& t : tiles)
+                for (int e = at[t.second]; e < at[t.second + 1]; e += kI3Chunk)
+                    its.push_back(
+                        make_int4(t.second, e, std::min(e + kI3Chunk, at[t.second + 1]), 0));
+            G.n_iitems3 = (int)its.size();
+            G.iitems3 = dev_copy(its.data(), its.size());
+            G.irec3 = dev_copy(rec.data(), M);
+        }
+        G.wpad3 = dev_alloc<float>((size_t)M * 3 * wpad3_len(NT));
+        pgk::build_wpad3(G, setup_stream());
+        PG_HIP(hipGetLastError());
+        PG_HIP(hipStreamSynchronize(setup_stream()));
     }
 
     G.img_tmp = dev_alloc<float2>(g.N());

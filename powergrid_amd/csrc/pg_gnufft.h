@@ -23,9 +23,17 @@ constexpr int kIT = 16;    // 2-D interp: tile edge in window starts
 constexpr int kIR = kIT + 7;  // staged grid region edge (8 taps)
 constexpr int kIChunk = 128;  // samples per interp work item
 constexpr int kIChunk4 = 64;  // the same for the four-segment staging
+constexpr int kI3Chunk = 64;  // and for the full 3-D grid
 // row pitches (in points) that an item of the four-segment staging may take
 // for its kIR x kIR region: kIR .. kIR + kI4Pitches - 1
 constexpr int kI4Pitches = 3;
+
+// 3-D spread: entries of a patch summed by one wavefront.  A lone wavefront
+// takes about 500 clocks per 4 entries, so 256 of them (14 us) keep the
+// longest item short against the whole launch
+constexpr int kP3Entries = 256;
+// a sample's padded weights along one dimension: 3 zeros, the taps, zeros
+inline int wpad3_len(int ntaps) { return ntaps > 8 ? 20 : 16; }
 
 struct Gnufft {
     Geometry geo;
@@ -60,7 +68,7 @@ struct Gnufft {
     int4* comb = nullptr;
     int n_comb = 0;
     int n_slots = 0;
-    float2* partial = nullptr;  // ceil(cap_batch/64) * n_slots * 16 * 64
+    float2* partial = nullptr;  // the slots of cap_batch grids, in whole chunks
     int* entries = nullptr;  // sample indices, grouped by patch
     // per entry k: the 16 weights wx*wy of the patch's points for that
     // entry's sample (ent_w[16k + 4a + q], point (a, q)), 0 outside its
@@ -100,11 +108,27 @@ struct Gnufft {
     float2* zmat = nullptr;
     float* dapxy = nullptr;
     int* zcls = nullptr;
-    // 3-D spread (and B < 16): point-stationary tiles
-    int ntx = 0, nty = 0, ntz = 0;
-    int* tile_off = nullptr;  // ntiles + 1
-    int* tile_idx = nullptr;  // concatenated sample indices
-    long long tile_entries = 0;
+    // 3-D plans without z classes (the full 3-D grid): the spread's work items
+    // over 4x4x4 patches (patch x + npx (y + npy z)), {patch or -1, entry
+    // begin, entry end, slot or -1}, n_items3 of them (a multiple of the
+    // block's wavefronts); entries3 holds {sample, where the patch's origin
+    // lies in the sample's padded weights: x | y << 10 | z << 20}, comb,
+    // n_comb and n_slots the patches of more than kP3Entries entries, summed
+    // in parts;
+    // wpad3 each sample's weights with zeros around them:
+    // wpad3[(3 i + d) wpad3_len + 3 + j] = w_d[j] of sample i
+    int4* items3 = nullptr;
+    int n_items3 = 0;
+    int2* entries3 = nullptr;
+    float* wpad3 = nullptr;
+    // and the interpolation's (6 or 8 taps): samples binned by the 8^3 tile of
+    // their window start re-based into [-ipadl, G - 1] (itx x ity tiles a
+    // layer); items {tile, record begin, record end, 0}, records {sample,
+    // start within the tile's region, taps the re-basing dropped, 0}, x | y
+    // << 8 | z << 16
+    int4* iitems3 = nullptr;
+    int n_iitems3 = 0;
+    int4* irec3 = nullptr;
     // kernel variants chosen by the autotuner for a batch of B grids: the
     // interpolation as a gather (0), LDS-staged with all segments at once over
     // bins of <= kIChunk samples (1) or four segments at a time over bins of

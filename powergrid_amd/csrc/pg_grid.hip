@@ -21,10 +21,10 @@
 //            precomputed); heavy patches are split into chunks of <= 64
 //            entries whose partial sums are added in a fixed order.  No
 //            atomics, no zero-fill, deterministic.
-//            3-D, >= 16 grids: one block per 8x8x4 tile, thread per point.
-//            3-D, < 16 grids: one thread per sample, hardware float atomics
-//            into a zeroed grid (the reference's OpenACC spread,
-//            gridding.cpp:102-106).
+//            3-D: 4x4x4 patches on the matrix cores (k_spread3), or, for a few
+//            grids of a plan of z-class planes, one thread per sample with
+//            hardware float atomics into a zeroed grid (the reference's
+//            OpenACC spread, gridding.cpp:102-106).
 #include "pg_gnufft.h"
 #include "pg_internal.h"
 #include "pg_fftreg.h"
@@ -504,6 +504,123 @@ __global__ void __launch_bounds__(kI4Threads, CPX ? 6 : 7) k_interp_lds4(
     PG_DPP_ADDQ(ti, 0x4E);
 #undef PG_DPP_ADDQ
     if (l4 == 0 && live) out[c * out_cstride + idx] = make_float2(tr, ti);
+}
+
+// The full 3-D grid with 6 or 8 taps: one block of 512 threads per (work item
+// of <= kI3Chunk samples whose window starts lie in one 8^3 tile, coil).
+// Per segment the R^3 region under the tile (R = 7 + NT) is staged in LDS
+// through a buffer resource (points outside the grid read zero), the next
+// segment's loads in flight during the taps.  Thread (s, y) = (tid / 8,
+// tid % 8) sums sample s over the x and z taps at y tap y:
+//   t = sum_z wz sum_x wx g(ox + x, oy + y, oz + z),
+// adds AA_l t to its running sum, and the 8 lanes of a sample are added at
+// the end with their wy.  A half-wavefront's tap read is then 4 runs of 64
+// bytes (32 separate samples would collide 3.5-fold on the banks, 4 runs
+// about twofold).  Each XCD takes one run of the items (in Morton order of
+// their tiles), one coil after another: the regions of a coil's L grids under
+// some sixteen neighbouring tiles then fit its L2.
+// Measured on 32 grids of 128^3, 131072 samples on 1024 spokes: 2130 us for
+// the gather kernel above (four lanes per sample: 16 cache lines per load),
+// 1830 us for a wavefront per sample gathering 8 rows of 64 bytes per load,
+// 680 us here.  Bound by the LDS reads (43% of its time with their bank
+// conflicts) and the vector units (36%) in turn.
+using pg::kI3Chunk;
+
+template <int NT, bool CPX>
+__global__ void __launch_bounds__(8 * kI3Chunk) k_interp3_lds(
+    const int4* __restrict__ items, int n_items, const int4* __restrict__ rec,
+    const float* __restrict__ wpad, int itx, int ity, int padl, const float2* __restrict__ grids,
+    long long G, int Gx, int Gy, int Gz, int nc, int L, const float* __restrict__ AA,
+    const float* __restrict__ AAi, int M, float2* __restrict__ out, long long out_cstride, int per)
+{
+    constexpr int R = 7 + NT;
+    constexpr int NQ = R * R * R;
+    constexpr int NTH = 8 * kI3Chunk;
+    constexpr int NP = (NQ + NTH - 1) / NTH;
+    constexpr int NTP = 16;
+    __shared__ float2 tile[NQ];
+    const int tid = threadIdx.x;
+    const int p = blockIdx.x, pr = p >> 3;
+    const int c = pr / per, k = (p & 7) * per + pr - c * per;
+    if (k >= n_items) return;
+    const int4 it = items[k];
+    const int n = it.z - it.y;
+    const int tx = it.x % itx, tr0 = it.x / itx;
+    const int rx0 = tx * 8 - padl, ry0 = (tr0 % ity) * 8 - padl, rz0 = (tr0 / ity) * 8 - padl;
+    const float2* gc = grids + (long long)c * L * G;
+    int voff[NP];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+        const int q = tid + u * NTH;
+        const int zr = q / (R * R), w = q - zr * (R * R);
+        const int xr = w / R, yr = w - xr * R;
+        const int x = rx0 + xr, y = ry0 + yr, z = rz0 + zr;
+        const bool ok = q < NQ && x >= 0 && x < Gx && y >= 0 && y < Gy && z >= 0 && z < Gz;
+        voff[u] = ok ? ((z * Gx + x) * Gy + y) * 8 : (int)0x80000000u;
+    }
+    float2 tv[NP];
+    auto load_segment = [&](int l) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(gc + l * G), (short)0, (int)G * 8, kBufferWord3);
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            tv[u] = __builtin_bit_cast(float2,
+                                       __builtin_amdgcn_raw_buffer_load_b64(rs, voff[u], 0, 0));
+    };
+    load_segment(0);
+    const int s = tid >> 3, ty = tid & 7;
+    const bool live = s < n && ty < NT;
+    const int4 r = rec[it.y + min(s, n - 1)];
+    const int ox = r.y & 255, oy = (r.y >> 8) & 255, oz = r.y >> 16;
+    const float2* tp = tile + (oz * R + ox) * R + oy + ty;
+    // the weights from the re-based window start on (taps moved off it carry
+    // weight zero)
+    const float* wp = wpad + (long long)r.x * (3 * NTP) + 3;
+    const int sx = r.z & 255, sy = (r.z >> 8) & 255, sz = r.z >> 16;
+    float wx[NT], wz[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        wx[q] = q + sx < NT ? wp[q + sx] : 0.f;
+        wz[q] = q + sz < NT ? wp[2 * NTP + q + sz] : 0.f;
+    }
+    const float wy = ty + sy < NT ? wp[NTP + ty + sy] : 0.f;
+    float tr = 0.f, ti = 0.f;
+#pragma unroll 1
+    for (int l = 0; l < L; ++l) {
+        if (l) __syncthreads();  // the previous segment's taps are done
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (u + 1 < NP || tid + u * NTH < NQ) tile[tid + u * NTH] = tv[u];
+        __syncthreads();
+        if (l + 1 < L) load_segment(l + 1);
+        if (live) {
+            const float a = AA ? AA[(long long)l * M + r.x] : 1.f;
+            const float b = CPX ? AAi[(long long)l * M + r.x] : 0.f;
+            float ar = 0.f, ai = 0.f;
+#pragma unroll
+            for (int z = 0; z < NT; ++z) {
+                float xr = 0.f, xi = 0.f;
+#pragma unroll
+                for (int x = 0; x < NT; ++x) {
+                    const float2 v = tp[(z * R + x) * R];
+                    xr += wx[x] * v.x;
+                    xi += wx[x] * v.y;
+                }
+                ar += wz[z] * xr;
+                ai += wz[z] * xi;
+            }
+            if (CPX) {
+                tr += a * ar - b * ai;
+                ti += a * ai + b * ar;
+            } else {
+                tr += a * ar;
+                ti += a * ai;
+            }
+        }
+    }
+    const float vr = group8_sum_to_7(live ? wy * tr : 0.f);
+    const float vi = group8_sum_to_7(live ? wy * ti : 0.f);
+    if (ty == 7 && s < n) out[c * out_cstride + r.x] = make_float2(vr, vi);
 }
 
 // value of sample i in grid b: AA_l * (in_c[i] or W (y_c[i] - Ax_c[i])),
@@ -1302,72 +1419,236 @@ __global__ void __launch_bounds__(64) k_spread_heavy_combine(const int4* __restr
           q % pg::kPatch] = t;
 }
 
-// ------------------------------------------- 3-D tile spread (B >= 16) ----
-constexpr int kChunk = 64;
+// ------------------------------------------- 3-D patch spread ------------
+// The full 3-D grid (trajectories that are not stacks of 2-D ones), any
+// number of grids.  A wavefront runs the work item items3[] = {patch (-1:
+// none), entry begin, entry end, slot or -1}: it forms a 4x4x4 patch of up
+// to 8 NCT grids as a product on the matrix cores,
+//   acc[64 points][16 NCT floats] += W[64 points][4 entries] V[4 entries][16 NCT floats]
+// four entries a step: per entry the weights wx wy wz of the patch's points,
+// formed from the sample's padded weights (wpad), and its row of values
+// (re and im as separate columns).  v_mfma_f32_16x16x4f32: A[i][k] in lane
+// i + 16k, B[k][j] in lane j + 16k, D[i][j] in lane j + 16 (i / 4), register
+// i % 4.  Point tile z holds the patch's plane z, i = 4 x + y; column j of
+// float tile t is float NCT j + t of the chunk's row, so a lane loads NCT
+// consecutive floats of its entry's row and ends with the 4 points along y
+// of plane z and row x = lane / 16.
+// Why this form: a thread per grid point (8x8x4 tiles, the values broadcast
+// from LDS) left 79% of its lanes outside the sample's window, and the
+// central tiles, which every spoke of a radial trajectory crosses, were one
+// block's serial loop; here 38% of the products are inside the window, they
+// run at the matrix rate (twice the vector one) and patches of more than
+// kP3Entries entries are cut into parts, added in part order by
+// k_spread3_combine.  32 grids of 128^3, 131072 samples on 1024 spokes: 4860 ->
+// 390 us, and 65 us for the parts.  The products themselves take 150 us (128
+// clocks per entry and 32 grids) and the 0.8 GB written 170; the rest is the
+// latency of each patch's first entries at 3 wavefronts per SIMD.  Few grids
+// (a single NUFFT, density compensation) leave columns empty; they took the
+// atomic spread before: 6 grids of 60^3, 36080 samples, 11.4 ms -> 0.06 ms
+// with the rest of the adjoint.
+// Deterministic: entries in sample order, parts in order.  A value that is
+// not finite reaches every point of the patches its window meets.
+typedef float pg_f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float pg_f2u __attribute__((ext_vector_type(2), aligned(4)));
 
-template <int NT, int BC>
-__global__ void __launch_bounds__(256) k_spread_tile3(
-    const int* __restrict__ lo, const float* __restrict__ w, int M, int Gx, int Gy, int Gz,
-    const int* __restrict__ tile_off, const int* __restrict__ tile_idx, int ntx, int nty,
-    const float2* __restrict__ V, int B, float2* __restrict__ grids, long long G)
+constexpr int kP3Waves = 4;
+
+template <int NTP>
+__global__ void __launch_bounds__(256) k_wpad3(const float* __restrict__ w, int NT, int M,
+                                               float* __restrict__ wpad)
 {
-    __shared__ int s_lo[kChunk][3];
-    __shared__ float s_w[kChunk][3][NT];
-    __shared__ float2 s_v[kChunk][BC];
+    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (long long)M * 3 * NTP) return;
+    const int i = (int)(e / (3 * NTP)), q = (int)(e - (long long)i * (3 * NTP));
+    const int d = q / NTP, j = q - d * NTP - 3;
+    wpad[e] = (j >= 0 && j < NT) ? w[(long long)(d * NT + j) * M + i] : 0.f;
+}
 
-    const int tile = blockIdx.x;
-    const int b0 = blockIdx.y * BC;
-    const int tid = threadIdx.x;
-    const int txy = ntx * nty;
-    const int tz = tile / txy, r = tile - tz * txy;
-    const int tx = r % ntx, ty = r / ntx;
-    const int px = tx * 8 + ((tid >> 3) & 7);
-    const int py = ty * 8 + (tid & 7);
-    const int pz = tz * 4 + (tid >> 6);
-    float2 acc[BC];
+template <int NTP, int NCT>
+__global__ void __launch_bounds__(64 * kP3Waves) k_spread3(
+    const int4* __restrict__ items, const int2* __restrict__ entries,
+    const float* __restrict__ wpad, const float2* __restrict__ V, int B,
+    float2* __restrict__ grids, long long G, int Gx, int Gy, int npx, int npy,
+    float2* __restrict__ partial, int n_slots)
+{
+    constexpr int CW = 8 * NCT;  // grids per chunk
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int4 it = items[blockIdx.x * kP3Waves + wv];
+    if (it.x < 0) return;
+    const int b0 = blockIdx.y * CW;
+    const int nf = 2 * min(CW, B - b0);  // floats of the chunk's rows
+    const int px = it.x % npx, pr = it.x / npx;
+    const int x0 = px * 4, y0 = (pr % npy) * 4, z0 = (pr / npy) * 4;
+    const int i = lane & 15, k = lane >> 4;
+    const int ax = i >> 2, ay = i & 3;
+    // this lane's floats of a row; past the chunk's floats its last ones
+    // (those columns are never stored), an odd grid's last pair moved into
+    // place (NCT 4, nf % 4 == 2; a last chunk of one grid reads from the grid
+    // before it)
+    const int fo = min(NCT * i, nf - NCT);
+    const bool shifted = NCT == 4 && NCT * i + NCT > nf && NCT * i < nf;
+    const float* Vf = reinterpret_cast<const float*>(V) + 2 * (long long)b0 + fo;
+    pg_f4 acc[4][NCT];
 #pragma unroll
-    for (int bb = 0; bb < BC; ++bb) acc[bb] = make_float2(0.f, 0.f);
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int t = 0; t < NCT; ++t) acc[z][t] = pg_f4{0.f, 0.f, 0.f, 0.f};
 
-    const int beg = tile_off[tile], end = tile_off[tile + 1];
-    for (int base = beg; base < end; base += kChunk) {
-        const int cnt = min(kChunk, end - base);
-        __syncthreads();
-        if (tid < cnt) {
-            const int i = tile_idx[base + tid];
+    // groups of 4 U entries, the next group's loads in flight during this
+    // group's products; the lanes hold 64 entries at a time and the next 64
+    // are requested a stage ahead
+    constexpr int U = 2, GE = 4 * U, PER = 64 / GE;
+    const int n = it.z - it.y;
+    const int ng = (n + GE - 1) / GE;
+    float wx[2][U], wy[2][U], v[2][U][NCT];
+    pg_f4u wz[2][U];
+    int2 cur = make_int2(0, 0), nxt = make_int2(0, 0);
+    auto entry = [&](int st) { return entries[it.y + min(64 * st + lane, n - 1)]; };
+    auto load_group = [&](int g, int q) {
+        if (g % PER == 0) {
+            cur = nxt;
+            nxt = entry(g / PER + 1);
+        }
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                s_lo[tid][d] = lo[(long long)d * M + i];
+        for (int u = 0; u < U; ++u) {
+            const int e = (g % PER) * GE + 4 * u + k;
+            const int si = __shfl(cur.x, e, 64), sp = __shfl(cur.y, e, 64);
+            const float* wp = wpad + (long long)si * (3 * NTP);
+            wx[q][u] = wp[(sp & 1023) + ax];
+            wy[q][u] = wp[NTP + ((sp >> 10) & 1023) + ay];
+            wz[q][u] = *reinterpret_cast<const pg_f4u*>(wp + 2 * NTP + (sp >> 20));
+            const float* row = Vf + 2LL * B * si;
+            if (NCT == 4) {
+                const pg_f4u w = *reinterpret_cast<const pg_f4u*>(row);
 #pragma unroll
-                for (int j = 0; j < NT; ++j) s_w[tid][d][j] = w[(long long)(d * NT + j) * M + i];
+                for (int t = 0; t < NCT; ++t) v[q][u][t] = w[t];
+            } else if (NCT == 2) {
+                const pg_f2u w = *reinterpret_cast<const pg_f2u*>(row);
+                v[q][u][0] = w[0];
+                v[q][u][1 % NCT] = w[1];
+            } else {
+                v[q][u][0] = row[0];
             }
         }
-        for (int t = tid; t < cnt * BC; t += blockDim.x) {
-            const int sl = t / BC, bb = t - sl * BC;
-            const int b = b0 + bb;
-            s_v[sl][bb] = (b < B) ? V[(long long)tile_idx[base + sl] * B + b] : make_float2(0.f, 0.f);
-        }
-        __syncthreads();
-        for (int sl = 0; sl < cnt; ++sl) {
-            const unsigned dx = (unsigned)(px - s_lo[sl][0]);
-            const unsigned dy = (unsigned)(py - s_lo[sl][1]);
-            const unsigned dz = (unsigned)(pz - s_lo[sl][2]);
-            if (dx < (unsigned)NT && dy < (unsigned)NT && dz < (unsigned)NT) {
-                const float ww = s_w[sl][0][dx] * s_w[sl][1][dy] * s_w[sl][2][dz];
+    };
+    auto sum_group = [&](int g, int q) {
 #pragma unroll
-                for (int bb = 0; bb < BC; ++bb) {
-                    const float2 v = s_v[sl][bb];
-                    acc[bb].x += ww * v.x;
-                    acc[bb].y += ww * v.y;
-                }
+        for (int u = 0; u < U; ++u) {
+            // entries past the end (the last one again): zero weights and values
+            const int m = GE * g + 4 * u + k < n ? -1 : 0;
+            const float wxy = __int_as_float(__float_as_int(wx[q][u] * wy[q][u]) & m);
+            float vm[NCT];
+#pragma unroll
+            for (int t = 0; t < NCT; ++t) {
+                float w = v[q][u][t];
+                if (NCT == 4 && t < 2) w = shifted ? v[q][u][(t + 2) % NCT] : w;
+                vm[t] = __int_as_float(__float_as_int(w) & m);
+            }
+#pragma unroll
+            for (int z = 0; z < 4; ++z) {
+                const float a = wxy * __int_as_float(__float_as_int(wz[q][u][z]) & m);
+#pragma unroll
+                for (int t = 0; t < NCT; ++t)
+                    acc[z][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vm[t], acc[z][t], 0, 0, 0);
+            }
+        }
+    };
+    if (n > 0) {
+        nxt = entry(0);
+        load_group(0, 0);
+        // (groups past the last repeat its entries and add nothing)
+        for (int g = 0; g < ng; g += 2) {
+            load_group(g + 1, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            sum_group(g, 0);
+            load_group(g + 2, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            sum_group(g + 1, 1);
+        }
+    }
+    // lane: points (x0 + k, y0 + r, z0 + z), floats NCT i + t of the chunk
+    if (NCT * i >= nf) return;
+    if (it.w >= 0) {
+        float* pp = reinterpret_cast<float*>(
+            partial + ((long long)blockIdx.y * n_slots + it.w) * 64 * CW) + NCT * i;
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int t = 0; t < NCT; ++t)
+                    pp[(z * 16 + k * 4 + r) * 2 * CW + t] = acc[z][t][r];
+        return;
+    }
+    const long long pt = ((long long)z0 * Gx + x0 + k) * Gy + y0;
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+        float* gz = reinterpret_cast<float*>(grids + b0 * G + pt + (long long)z * Gx * Gy);
+        if (NCT == 1) {
+            float* gp = gz + (i >> 1) * 2 * G + (i & 1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) gp[2 * r] = acc[z][0][r];
+        } else {
+            // four points along y: 32 contiguous bytes at a 32-byte boundary
+#pragma unroll
+            for (int h = 0; h < NCT / 2; ++h) {
+                const int gb = (NCT / 2) * i + h;
+                if (2 * gb >= nf) break;
+                float4* g4 = reinterpret_cast<float4*>(gz + gb * 2 * G);
+                const pg_f4 re = acc[z][(2 * h) % NCT], im = acc[z][(2 * h + 1) % NCT];
+                g4[0] = make_float4(re[0], im[0], re[1], im[1]);
+                g4[1] = make_float4(re[2], im[2], re[3], im[3]);
             }
         }
     }
-    if (px < Gx && py < Gy && pz < Gz) {
-        const long long p = (long long)pz * Gx * Gy + (long long)px * Gy + py;
-#pragma unroll
-        for (int bb = 0; bb < BC; ++bb)
-            if (b0 + bb < B) grids[(long long)(b0 + bb) * G + p] = acc[bb];
+}
+
+// patches summed in parts: comb = {patch, first slot, parts, 0}; block
+// (patch, grid chunk, 256 of its 64 CW sums), the parts added in slot order
+template <int CW>
+__global__ void __launch_bounds__(256) k_spread3_combine(
+    const int4* __restrict__ comb, const float2* __restrict__ partial, int n_slots, int B,
+    float2* __restrict__ grids, long long G, int Gx, int Gy, int npx, int npy)
+{
+    const int4 cb = comb[blockIdx.x];
+    const int e = blockIdx.z * 256 + threadIdx.x;
+    const int p = e / CW, b = blockIdx.y * CW + e % CW;
+    if (b >= B) return;
+    const float2* pp = partial + ((long long)blockIdx.y * n_slots + cb.y) * 64 * CW + e;
+    float2 t = pp[0];
+#pragma unroll 8
+    for (int q = 1; q < cb.z; ++q) {
+        const float2 v = pp[(long long)q * 64 * CW];
+        t.x += v.x;
+        t.y += v.y;
     }
+    const int px = cb.x % npx, pr = cb.x / npx;
+    const int x0 = px * 4, y0 = (pr % npy) * 4, z0 = (pr / npy) * 4;
+    grids[b * G + ((long long)(z0 + (p >> 4)) * Gx + x0 + ((p >> 2) & 3)) * Gy + y0 + (p & 3)] = t;
+}
+
+template <int NTP>
+void launch_spread3(const pg::Gnufft& G, const float2* V, int B, float2* grids, float2* partial,
+                    hipStream_t s)
+{
+    const pg::Geometry& g = G.geo;
+    const int npx = g.Gx / 4, npy = g.Gy / 4;
+    auto launch = [&](auto kern, auto comb, int cw) {
+        const dim3 grid(G.n_items3 / kP3Waves, (B + cw - 1) / cw);
+        hipLaunchKernelGGL(kern, grid, dim3(64 * kP3Waves), 0, s, G.items3, G.entries3, G.wpad3, V,
+                           B, grids, g.G(), g.Gx, g.Gy, npx, npy, partial,
+                           G.n_slots);
+        if (G.n_comb > 0)
+            hipLaunchKernelGGL(comb, dim3(G.n_comb, grid.y, cw / 4), dim3(256), 0, s, G.comb, partial,
+                               G.n_slots, B, grids, g.G(), g.Gx, g.Gy, npx, npy);
+    };
+    // columns for the grids there are: 8, 16 or (in chunks of) 32
+    if (B <= 8)
+        launch(k_spread3<NTP, 1>, k_spread3_combine<8>, 8);
+    else if (B <= 16)
+        launch(k_spread3<NTP, 2>, k_spread3_combine<16>, 16);
+    else
+        launch(k_spread3<NTP, 4>, k_spread3_combine<32>, 32);
 }
 
 // --------------------------------------- atomic spread (one NUFFT at a time)
@@ -1460,6 +1741,20 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
                            (const int*)G.zcls, pstride);
         return;
     }
+    if constexpr (D3 && NT <= 8) {
+        // (32-bit byte offsets within a grid)
+        if (G.n_iitems3 > 0 && g.G() * 8 < (1LL << 31)) {
+            const int per = (G.n_iitems3 + 7) / 8;
+            auto launch = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)(8 * per * nc)), dim3(8 * kI3Chunk), 0, s, G.iitems3,
+                                   G.n_iitems3, G.irec3, G.wpad3, G.itx, G.ity, G.ipadl, grids,
+                                   g.G(), g.Gx, g.Gy, g.Gz, nc, L, AA, AAi, G.M, out, out_cstride,
+                                   per);
+            };
+            AAi ? launch(k_interp3_lds<NT, true>) : launch(k_interp3_lds<NT, false>);
+            return;
+        }
+    }
     hipLaunchKernelGGL((k_interp<NT, D3>), dim3(nsb * nc), dim3(256), 0, s, G.lo, G.w, G.M, g.Gx,
                        g.Gy, g.Gz, grids, g.G(), nc, L, AA, AAi, out, out_cstride, nsb, xmap,
                        (const int*)nullptr, 0LL);
@@ -1473,7 +1768,8 @@ void spread_dispatch(const pg::Gnufft& G, const float2* in, long long in_cstride
 {
     const pg::Geometry& g = G.geo;
     const int B = nc * L;
-    if (D3 && !planes && B < 16) {
+    if (D3 && !planes && G.nzc > 0) {
+        // a plan of z-class planes has no 3-D work lists
         const long long n = (long long)B * g.G();
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, grids, n);
         hipLaunchKernelGGL((k_spread_atomic<NT, D3>), dim3((G.M + 255) / 256, B), dim3(256), 0, s,
@@ -1544,13 +1840,10 @@ void spread_dispatch(const pg::Gnufft& G, const float2* in, long long in_cstride
                                npy, partial, G.n_slots, B, grids, gsz, g.Gy, G.npp, pstride);
         return;
     }
-    PG_REQUIRE(G.tile_off && G.tile_idx, PG_ERR_STATE,
-               "plan built for z-class planes: no 3-D tile lists for a batch of this size");
-    constexpr int BC = 16;
-    const int ntiles = G.ntx * G.nty * G.ntz;
-    hipLaunchKernelGGL((k_spread_tile3<NT, BC>), dim3(ntiles, (B + BC - 1) / BC), dim3(256), 0, s,
-                       G.lo, G.w, G.M, g.Gx, g.Gy, g.Gz, G.tile_off, G.tile_idx, G.ntx, G.nty,
-                       vals, B, grids, g.G());
+    if (NT == 12)
+        launch_spread3<20>(G, vals, B, grids, partial, s);
+    else
+        launch_spread3<16>(G, vals, B, grids, partial, s);
 }
 
 }  // namespace
@@ -1619,7 +1912,21 @@ void launch_interp(const pg::Gnufft& G, const float2* grids, int nc, int L, cons
     }
 }
 
-bool spread_uses_values(const pg::Gnufft& G, int B) { return !(G.geo.dims == 3 && B < 16); }
+bool spread_uses_values(const pg::Gnufft& G, int B)
+{
+    return G.geo.dims == 2 || G.nzc == 0 || zclass_active(G, B);
+}
+
+void build_wpad3(const pg::Gnufft& G, hipStream_t s)
+{
+    const int ntp = pg::wpad3_len(G.geo.ntaps);
+    const long long n = (long long)G.M * 3 * ntp;
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (ntp == 20)
+        hipLaunchKernelGGL(k_wpad3<20>, grid, dim3(256), 0, s, G.w, G.geo.ntaps, G.M, G.wpad3);
+    else
+        hipLaunchKernelGGL(k_wpad3<16>, grid, dim3(256), 0, s, G.w, G.geo.ntaps, G.M, G.wpad3);
+}
 
 void launch_spread_values(const pg::Gnufft& G, const float2* in, long long in_cstride, int nc,
                           int L, const float* AA, const float* AAi, const float2* resid_y,

@@ -88,11 +88,6 @@ struct Geometry {
     long long G() const { return (long long)Gx * Gy * Gz; }
 };
 
-// Spread binning: for each grid tile, the samples whose window intersects it.
-constexpr int kSpreadTX = 16;  // tile extent along x (grid points)
-constexpr int kSpreadTY = 16;  // tile extent along y
-constexpr int kSpreadTZ = 4;   // tile extent along z (3-D)
-
 struct Gnufft;
 
 // launch(first, count) over [0, n) in runs that fit one grid dimension (y, z)
@@ -184,6 +179,8 @@ void launch_spread(const pg::Gnufft& G, const float2* in, long long in_cstride, 
                    const float* AA, const float* AAi, const float2* resid_y, const double2* ax64,
                    const float* Wd, float2* grids, bool vals_ready, hipStream_t s,
                    bool planes = false, float2* vals = nullptr, float2* partial = nullptr);
+// G.wpad3 from G.w (asynchronous on s)
+void build_wpad3(const pg::Gnufft& G, hipStream_t s);
 // whether launch_spread reads per-sample values (all but the 3-D atomic path)
 bool spread_uses_values(const pg::Gnufft& G, int B);
 // whether the LDS-staged interpolation serves L segments of plan G (the

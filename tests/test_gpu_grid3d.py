@@ -1,0 +1,67 @@
+"""GPU: gridding on the full 3-D grid (trajectories that are not stacks of
+2-D ones) against the FP64 restatement (oracle): every chunk width of the
+patch spread, patches summed in parts, ragged items, windows past the grid's
+edges, 6, 8 and 12 taps.
+
+Tolerance 2e-6: FP32 sums of products of three taps (each rounded, eps = 6e-8)
+and a 3-D FFT, below 1e-6 in relative 2-norm."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-6
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def _traj(rng, N, Nz, M, centre):
+    k = [rng.uniform(-N / 2, N / 2, M), rng.uniform(-N / 2, N / 2, M),
+         rng.uniform(-Nz / 2, Nz / 2, M)]
+    for a in k:
+        a[:int(centre * M)] *= 0.05  # crowd the central patches
+        a[-1] = -N / 2 - 1.7 if a is k[0] else a[-1]  # a window partly off the grid
+    k[1][-2] = N  # and one wholly off it
+    return [a.astype(np.float32) for a in k]
+
+
+def _complex(rng, *shape):
+    return (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64)
+
+
+@pytest.mark.parametrize("N,Nz,M,nc,L,width,centre", [
+    (12, 10, 301, 1, 1, 4.0, 0.0), (12, 10, 301, 4, 2, 4.0, 0.0), (12, 10, 301, 9, 1, 4.0, 0.0),
+    (12, 10, 65, 8, 2, 4.0, 0.0), (12, 10, 301, 17, 1, 4.0, 0.0), (12, 10, 301, 33, 1, 4.0, 0.0),
+    (10, 4, 97, 13, 5, 3.0, 0.2), (16, 16, 5000, 6, 3, 4.0, 0.5), (16, 16, 9000, 3, 1, 4.0, 0.5)])
+def test_operator(orc, N, Nz, M, nc, L, width, centre):
+    import powergrid_amd as P
+    rng = np.random.default_rng(M + nc)
+    k = _traj(rng, N, Nz, M, centre)
+    n = N * N * Nz
+    t = np.linspace(1e-3, 9e-3, M).astype(np.float32)
+    fm = rng.uniform(-300, 300, n).astype(np.float32)
+    sens, x, y = _complex(rng, nc, n), _complex(rng, n), _complex(rng, nc * M)
+    Gg = P.Gnufft(M, 2.0, N, N, Nz, *k, kernel_width=width)
+    assert P.zclasses(Gg) == 0
+    A = P.SENSE(P.TimeSegmentation(Gg, fm, t, M, n, L), sens, M, n, nc)
+    G = orc.Gnufft(M, 2.0, N, N, Nz, *k, width, prec="d")
+    O = orc.SENSE(orc.TimeSegmentation(G, fm, t, M, n, L), sens.astype(complex).ravel(), M, n, nc)
+    assert _rel(A * x, O * x.astype(complex)) < TOL
+    assert _rel(A / y, O / y.astype(complex)) < TOL
+    assert np.array_equal(A / y, A / y)  # deterministic
+
+
+@pytest.mark.parametrize("gridos,width", [(2.0, 4.0), (2.0, 3.0), (3.0, 4.0)])
+def test_spatial_interpolation(orc, gridos, width):
+    import powergrid_amd as P
+    rng = np.random.default_rng(3)
+    N, Nz, M = 12, 8, 400
+    k = _traj(rng, N, Nz, M, 0.3)
+    Gg = P.Gnufft(M, gridos, N, N, Nz, *k, kernel_width=width)
+    grid, d = _complex(rng, Gg.grid_size), _complex(rng, M)
+    geo = (*k, N, N, Nz)
+    assert _rel(Gg.forwardSpatialInterp(grid),
+                orc.grid_forward(grid.astype(complex), *geo, gridos, width)) < TOL
+    assert _rel(Gg.adjointSpatialInterp(d),
+                orc.grid_adjoint(d.astype(complex), *geo, Gg.grid_size, gridos, width)) < TOL
