@@ -21,6 +21,7 @@
 //   sinc(x) = sin(pi x)/(pi x) (1 below 1e-4), with the field-map difference
 //   maps G staged beside the pixel coordinates.
 #include "pg_dft.h"
+#include "pg_fftreg.h"
 
 #include <mutex>
 
@@ -54,7 +55,9 @@ struct R2Args {
     float inx, iny, inz;  // 1/Nx, 1/Ny, 1/Nz
 };
 
-template <int NCB, bool F64, bool R2>
+// FP64 phase, trig and sums (precision 1): one wavefront per 64 outputs and
+// input slice, the inputs staged in LDS; bound by the FP64 sine and cosine.
+template <int NCB, bool R2>
 __global__ void __launch_bounds__(kT) k_gdft_fwd(
     const float* __restrict__ kx, const float* __restrict__ ky, const float* __restrict__ kz,
     const float* __restrict__ t, const float* __restrict__ ix, const float* __restrict__ iy,
@@ -75,7 +78,6 @@ __global__ void __launch_bounds__(kT) k_gdft_fwd(
     const int c0 = blockIdx.z * NCB;
     const int j0 = blockIdx.y * slice_len;
     const int j1 = min(N, j0 + slice_len);
-    const float tw = 6.283185307179586f;
     float ki[3] = {0, 0, 0};
     float ti = 0;
     if (live) {
@@ -87,9 +89,6 @@ __global__ void __launch_bounds__(kT) k_gdft_fwd(
     double ar[NCB], ai[NCB];
 #pragma unroll
     for (int c = 0; c < NCB; ++c) ar[c] = ai[c] = 0.0;
-    float fr[NCB], fi[NCB];
-#pragma unroll
-    for (int c = 0; c < NCB; ++c) fr[c] = fi[c] = 0.f;
 
     for (int jb = j0; jb < j1; jb += kT) {
         __syncthreads();
@@ -98,7 +97,7 @@ __global__ void __launch_bounds__(kT) k_gdft_fwd(
             s_r[threadIdx.x][0] = ix[j];
             s_r[threadIdx.x][1] = iy[j];
             s_r[threadIdx.x][2] = iz[j];
-            s_r[threadIdx.x][3] = F64 ? fm[j] : (float)((double)fm[j] / (2.0 * M_PI));
+            s_r[threadIdx.x][3] = fm[j];
             if (R2) {
                 s_g[threadIdx.x][0] = r2.gx[j];
                 s_g[threadIdx.x][1] = r2.gy[j];
@@ -118,59 +117,37 @@ __global__ void __launch_bounds__(kT) k_gdft_fwd(
         __syncthreads();
         const int cnt = min(kT, j1 - jb);
         for (int q = 0; q < cnt; ++q) {
-            float cs, sn;
-            if (F64) {
-                const double ph = 2.0 * M_PI * ((double)ki[0] * s_r[q][0] + (double)ki[1] * s_r[q][1] +
-                                                (double)ki[2] * s_r[q][2]) +
-                                  (double)s_r[q][3] * ti;
-                double sd, cd;
-                sincos(ph, &sd, &cd);
-                if (R2) {
-                    const double b = sinc_d((double)ki[0] * r2.inx + (double)s_g[q][0] * ti) *
-                                     sinc_d((double)ki[1] * r2.iny + (double)s_g[q][1] * ti) *
-                                     sinc_d((double)ki[2] * r2.inz + (double)s_g[q][2] * ti);
-                    sd *= b;
-                    cd *= b;
-                }
+            const double ph = 2.0 * M_PI * ((double)ki[0] * s_r[q][0] + (double)ki[1] * s_r[q][1] +
+                                            (double)ki[2] * s_r[q][2]) +
+                              (double)s_r[q][3] * ti;
+            double sd, cd;
+            sincos(ph, &sd, &cd);
+            if (R2) {
+                const double b = sinc_d((double)ki[0] * r2.inx + (double)s_g[q][0] * ti) *
+                                 sinc_d((double)ki[1] * r2.iny + (double)s_g[q][1] * ti) *
+                                 sinc_d((double)ki[2] * r2.inz + (double)s_g[q][2] * ti);
+                sd *= b;
+                cd *= b;
+            }
 #pragma unroll
-                for (int c = 0; c < NCB; ++c) {
-                    const float2 v = s_v[q][c];
-                    ar[c] += cd * v.x + sd * v.y;
-                    ai[c] += -sd * v.x + cd * v.y;
-                }
-            } else {
-                float p = ki[0] * s_r[q][0] + ki[1] * s_r[q][1] + ki[2] * s_r[q][2] + s_r[q][3] * ti;
-                p = p - rintf(p);
-                sn = __builtin_amdgcn_sinf(p);
-                cs = __builtin_amdgcn_cosf(p);
-                if (R2) {
-                    const float b = sinc_f(ki[0] * r2.inx + s_g[q][0] * ti) *
-                                    sinc_f(ki[1] * r2.iny + s_g[q][1] * ti) *
-                                    sinc_f(ki[2] * r2.inz + s_g[q][2] * ti);
-                    sn *= b;
-                    cs *= b;
-                }
-#pragma unroll
-                for (int c = 0; c < NCB; ++c) {
-                    const float2 v = s_v[q][c];
-                    fr[c] += cs * v.x + sn * v.y;
-                    fi[c] += -sn * v.x + cs * v.y;
-                }
+            for (int c = 0; c < NCB; ++c) {
+                const float2 v = s_v[q][c];
+                ar[c] += cd * v.x + sd * v.y;
+                ai[c] += -sd * v.x + cd * v.y;
             }
         }
     }
-    (void)tw;
     if (live) {
 #pragma unroll
         for (int c = 0; c < NCB; ++c) {
             if (c0 + c >= nc) break;
-            const float2 r = F64 ? make_float2((float)ar[c], (float)ai[c]) : make_float2(fr[c], fi[c]);
-            part[((long long)blockIdx.y * nc + c0 + c) * M + i] = r;
+            part[((long long)blockIdx.y * nc + c0 + c) * M + i] =
+                make_float2((float)ar[c], (float)ai[c]);
         }
     }
 }
 
-template <int NCB, bool F64, bool R2>
+template <int NCB, bool R2>
 __global__ void __launch_bounds__(kT) k_gdft_adj(
     const float* __restrict__ kx, const float* __restrict__ ky, const float* __restrict__ kz,
     const float* __restrict__ t, const float* __restrict__ ix, const float* __restrict__ iy,
@@ -194,7 +171,7 @@ __global__ void __launch_bounds__(kT) k_gdft_adj(
         rj[0] = ix[j];
         rj[1] = iy[j];
         rj[2] = iz[j];
-        fj = F64 ? fm[j] : (float)((double)fm[j] / (2.0 * M_PI));
+        fj = fm[j];
         if (R2) {
             gj[0] = r2.gx[j];
             gj[1] = r2.gy[j];
@@ -202,15 +179,10 @@ __global__ void __launch_bounds__(kT) k_gdft_adj(
         }
     }
     double xr = 0, xi = 0;
-    float gr = 0, gi = 0;
     for (int c0 = 0; c0 < nc; c0 += NCB) {
         double ar[NCB], ai[NCB];
-        float fr[NCB], fi[NCB];
 #pragma unroll
-        for (int c = 0; c < NCB; ++c) {
-            ar[c] = ai[c] = 0;
-            fr[c] = fi[c] = 0;
-        }
+        for (int c = 0; c < NCB; ++c) ar[c] = ai[c] = 0;
         for (int ib = i0; ib < i1; ib += kT) {
             __syncthreads();
             const int i = ib + threadIdx.x;
@@ -227,45 +199,24 @@ __global__ void __launch_bounds__(kT) k_gdft_adj(
             __syncthreads();
             const int cnt = min(kT, i1 - ib);
             for (int q = 0; q < cnt; ++q) {
-                if (F64) {
-                    const double ph = 2.0 * M_PI * ((double)s_k[q][0] * rj[0] + (double)s_k[q][1] * rj[1] +
-                                                    (double)s_k[q][2] * rj[2]) +
-                                      (double)fj * s_k[q][3];
-                    double sd, cd;
-                    sincos(ph, &sd, &cd);
-                    if (R2) {
-                        const double tq = s_k[q][3];
-                        const double b = sinc_d((double)s_k[q][0] * r2.inx + (double)gj[0] * tq) *
-                                         sinc_d((double)s_k[q][1] * r2.iny + (double)gj[1] * tq) *
-                                         sinc_d((double)s_k[q][2] * r2.inz + (double)gj[2] * tq);
-                        sd *= b;
-                        cd *= b;
-                    }
+                const double ph = 2.0 * M_PI * ((double)s_k[q][0] * rj[0] + (double)s_k[q][1] * rj[1] +
+                                                (double)s_k[q][2] * rj[2]) +
+                                  (double)fj * s_k[q][3];
+                double sd, cd;
+                sincos(ph, &sd, &cd);
+                if (R2) {
+                    const double tq = s_k[q][3];
+                    const double b = sinc_d((double)s_k[q][0] * r2.inx + (double)gj[0] * tq) *
+                                     sinc_d((double)s_k[q][1] * r2.iny + (double)gj[1] * tq) *
+                                     sinc_d((double)s_k[q][2] * r2.inz + (double)gj[2] * tq);
+                    sd *= b;
+                    cd *= b;
+                }
 #pragma unroll
-                    for (int c = 0; c < NCB; ++c) {
-                        const float2 v = s_v[q][c];
-                        ar[c] += cd * v.x - sd * v.y;
-                        ai[c] += sd * v.x + cd * v.y;
-                    }
-                } else {
-                    float p = s_k[q][0] * rj[0] + s_k[q][1] * rj[1] + s_k[q][2] * rj[2] + fj * s_k[q][3];
-                    p = p - rintf(p);
-                    float sn = __builtin_amdgcn_sinf(p);
-                    float cs = __builtin_amdgcn_cosf(p);
-                    if (R2) {
-                        const float tq = s_k[q][3];
-                        const float b = sinc_f(s_k[q][0] * r2.inx + gj[0] * tq) *
-                                        sinc_f(s_k[q][1] * r2.iny + gj[1] * tq) *
-                                        sinc_f(s_k[q][2] * r2.inz + gj[2] * tq);
-                        sn *= b;
-                        cs *= b;
-                    }
-#pragma unroll
-                    for (int c = 0; c < NCB; ++c) {
-                        const float2 v = s_v[q][c];
-                        fr[c] += cs * v.x - sn * v.y;
-                        fi[c] += sn * v.x + cs * v.y;
-                    }
+                for (int c = 0; c < NCB; ++c) {
+                    const float2 v = s_v[q][c];
+                    ar[c] += cd * v.x - sd * v.y;
+                    ai[c] += sd * v.x + cd * v.y;
                 }
             }
         }
@@ -273,7 +224,7 @@ __global__ void __launch_bounds__(kT) k_gdft_adj(
 #pragma unroll
             for (int c = 0; c < NCB; ++c) {
                 if (c0 + c >= nc) break;
-                double vr = F64 ? ar[c] : fr[c], vi = F64 ? ai[c] : fi[c];
+                double vr = ar[c], vi = ai[c];
                 if (S) {
                     const float2 s = S[(long long)(c0 + c) * N + j];
                     const double tr = vr * s.x + vi * s.y;  // v * conj(s)
@@ -281,17 +232,292 @@ __global__ void __launch_bounds__(kT) k_gdft_adj(
                     vr = tr;
                     vi = ti;
                 }
-                if (F64) {
-                    xr += vr;
-                    xi += vi;
-                } else {
-                    gr += (float)vr;
-                    gi += (float)vi;
-                }
+                xr += vr;
+                xi += vi;
             }
         }
     }
-    if (j < N) part[(long long)blockIdx.y * N + j] = F64 ? make_float2((float)xr, (float)xi) : make_float2(gr, gi);
+    if (j < N) part[(long long)blockIdx.y * N + j] = make_float2((float)xr, (float)xi);
+}
+
+// ------------------------------------------------ FP32 on the matrix cores --
+// Both directions are products: with the phase p of (output o, input q),
+//   forward  Y[o][2c], Y[o][2c+1] = sum_q cos(p) (vr, vi)_qc + sin(p) (vi, -vr)_qc
+//   adjoint  the same with (-vi, vr)
+// over the inputs' values v_qc (S_c x, or y_c).  A wavefront takes 64 outputs
+// and 4 inputs a step: lane (i, k) = (lane % 16, lane / 16) forms the phase,
+// sine and cosine of output 16 t + i and input k for each of the four output
+// tiles t, which is the A operand A[i][k] of v_mfma_f32_16x16x4f32; column j
+// of the B operand B[k][j] (lane j + 16 k) is float j of input k's row of
+// 16 CT values (8 CT coils, re and im), the second one its neighbour's with
+// the sign.  The phase arithmetic is that of the FP64-free kernels above
+// (the same products, reduced to [-1/2, 1/2] revolutions, v_sin and v_cos)
+// and the sums are FP32.  Per 64 pairs: 16 vector instructions, sine and cosine
+// at a quarter of the rate (88 clocks, the bound), beside 2 CT products of 32
+// clocks on the matrix cores; forming the sums on the vector units took 32 more
+// instructions and 5 LDS broadcasts for 8 coils.
+// The four wavefronts of a block take a quarter of the input slice each and
+// are summed through LDS in order, so a quarter of the partial sums reach
+// memory.  4096 samples x 4096 voxels, 8 coils: forward 34 -> 20.5 us, adjoint
+// 29 -> 20.5 us (9.4 of it the vector instructions, the rest launch, staging
+// and the wavefronts' sum), and the slice sums 18.5 -> 4.5 us each.
+typedef float pgd_f4 __attribute__((ext_vector_type(4)));
+constexpr int kMW = 4;       // wavefronts per block
+constexpr int kMChunk = 64;  // inputs staged per wavefront at a time
+
+template <int CT>
+struct MfmaLds {
+    union {
+        struct {
+            float v[kMW][kMChunk][16 * CT + 4];
+            float4 r[kMW][kMChunk];
+            float3 g[kMW][kMChunk];
+        } in;
+        float sum[kMW][64][16 * CT + 1];
+    };
+};
+
+// the sums over inputs [q0, q1) (this wavefront's share) for outputs with
+// coordinates co[t] (+ gradient maps go[t] of an R2 adjoint): acc[t][n], tile
+// t, float tile n.  load(q, row, rr, gg) stages input q (a lane's own).
+template <int CT, bool R2, bool ADJ, class Load>
+__device__ __forceinline__ void dft_products(const float4 (&co)[4], const float3 (&go)[4], int q0,
+                                             int q1, float (*sv)[16 * CT + 4], float4* sr, float3* sg,
+                                             const R2Args& r2, Load load, pgd_f4 (&acc)[4][CT])
+{
+    const int lane = threadIdx.x & 63, j = lane & 15, k = lane >> 4;
+    // the second product's column: its neighbour's value, negated for the im
+    // (forward) or re (adjoint) columns
+    const int flip = ((j & 1) != 0) != ADJ ? (int)0x80000000u : 0;
+    for (int qb = q0; qb < q1; qb += kMChunk) {
+        const int n = min(kMChunk, q1 - qb);
+        load(qb + lane, lane < n, sv[lane], sr[lane], sg[lane]);
+        pgf::wave_lds_sync();
+#pragma unroll 2
+        for (int s = 0; s < n; s += 4) {
+            const float4 r = sr[s + k];
+            float3 gq = make_float3(0.f, 0.f, 0.f);
+            if (R2 && !ADJ) gq = sg[s + k];
+            float b[CT], bx[CT];
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                b[c] = sv[s + k][16 * c + j];
+                const int nb = __builtin_amdgcn_update_dpp(0, __float_as_int(b[c]), 0xB1, 0xF, 0xF,
+                                                           false);  // quad_perm [1,0,3,2]
+                bx[c] = __int_as_float(nb ^ flip);
+            }
+            float cs[4], sn[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                float p = co[t].x * r.x + co[t].y * r.y + co[t].z * r.z + r.w * co[t].w;
+                p = p - rintf(p);
+                sn[t] = __builtin_amdgcn_sinf(p);
+                cs[t] = __builtin_amdgcn_cosf(p);
+                if (R2) {
+                    // k and t of the sample, the maps of the voxel
+                    const float4 kk = ADJ ? r : co[t];
+                    const float3 gg = ADJ ? go[t] : gq;
+                    const float f = sinc_f(kk.x * r2.inx + gg.x * kk.w) *
+                                    sinc_f(kk.y * r2.iny + gg.y * kk.w) *
+                                    sinc_f(kk.z * r2.inz + gg.z * kk.w);
+                    sn[t] *= f;
+                    cs[t] *= f;
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(cs[t], b[c], acc[t][c], 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(sn[t], bx[c], acc[t][c], 0, 0, 0);
+        }
+        pgf::wave_lds_sync();  // the next chunk replaces these inputs
+    }
+}
+
+// this wavefront's sums to LDS: sum[wave][output][float]
+template <int CT>
+__device__ __forceinline__ void dft_store(float (*out)[16 * CT + 1], const pgd_f4 (&acc)[4][CT])
+{
+    const int lane = threadIdx.x & 63, j = lane & 15, k = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[16 * t + 4 * k + r][16 * c + j] = acc[t][c][r];
+}
+
+template <int CT, bool R2>
+__global__ void __launch_bounds__(64 * kMW) k_gdft_fwd_mfma(
+    const float* __restrict__ kx, const float* __restrict__ ky, const float* __restrict__ kz,
+    const float* __restrict__ t, const float* __restrict__ ix, const float* __restrict__ iy,
+    const float* __restrict__ iz, const float* __restrict__ fm, const float2* __restrict__ x,
+    const float2* __restrict__ S, int nc, int M, int N, int slice_len, int shot_len,
+    long long s_shot, float2* __restrict__ part, R2Args r2)
+{
+    __shared__ MfmaLds<CT> lds;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int tps = (shot_len + 63) / 64;  // output tiles per shot
+    const int sh = blockIdx.x / tps;
+    const int o0 = (blockIdx.x - sh * tps) * 64;
+    if (S) S += sh * s_shot;
+    const int c0 = blockIdx.z * 8 * CT;
+    float4 co[4];
+    float3 go[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = sh * shot_len + min(o0 + 16 * u + (lane & 15), shot_len - 1);
+        co[u] = make_float4(kx[i], ky[i], kz[i], t[i]);
+        go[u] = make_float3(0.f, 0.f, 0.f);
+    }
+    pgd_f4 acc[4][CT];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[u][c] = pgd_f4{0.f, 0.f, 0.f, 0.f};
+    // this wavefront's quarter of the slice, in whole steps of 4 inputs
+    const int j0 = blockIdx.y * slice_len, j1 = min(N, j0 + slice_len);
+    const int quarter = ((j1 - j0 + 4 * kMW - 1) / (4 * kMW)) * 4;
+    const int q0 = min(j1, j0 + wv * quarter), q1 = min(j1, q0 + quarter);
+    dft_products<CT, R2, false>(
+        co, go, q0, q1, lds.in.v[wv], lds.in.r[wv], lds.in.g[wv], r2,
+        [&](int q, bool ok, float* row, float4& rr, float3& gg) {
+            const int qc = ok ? q : 0;
+            const float2 xv = x[qc];
+            rr = make_float4(ix[qc], iy[qc], iz[qc], (float)((double)fm[qc] / (2.0 * M_PI)));
+            if (R2) gg = make_float3(r2.gx[qc], r2.gy[qc], r2.gz[qc]);
+            float2 sm[8 * CT];
+            if (S) {
+#pragma unroll
+                for (int c = 0; c < 8 * CT; ++c)
+                    sm[c] = S[(long long)min(c0 + c, nc - 1) * N + qc];
+            }
+#pragma unroll
+            for (int c = 0; c < 8 * CT; ++c) {
+                float2 v = xv;
+                if (S)
+                    v = make_float2(sm[c].x * xv.x - sm[c].y * xv.y, sm[c].x * xv.y + sm[c].y * xv.x);
+                const bool on = ok && c0 + c < nc;
+                row[2 * c] = on ? v.x : 0.f;
+                row[2 * c + 1] = on ? v.y : 0.f;
+            }
+        },
+        acc);
+    __syncthreads();
+    dft_store<CT>(lds.sum[wv], acc);
+    __syncthreads();
+    const int o = o0 + lane;
+    if (o >= shot_len) return;
+#pragma unroll
+    for (int u = 0; u < 2 * CT; ++u) {
+        const int c = wv * 2 * CT + u;
+        if (c0 + c >= nc) break;
+        float2 a = make_float2(lds.sum[0][lane][2 * c], lds.sum[0][lane][2 * c + 1]);
+#pragma unroll
+        for (int w = 1; w < kMW; ++w) {
+            a.x += lds.sum[w][lane][2 * c];
+            a.y += lds.sum[w][lane][2 * c + 1];
+        }
+        part[((long long)blockIdx.y * nc + c0 + c) * M + sh * shot_len + o] = a;
+    }
+}
+
+template <int CT, bool R2>
+__global__ void __launch_bounds__(64 * kMW) k_gdft_adj_mfma(
+    const float* __restrict__ kx, const float* __restrict__ ky, const float* __restrict__ kz,
+    const float* __restrict__ t, const float* __restrict__ ix, const float* __restrict__ iy,
+    const float* __restrict__ iz, const float* __restrict__ fm, const float2* __restrict__ y,
+    long long ystride, const float2* __restrict__ S, int nc, int M, int N, int slice_len,
+    int shot_len, long long s_shot, float2* __restrict__ part, R2Args r2)
+{
+    __shared__ MfmaLds<CT> lds;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int o0 = blockIdx.x * 64;
+    // gridDim.y / nshot slices per shot, each within its shot
+    const int sps = (int)gridDim.y / (M / shot_len);
+    const int sh = blockIdx.y / sps;
+    const int i0 = sh * shot_len + (blockIdx.y - sh * sps) * slice_len;
+    const int i1 = min(sh * shot_len + shot_len, i0 + slice_len);
+    if (S) S += sh * s_shot;
+    float4 co[4];
+    float3 go[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int j = min(o0 + 16 * u + (lane & 15), N - 1);
+        co[u] = make_float4(ix[j], iy[j], iz[j], (float)((double)fm[j] / (2.0 * M_PI)));
+        go[u] = R2 ? make_float3(r2.gx[j], r2.gy[j], r2.gz[j]) : make_float3(0.f, 0.f, 0.f);
+    }
+    const int quarter = ((max(i1 - i0, 0) + 4 * kMW - 1) / (4 * kMW)) * 4;
+    const int q0 = min(i1, i0 + wv * quarter), q1 = min(i1, q0 + quarter);
+    const int o = min(o0 + lane, N - 1);
+    double gr = 0.0, gi = 0.0;
+    for (int c0 = 0; c0 < nc; c0 += 8 * CT) {
+        pgd_f4 acc[4][CT];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[u][c] = pgd_f4{0.f, 0.f, 0.f, 0.f};
+        if (c0) __syncthreads();  // the previous coils' sums are read
+        dft_products<CT, R2, true>(
+            co, go, q0, q1, lds.in.v[wv], lds.in.r[wv], lds.in.g[wv], r2,
+            [&](int q, bool ok, float* row, float4& rr, float3&) {
+                const int qc = ok ? q : 0;
+                rr = make_float4(kx[qc], ky[qc], kz[qc], t[qc]);
+                float2 v[8 * CT];
+#pragma unroll
+                for (int c = 0; c < 8 * CT; ++c) v[c] = y[min(c0 + c, nc - 1) * ystride + qc];
+#pragma unroll
+                for (int c = 0; c < 8 * CT; ++c) {
+                    const bool on = ok && c0 + c < nc;
+                    row[2 * c] = on ? v[c].x : 0.f;
+                    row[2 * c + 1] = on ? v[c].y : 0.f;
+                }
+            },
+            acc);
+        __syncthreads();
+        dft_store<CT>(lds.sum[wv], acc);
+        __syncthreads();
+        // output o, this wavefront's 2 CT coils: conj(S_c) times the sums
+#pragma unroll
+        for (int u = 0; u < 2 * CT; ++u) {
+            const int c = wv * 2 * CT + u;
+            if (c0 + c >= nc) break;
+            float2 a = make_float2(lds.sum[0][lane][2 * c], lds.sum[0][lane][2 * c + 1]);
+#pragma unroll
+            for (int w = 1; w < kMW; ++w) {
+                a.x += lds.sum[w][lane][2 * c];
+                a.y += lds.sum[w][lane][2 * c + 1];
+            }
+            double vr = a.x, vi = a.y;
+            if (S) {
+                const float2 s = S[(long long)(c0 + c) * N + o];
+                const double tr = vr * s.x + vi * s.y;
+                const double ti = vi * s.x - vr * s.y;
+                vr = tr;
+                vi = ti;
+            }
+            gr += vr;
+            gi += vi;
+        }
+    }
+    // the four wavefronts' coils, in order
+    __syncthreads();
+    double2* red = reinterpret_cast<double2*>(&lds);
+    static_assert(sizeof(lds) >= kMW * 64 * sizeof(double2), "coil sums");
+    red[wv * 64 + lane] = make_double2(gr, gi);
+    __syncthreads();
+    if (wv == 0 && o0 + lane < N) {
+        for (int w = 1; w < kMW; ++w) {
+            gr += red[w * 64 + lane].x;
+            gi += red[w * 64 + lane].y;
+        }
+        part[(long long)blockIdx.y * N + o] = make_float2((float)gr, (float)gi);
+    }
 }
 
 // out[(i / row) * ostride + i % row] (+)= sum of the slices of element i:
@@ -305,6 +531,7 @@ __global__ void k_sum_slices(const float2* part, int nslice, int group, long lon
     float2 s = make_float2(0.f, 0.f);
     for (int g0 = 0; g0 < nslice; g0 += group) {
         float2 t = part[(long long)g0 * n + i];
+#pragma unroll 8
         for (int k = g0 + 1; k < g0 + group; ++k) {
             const float2 p = part[(long long)k * n + i];
             t.x += p.x;
@@ -319,6 +546,15 @@ __global__ void k_sum_slices(const float2* part, int nslice, int group, long lon
         s = make_float2(a.x + s.x, a.y + s.y);
     }
     out[o] = s;
+}
+
+void sum_slices(const float2* part, int nslice, int group, long long n, long long row,
+                long long ostride, int acc, float2* out, hipStream_t s)
+{
+    // (short outputs in blocks of one wavefront, to spread over the chip)
+    const int nt = n < 65536 ? 64 : 256;
+    hipLaunchKernelGGL(k_sum_slices, dim3((unsigned)((n + nt - 1) / nt)), dim3(nt), 0, s, part,
+                       nslice, group, n, row, ostride, acc, out);
 }
 
 R2Args r2_args(const pgd::DftData& d)
@@ -338,6 +574,10 @@ int slices_for(long long outputs, long long inputs, int nshot = 1)
     return s;
 }
 
+// the matrix-core kernels split a slice over the block's wavefronts, so the
+// same wavefronts are in flight with a quarter of the slices
+int mfma_slices(int slices) { return slices / kMW > 1 ? slices / kMW : 1; }
+
 }  // namespace
 
 namespace pgd {
@@ -355,26 +595,34 @@ void forward(const DftData& d, const float2* x, const float2* S, int nc, float2*
     if (nshot < 1 || d.M % nshot)
         throw pg::Error{PG_ERR_ARG, "the DFT's shots must split its samples evenly"};
     const int shot_len = d.M / nshot;
-    const int ns = slices_for(d.M, d.N);
-    const int slen = (d.N + ns - 1) / ns;
-    constexpr int NCB = 8;
-    dim3 grid(nshot * ((shot_len + kT - 1) / kT), ns, (nc + NCB - 1) / NCB);
     const R2Args r2 = r2_args(d);
-#define PG_GDFT_FWD(F64, R2)                                                                     \
-    hipLaunchKernelGGL((k_gdft_fwd<NCB, F64, R2>), grid, dim3(kT), 0, s, d.kx, d.ky, d.kz, d.t,  \
-                       d.ix, d.iy, d.iz, d.fm, x, S, nc, d.M, d.N, slen, shot_len, s_shot, part, \
-                       r2)
+    int ns;
     if (d.precision == 1) {
-        if (d.gx) PG_GDFT_FWD(true, true);
-        else PG_GDFT_FWD(true, false);
+        ns = slices_for(d.M, d.N);
+        const int slen = (d.N + ns - 1) / ns;
+        constexpr int NCB = 8;
+        const dim3 grid(nshot * ((shot_len + kT - 1) / kT), ns, (nc + NCB - 1) / NCB);
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(kT), 0, s, d.kx, d.ky, d.kz, d.t, d.ix, d.iy, d.iz,
+                               d.fm, x, S, nc, d.M, d.N, slen, shot_len, s_shot, part, r2);
+        };
+        d.gx ? launch(k_gdft_fwd<NCB, true>) : launch(k_gdft_fwd<NCB, false>);
     } else {
-        if (d.gx) PG_GDFT_FWD(false, true);
-        else PG_GDFT_FWD(false, false);
+        ns = mfma_slices(slices_for(d.M, d.N));
+        const int slen = (d.N + ns - 1) / ns;
+        auto launch = [&](auto kern, int coils) {
+            hipLaunchKernelGGL(kern, dim3(nshot * ((shot_len + 63) / 64), ns, (nc + coils - 1) / coils),
+                               dim3(64 * kMW), 0, s, d.kx, d.ky, d.kz, d.t, d.ix, d.iy, d.iz, d.fm, x,
+                               S, nc, d.M, d.N, slen, shot_len, s_shot, part, r2);
+        };
+        // columns for 8 or (in chunks of) 16 coils
+        if (nc <= 8)
+            d.gx ? launch(k_gdft_fwd_mfma<1, true>, 8) : launch(k_gdft_fwd_mfma<1, false>, 8);
+        else
+            d.gx ? launch(k_gdft_fwd_mfma<2, true>, 16) : launch(k_gdft_fwd_mfma<2, false>, 16);
     }
-#undef PG_GDFT_FWD
     const long long n = (long long)nc * d.M;
-    hipLaunchKernelGGL(k_sum_slices, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, part, ns, ns,
-                       n, (long long)d.M, ostride, 0, out);
+    sum_slices(part, ns, ns, n, (long long)d.M, ostride, 0, out, s);
 }
 
 void adjoint(const DftData& d, const float2* y, const float2* S, int nc, float2* out, float2* part,
@@ -384,26 +632,31 @@ void adjoint(const DftData& d, const float2* y, const float2* S, int nc, float2*
     if (nshot < 1 || d.M % nshot)
         throw pg::Error{PG_ERR_ARG, "the DFT's shots must split its samples evenly"};
     const int shot_len = d.M / nshot;
-    const int sps = slices_for(d.N, shot_len, nshot);
-    const int slen = (shot_len + sps - 1) / sps;
-    constexpr int NCB = 8;
-    dim3 grid((d.N + kT - 1) / kT, nshot * sps, 1);
     const R2Args r2 = r2_args(d);
-#define PG_GDFT_ADJ(F64, R2)                                                                     \
-    hipLaunchKernelGGL((k_gdft_adj<NCB, F64, R2>), grid, dim3(kT), 0, s, d.kx, d.ky, d.kz, d.t,  \
-                       d.ix, d.iy, d.iz, d.fm, y, ystride, S, nc, d.M, d.N, slen, shot_len,      \
-                       s_shot, part, r2)
+    int sps = slices_for(d.N, shot_len, nshot);
+    if (d.precision != 1) sps = mfma_slices(sps);
+    const int slen = (shot_len + sps - 1) / sps;
     if (d.precision == 1) {
-        if (d.gx) PG_GDFT_ADJ(true, true);
-        else PG_GDFT_ADJ(true, false);
+        constexpr int NCB = 8;
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((d.N + kT - 1) / kT, nshot * sps), dim3(kT), 0, s, d.kx,
+                               d.ky, d.kz, d.t, d.ix, d.iy, d.iz, d.fm, y, ystride, S, nc, d.M, d.N,
+                               slen, shot_len, s_shot, part, r2);
+        };
+        d.gx ? launch(k_gdft_adj<NCB, true>) : launch(k_gdft_adj<NCB, false>);
     } else {
-        if (d.gx) PG_GDFT_ADJ(false, true);
-        else PG_GDFT_ADJ(false, false);
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((d.N + 63) / 64, nshot * sps), dim3(64 * kMW), 0, s, d.kx,
+                               d.ky, d.kz, d.t, d.ix, d.iy, d.iz, d.fm, y, ystride, S, nc, d.M, d.N,
+                               slen, shot_len, s_shot, part, r2);
+        };
+        if (nc <= 8)
+            d.gx ? launch(k_gdft_adj_mfma<1, true>) : launch(k_gdft_adj_mfma<1, false>);
+        else
+            d.gx ? launch(k_gdft_adj_mfma<2, true>) : launch(k_gdft_adj_mfma<2, false>);
     }
-#undef PG_GDFT_ADJ
-    hipLaunchKernelGGL(k_sum_slices, dim3((unsigned)((d.N + 255) / 256)), dim3(256), 0, s, part,
-                       nshot * sps, sps, (long long)d.N, (long long)d.N, (long long)d.N,
-                       accumulate ? 1 : 0, out);
+    sum_slices(part, nshot * sps, sps, (long long)d.N, (long long)d.N, (long long)d.N,
+               accumulate ? 1 : 0, out, s);
 }
 
 size_t static_scratch_elems() { return kScratchElems; }
