@@ -324,14 +324,13 @@ int pg_recon_solve_batch(size_t K, const pg_op* A, const pg_penalty* R, const vo
                          void* stream);
 
 /* ---- tuning (no counterpart in the reference) ----------------------------
- * "spread_mfma" 1: the 2-D batched spread runs on the matrix cores when the
- * grid count is a multiple of 4; 0 (default): on the vector units.  Both
- * give the same sums up to FP32 rounding order.
+ * "spread_mfma", "spread_stage": accepted and without effect (the 2-D spread
+ * has one form, on the matrix cores).
  * "autotune" 1: when an operator is first prepared for a batch of B grids,
  * its Gnufft plan times each variant of the 2-D (or z-class plane) batched
  * interpolation (gather, or LDS-staged tiles with sample bins of 128 or 64)
- * and spread (vector units or matrix cores) on its own workspaces and keeps
- * the fastest for that B, overriding "spread_mfma" and "interp_lds4";
+ * on its own workspaces and keeps the fastest for that B, overriding
+ * "interp_lds4";
  * 0 (default): the fixed choice.  The variants differ in
  * FP32 summation order only, but with autotuning on, which one runs -- and
  * so the last bits of a result -- depends on the timing.
@@ -365,10 +364,6 @@ int pg_recon_solve_batch(size_t K, const pg_op* A, const pg_penalty* R, const vo
  * "zfwd_fuse" 1 (default): the forward z stage on the matrix cores (Ny 64 or
  * 128 at gridos 2) and the class planes' y FFT run as one kernel, the class
  * planes kept in LDS; 0: two kernels.  Same products, same order.
- * "spread_stage" 1 (default): the compact-row spread loads the row slices of
- * each group of up to 32 patch entries into LDS with all loads in flight,
- * then sums from LDS (when a 64-grid chunk needs at most 48 floats of a
- * row); 0: one row load per entry and lane.  Same products, same order.
  * Settings take effect for launches (and solve graphs) made after the call;
  * "zclass" for plans created after it. */
 int pg_set_tuning(const char* key, int value);
@@ -379,8 +374,8 @@ int pg_gnufft_zclasses(pg_op h, size_t* nzc);
  * or a TimeSegmentation or SENSE over one) at B grids: interp_lds 1 =
  * LDS-staged tiles with every segment at once over bins of <= 128 samples,
  * 2 = four segments at a time over bins of <= 64 samples, 0 = gather;
- * spread_mfma 1 = matrix cores, 0 = vector units; both -1 when the plan was
- * not tuned for B */
+ * spread_mfma 1 = matrix cores (the one form); both -1 when the plan was not
+ * tuned for B */
 int pg_op_tuning(pg_op h, int B, int* interp_lds, int* spread_mfma);
 
 /* ---- measurement --------------------------------------------------------

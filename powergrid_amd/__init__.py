@@ -382,25 +382,23 @@ class SENSE(_Op):
 
 def op_tuning(op, B):
     """The kernel variants the autotuner chose for the Gnufft plan under op at
-    B grids: (interp_lds, spread_mfma), each 1/0, or (-1, -1) when untuned."""
+    B grids: (interp_lds, 1), or (-1, -1) when untuned."""
     a, b = C.c_int(), C.c_int()
     check(lib().pg_op_tuning(op.handle, int(B), C.byref(a), C.byref(b)))
     return a.value, b.value
 
 
 def set_tuning(key, value):
-    """pg_set_tuning: "spread_mfma" 1 runs the 2-D batched spread on the
-    matrix cores (grid count a multiple of 4), 0 (default) on the vector
-    units; "autotune" 1 lets each plan time its interpolation and spread
-    variants when first prepared for a grid count and keep the faster;
+    """pg_set_tuning: "spread_mfma" and "spread_stage" are accepted and have no
+    effect; "autotune" 1 lets each plan time its interpolation variants when
+    first prepared for a grid count and keep the fastest;
     "zclass" 1 (default) builds 3-D plans of stacked trajectories for z-class
     planes, 0 for the full 3-D grid (plans created afterwards); "spread_rows"
     1 (default) spreads time-segmented batches from compact sample rows (coil
     values and segment weights), 0 from rows of nc*L values; "trace" 1
     pushes roctx tracing ranges (trace()); "zfuse" 1 (default) runs the
     adjoint y IFFT and z stage of z-class planes as one kernel;
-    "spread_stage" 1 (default) stages the compact rows of each group of
-    patch entries in LDS, 0 reads them per entry; "zstage_mfma" 1 (default)
+    "zstage_mfma" 1 (default)
     forms the forward z stage's class sums on the matrix cores; "zadj_mfma"
     1 (default) the fused adjoint's, with its y IFFTs on four wavefronts;
     "zfwd_fuse" 1 (default) runs the matrix-core forward z stage and the

@@ -281,13 +281,13 @@ void Gnufft::ensure_batch(int B)
     tbuf = dev_alloc<float2>((size_t)B * std::max(g.Nz, nzc) * g.Nx * g.Gy);
     if (g.dims == 3) tbuf2 = dev_alloc<float2>((size_t)B * g.Nz * g.Gx * g.Gy);
     dev_free(vals);
-    vals = dev_alloc<float2>((size_t)M * B);
+    vals = dev_alloc<float2>((size_t)M * B + 16);  // (the spread reads whole vectors)
     dev_free(partial);
-    // 2-D patches: 16 points in chunks of 64 grids; 3-D patches: 64 points in
-    // chunks of 32
+    // 2-D patches: 16 points of every grid; 3-D patches: 64 points in chunks
+    // of 32 grids
     if (n_slots > 0)
         partial = dev_alloc<float2>(n_items3 > 0 ? (size_t)((B + 31) / 32) * n_slots * 64 * 32
-                                                 : (size_t)((B + 63) / 64) * n_slots * 16 * 64);
+                                                 : (size_t)n_slots * 16 * B);
     cap_batch = B;
 }
 
@@ -797,7 +797,8 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
             if (pass == 1) {
                 // weights of entry k (patch q, sample i) on the patch's 16 points,
                 // wx * wy formed in FP64 and rounded once
-                std::vector<float> ew((size_t)16 * std::max<long long>(1, cnt[npall]), 0.0f);
+                // (64 more: the spread reads the weights of four entries)
+                std::vector<float> ew((size_t)16 * cnt[npall] + 64, 0.0f);
                 auto fill = [&](long long q0, long long q1) {
                     for (long long q = q0; q < q1; ++q) {
                         const long long qq = q % np;
@@ -837,16 +838,22 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                 G.ent_w = dev_copy(ew.data(), ew.size());
             }
         }
-        // XCD groups: the patches in (plane, Hilbert) order over the npx x npy
-        // patch grid, cut into 8 runs of equal work; group g's blocks get ids
-        // congruent to g mod 8 (workgroups are dealt to the 8 XCDs
-        // round-robin), so a sample's row of values is read into one L2
+        // Strips of four patches that follow each other along y: 128
+        // contiguous bytes of every grid row.  A strip's patches are written by
+        // wavefronts of one block, so that they leave the L2 as whole lines:
+        // 32-byte pieces written far apart in time reach 0.75 TB/s of HBM
+        // (6.4 GB of planes: 8.6 ms), the same pieces four to a block 3.4 TB/s.
+        // XCD groups: the strips in (plane, Hilbert) order, cut into 8 runs of
+        // equal work; group g's blocks get ids congruent to g mod 8 (workgroups
+        // are dealt to the 8 XCDs round-robin), so a sample's row of values is
+        // read into one L2
         const int kXcd = 8;
+        const int nsy = (npy + 3) / 4, nst = npx * nsy;  // strips of a plane
         int hn = 1;
-        while (hn < std::max(npx, npy)) hn <<= 1;
-        std::vector<long long> hkey(np);
-        for (long long q = 0; q < np; ++q) {
-            int x = (int)(q / npy), y = (int)(q % npy);
+        while (hn < std::max(npx, nsy)) hn <<= 1;
+        std::vector<std::pair<long long, int>> horder(nst);
+        for (int q = 0; q < nst; ++q) {
+            int x = q / nsy, y = q % nsy;
             long long d = 0;
             for (int sq = hn / 2; sq > 0; sq /= 2) {
                 const int rx = (x & sq) > 0, ry = (y & sq) > 0;
@@ -859,93 +866,130 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                     std::swap(x, y);
                 }
             }
-            hkey[q] = d;
+            horder[q] = {d, q};
         }
-        std::vector<int> horder(np);
-        for (long long q = 0; q < np; ++q) horder[q] = (int)q;
-        std::stable_sort(horder.begin(), horder.end(),
-                         [&](int u, int v) { return hkey[u] < hkey[v]; });
-        auto pweight = [&](long long q) { return (double)(cnt[q + 1] - cnt[q]) + 16.0; };
-        double wtot = 0;
-        for (long long q = 0; q < npall; ++q) wtot += pweight(q);
-        std::vector<std::vector<int>> grp(kXcd);
-        {
-            double run = 0;
-            for (int p = 0; p < npl; ++p)
-                for (int q0 : horder) {
-                    const int q = (int)((long long)p * np + q0);
-                    const double mid = run + 0.5 * pweight(q);
-                    grp[std::min(kXcd - 1, (int)(mid * kXcd / wtot))].push_back(q);
-                    run += pweight(q);
-                }
-        }
+        std::sort(horder.begin(), horder.end());
+        // a strip's first patch and its number of patches (fewer than four at
+        // the end of a row)
+        auto strip = [&](int p, int st, int& n) {
+            const int x = st / nsy, y = (st % nsy) * 4;
+            n = std::min(4, npy - y);
+            return (int)((long long)p * np + (long long)x * npy + y);
+        };
         // per group: blocks of kW = kSpreadWaves wavefront items {patch, entry
         // begin, entry end, slot}.  A patch of n <= 64 kW entries is one unit
         // taking gs = 1 (n <= 64) or the power of two >= n/64 wavefronts and
         // writes the grid (slot -1); a heavier patch is cut into ceil(n/(64
         // kW)) units of kW wavefronts, each writing a partial slot that a
-        // second pass adds up in slot order.
+        // second pass adds up in slot order.  The units of a strip that take
+        // kW/4 wavefronts or fewer run in one block (their gs the largest of
+        // them; with gs = 1, two strips to a block of 8), the others by
+        // themselves, those of equal gs together.
         struct Unit {
             int q, e0, e1, slot, gs;
         };
         const int kW = kSpreadWaves, kUnitMax = kW * 64;
-        int nlg = 0;  // gs = 1, 2, ..., kW
-        while ((1 << nlg) < kW) ++nlg;
-        ++nlg;
         struct SBlock {
-            int gs;
-            int cost;
+            int gs, cost;
             int4 w[kSpreadWaves];
+        };
+        auto place = [&](SBlock& sb, int first, const Unit& un, int gs) {
+            const long long n = un.e1 - un.e0;
+            for (int w = 0; w < gs; ++w) {
+                const int e0 = (int)(un.e0 + n * w / gs), e1 = (int)(un.e0 + n * (w + 1) / gs);
+                sb.w[first + w] = make_int4(un.q, e0, e1, un.slot);
+                sb.cost = std::max(sb.cost, e1 - e0);
+            }
+        };
+        auto new_block = [&](int gs) {
+            SBlock sb;
+            sb.gs = gs;
+            sb.cost = 0;
+            for (int w = 0; w < kW; ++w) sb.w[w] = make_int4(-1, 0, 0, -1);
+            return sb;
         };
         std::vector<int4> comb;
         int nslots = 0;
         std::vector<std::vector<SBlock>> gblk(kXcd);
-        for (int gi = 0; gi < kXcd; ++gi) {
-            std::vector<std::vector<Unit>> byg(nlg);
-            for (int q : grp[gi]) {
-                const int b0 = (int)cnt[q], n = (int)(cnt[q + 1] - cnt[q]);
-                if (n > kUnitMax) {
-                    const int parts = (n + kUnitMax - 1) / kUnitMax;
-                    comb.push_back(make_int4(q, nslots, parts, 0));
-                    for (int k = 0; k < parts; ++k)
-                        byg[nlg - 1].push_back(Unit{q, b0 + (int)((long long)n * k / parts),
-                                                    b0 + (int)((long long)n * (k + 1) / parts),
-                                                    nslots + k, kW});
-                    nslots += parts;
-                    continue;
-                }
-                int gs = 1, lg = 0;
-                while ((long long)gs * 64 < n) {
-                    gs *= 2;
-                    ++lg;
-                }
-                byg[lg].push_back(Unit{q, b0, b0 + n, -1, gs});
-            }
-            for (int lg = 0; lg < nlg; ++lg) {
-                const int gs = 1 << lg, per = kW / gs;
-                auto& v = byg[lg];
-                std::stable_sort(v.begin(), v.end(),
-                                 [](const Unit& u, const Unit& w) { return u.e1 - u.e0 > w.e1 - w.e0; });
-                for (size_t k0 = 0; k0 < v.size(); k0 += per) {
-                    SBlock sb;
-                    sb.gs = gs;
-                    sb.cost = 0;
-                    for (int w = 0; w < kW; ++w) sb.w[w] = make_int4(-1, 0, 0, -1);
-                    for (int pk = 0; pk < per && k0 + pk < v.size(); ++pk) {
-                        const Unit& un = v[k0 + pk];
-                        const long long n = un.e1 - un.e0;
-                        for (int w = 0; w < gs; ++w) {
-                            const int e0 = (int)(un.e0 + n * w / gs), e1 = (int)(un.e0 + n * (w + 1) / gs);
-                            sb.w[pk * gs + w] = make_int4(un.q, e0, e1, un.slot);
-                            sb.cost = std::max(sb.cost, e1 - e0);
+        double wtot = 0;
+        for (long long q = 0; q < npall; ++q) wtot += (double)(cnt[q + 1] - cnt[q]) + 16.0;
+        {
+            double run = 0;
+            size_t at = 0;  // strips taken so far, over all planes
+            for (int gi = 0; gi < kXcd; ++gi) {
+                std::vector<Unit> alone[8];  // by log2 gs
+                std::vector<SBlock> strips;
+                int open = -1;  // the block of gs = 1 with room for a strip
+                for (; at < (size_t)npl * nst; ++at) {
+                    int ns = 0;
+                    const int q0 = strip((int)(at / nst), horder[at % nst].second, ns);
+                    double w = 0;
+                    for (int k = 0; k < ns; ++k) w += (double)(cnt[q0 + k + 1] - cnt[q0 + k]) + 16.0;
+                    if (gi + 1 < kXcd && run + 0.5 * w >= wtot * (gi + 1) / kXcd) break;
+                    run += w;
+                    std::vector<Unit> un(ns, Unit{-1, 0, 0, -1, 0});
+                    int gs = 1;
+                    for (int k = 0; k < ns; ++k) {
+                        const int q = q0 + k, b0 = (int)cnt[q], n = (int)(cnt[q + 1] - cnt[q]);
+                        if (n > kUnitMax) {
+                            const int parts = (n + kUnitMax - 1) / kUnitMax;
+                            comb.push_back(make_int4(q, nslots, parts, 0));
+                            int lg = 0;
+                            while ((1 << lg) < kW) ++lg;
+                            for (int s = 0; s < parts; ++s)
+                                alone[lg].push_back(Unit{q, b0 + (int)((long long)n * s / parts),
+                                                         b0 + (int)((long long)n * (s + 1) / parts),
+                                                         nslots + s, kW});
+                            nslots += parts;
+                            continue;
+                        }
+                        Unit u{q, b0, b0 + n, -1, 1};
+                        int lg = 0;
+                        while ((long long)u.gs * 64 < n) {
+                            u.gs *= 2;
+                            ++lg;
+                        }
+                        if (4 * u.gs > kW) {
+                            alone[lg].push_back(u);
+                        } else {
+                            un[k] = u;
+                            gs = std::max(gs, u.gs);
                         }
                     }
-                    gblk[gi].push_back(sb);
+                    const int per = kW / (4 * gs);  // strips to a block
+                    int first = 0;
+                    if (gs == 1 && open >= 0) {
+                        first = 4;
+                    } else {
+                        strips.push_back(new_block(gs));
+                        if (gs == 1 && per > 1) open = (int)strips.size() - 1;
+                    }
+                    SBlock& sb = first ? strips[open] : strips.back();
+                    for (int k = 0; k < ns; ++k)
+                        if (un[k].q >= 0) place(sb, first + k * gs, un[k], gs);
+                    if (first) open = -1;
                 }
+                for (int lg = 7; lg >= 0; --lg) {
+                    const int gs = 1 << lg, per = kW / gs;
+                    auto& v = alone[lg];
+                    std::stable_sort(v.begin(), v.end(), [](const Unit& u, const Unit& w) {
+                        return u.e1 - u.e0 > w.e1 - w.e0;
+                    });
+                    for (size_t k0 = 0; k0 < v.size(); k0 += per) {
+                        SBlock sb = new_block(gs);
+                        for (int pk = 0; pk < per && k0 + pk < v.size(); ++pk)
+                            place(sb, pk * gs, v[k0 + pk], gs);
+                        gblk[gi].push_back(sb);
+                    }
+                }
+                gblk[gi].insert(gblk[gi].end(), strips.begin(), strips.end());
+                // the longest blocks first, by stages of 32 entries (along the
+                // curve among equals)
+                std::stable_sort(gblk[gi].begin(), gblk[gi].end(),
+                                 [](const SBlock& u, const SBlock& w) {
+                                     return (u.cost + 31) / 32 > (w.cost + 31) / 32;
+                                 });
             }
-            // the longest blocks first
-            std::stable_sort(gblk[gi].begin(), gblk[gi].end(),
-                             [](const SBlock& u, const SBlock& w) { return u.cost > w.cost; });
         }
         size_t nmax = 0;
         for (int gi = 0; gi < kXcd; ++gi) nmax = std::max(nmax, gblk[gi].size());
@@ -961,7 +1005,8 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
         {
             // groups are aligned runs of gs wavefronts with one patch and slot
             // and consecutive ranges; all ranges of a patch tile its entries
-            std::vector<std::vector<std::pair<int, int>>> rng(npall);
+            std::vector<long long> seen(npall, 0);
+            std::vector<char> met(npall, 0);
             for (size_t blk = 0; blk < nmax * kXcd; ++blk) {
                 const int gs = bgs[blk];
                 for (int w = 0; w < kW; ++w) {
@@ -970,20 +1015,16 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                     PG_REQUIRE(it.x == ld.x && it.w == ld.w, PG_ERR_STATE, "spread work groups");
                     if (w % gs) PG_REQUIRE(witems[blk * kW + w - 1].z == it.y, PG_ERR_STATE, "spread work groups");
                     if (it.x < 0) continue;
-                    PG_REQUIRE(it.x < npall && it.z >= it.y, PG_ERR_STATE, "spread work list");
-                    rng[it.x].push_back({it.y, it.z});
+                    PG_REQUIRE(it.x < npall && it.z >= it.y && it.z <= it.y + 64 &&
+                                   it.y >= cnt[it.x] && it.z <= cnt[it.x + 1],
+                               PG_ERR_STATE, "spread work list");
+                    seen[it.x] += it.z - it.y;
+                    met[it.x] = 1;
                 }
             }
-            for (long long q = 0; q < npall; ++q) {
-                auto& r = rng[q];
-                std::sort(r.begin(), r.end());
-                long long at = cnt[q];
-                for (auto& pr : r) {
-                    PG_REQUIRE(pr.first == at, PG_ERR_STATE, "spread work list coverage");
-                    at = pr.second;
-                }
-                PG_REQUIRE(at == cnt[q + 1] && !r.empty(), PG_ERR_STATE, "spread work list coverage");
-            }
+            for (long long q = 0; q < npall; ++q)
+                PG_REQUIRE(met[q] && seen[q] == cnt[q + 1] - cnt[q], PG_ERR_STATE,
+                           "spread work list coverage");
         }
         G.n_comb = (int)comb.size();
         G.n_slots = nslots;
@@ -1390,9 +1431,8 @@ static void require_fft(const Gnufft& G)
 static std::atomic<int> g_autotune{0};
 
 // Times each variant of plan G's batched interpolation (LDS-staged or
-// gather) and spread (vector units or matrix cores) for nc x L grids, on the
-// plan's own workspaces (their contents do not matter for timing), and keeps
-// the faster of each.  Set-up work on the thread's set-up stream, before any
+// gather) for nc x L grids, on the plan's own workspaces (their contents do
+// not matter for timing), and keeps the fastest.  Set-up work on the thread's set-up stream, before any
 // capture; a plan is tuned once per grid count.
 static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi)
 {
@@ -1432,7 +1472,7 @@ static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi
         PG_HIP(hipEventElapsedTime(&ms, e[0], e[1]));
         return ms;
     };
-    G.tuned.push_back(Gnufft::Tuned{B, 1, 0});
+    G.tuned.push_back(Gnufft::Tuned{B, 1});
     Gnufft::Tuned& t = G.tuned.back();
     if (pgk::interp_lds_possible(G, L, AA != nullptr)) {
         // gather (0), all segments staged over bins of <= 128 samples (1),
@@ -1454,17 +1494,6 @@ static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi
         t.lds = pick;
     } else {
         t.lds = 0;
-    }
-    if (B % 4 == 0) {
-        auto spread = [&] {
-            pgk::launch_spread(G, nullptr, G.M, nc, L, AA, AAi, nullptr, nullptr, nullptr, G.grids,
-                               true, ss, planes);
-        };
-        t.mfma = 0;
-        const float ms_vec = timed(spread);
-        t.mfma = 1;
-        const float ms_mfma = timed(spread);
-        t.mfma = ms_mfma < ms_vec ? 1 : 0;
     }
     PG_HIP(hipGetLastError());
     // the fills (and any timing launch) are done before the caller's stream
@@ -3540,7 +3569,7 @@ int pg_op_tuning(pg_op h, int B, int* interp_lds, int* spread_mfma)
     PG_REQUIRE(op->kind == K_NUFFT, PG_ERR_ARG, "not a Gnufft or an operator over one");
     const Gnufft::Tuned* t = static_cast<NufftOp*>(op)->G.tuned_for(B);
     *interp_lds = t ? t->lds : -1;
-    *spread_mfma = t ? t->mfma : -1;
+    *spread_mfma = t ? 1 : -1;  // the one form of the spread
     PG_CATCH
 }
 
@@ -3559,8 +3588,8 @@ int pg_set_tuning(const char* key, int value)
 {
     PG_TRY PG_REQUIRE(key, PG_ERR_ARG, "null key");
     const std::string k(key);
-    if (k == "spread_mfma")
-        pgk::g_spread_mfma.store(value ? 1 : 0);
+    if (k == "spread_mfma" || k == "spread_stage")
+        ;  // the 2-D spread has one form
     else if (k == "zclass")
         pgk::g_zclass.store(value ? 1 : 0);
     else if (k == "spread_rows")
@@ -3575,11 +3604,6 @@ int pg_set_tuning(const char* key, int value)
         pgk::g_zamfma.store(value ? 1 : 0);
     else if (k == "zfwd_fuse")
         pgk::g_zfwd.store(value ? 1 : 0);
-
-
-    else if (k == "spread_stage")
-        pgk::g_spread_stage.store(value ? 1 : 0);
-
     else if (k == "batch_streams")
         g_batch_streams.store(value < 0 ? 0 : (value > 8 ? 8 : value));
     else if (k == "interp_lds4")

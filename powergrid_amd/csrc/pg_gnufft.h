@@ -132,10 +132,9 @@ struct Gnufft {
     // kernel variants chosen by the autotuner for a batch of B grids: the
     // interpolation as a gather (0), LDS-staged with all segments at once over
     // bins of <= kIChunk samples (1) or four segments at a time over bins of
-    // <= kIChunk4 samples (2); the matrix-core (1) or vector-unit (0) spread;
-    // no entry: the defaults
+    // <= kIChunk4 samples (2); no entry: the default
     struct Tuned {
-        int B, lds, mfma;
+        int B, lds;
     };
     std::vector<Tuned> tuned;
     const Tuned* tuned_for(int B) const

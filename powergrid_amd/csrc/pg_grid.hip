@@ -15,12 +15,12 @@
 //            holds its coils' grids.
 // spread  -- first the value of every (sample, grid) pair is formed once
 //            (AA weight, CG residual), sample-major.
-//            2-D: one wavefront per 4x4 grid patch, lane = grid
-//            (coil x segment), accumulating in registers over the samples
-//            whose window meets the patch (per-entry patch weights are
-//            precomputed); heavy patches are split into chunks of <= 64
-//            entries whose partial sums are added in a fixed order.  No
-//            atomics, no zero-fill, deterministic.
+//            2-D: 4x4 grid patches as products on the matrix cores (patch
+//            points x coils x segments) over the samples whose window meets
+//            the patch (per-entry patch weights are precomputed); heavy
+//            patches are split into runs of <= 64 entries whose sums are
+//            added in a fixed order.  No atomics, no zero-fill,
+//            deterministic.
 //            3-D: 4x4x4 patches on the matrix cores (k_spread3), or, for a few
 //            grids of a plan of z-class planes, one thread per sample with
 //            hardware float atomics into a zeroed grid (the reference's
@@ -763,653 +763,308 @@ void launch_rows(const float2* in, long long in_cstride, const float2* resid_y, 
                        nc, S, reinterpret_cast<float*>(rows));
 }
 
-// conj(a + i ai) v for the compact-row spreads, with the FMA contraction
-// written out so that every kernel forms the same bits
-__device__ __forceinline__ float2 row_conj_weight(float a, float ai, float2 v)
-{
-    return make_float2(__builtin_fmaf(a, v.x, ai * v.y), __builtin_fmaf(a, v.y, -(ai * v.x)));
-}
-
 // ------------------------------------------------- 2-D patch spread --------
-// A block of W = kSpreadWaves wavefronts; lane = grid (coil x segment).
-// Wavefront w runs the work item witems[W block + w] = {patch (-1: none),
-// entry begin, entry end, slot}: it accumulates the 4x4 patch in registers
-// over its entries.  Entry k carries its sample index and the 16 weights wx*wy of the
-// patch's points (zero outside the sample's clamped window), precomputed
-// with the trajectory.  Per stage of up to 64 entries a wavefront stages the
-// weights in LDS (read back as broadcasts) and the indices one per lane
-// (readlane); the only global load per entry is the sample's contiguous row
-// of grid values, and the next 8 rows are in flight while the current 8 are
-// summed.  A patch of 65..64 W entries is split over gs = 2..W consecutive
-// wavefronts of a block (bgs[block] = gs, the same for all groups of a
-// block), whose sums are added through LDS in a fixed tree order; the
-// group's first wavefront writes the patch, or its partial slot when the
-// patch is one of the parts of a heavier patch (added by
-// k_spread_heavy_combine).  No atomics, no zero-fill, deterministic.
+// A block of W = kSpreadWaves wavefronts; wavefront w runs the work item
+// witems[W block + w] = {patch (-1: none), entry begin, entry end, slot} of at
+// most 64 entries for one chunk of the grids: a 4x4 patch as products on the
+// matrix cores,
+//   acc_l[16 points][16 CT floats] += W[16 points][4 entries] (AA_l r)[4 entries][16 CT floats]
+// four entries a step, v_mfma_f32_16x16x4f32 (A[i][k] in lane i + 16k, B[k][j]
+// in lane j + 16k, D[i][j] in lane j + 16 (i / 4), register i % 4).  W are the
+// entries' 16 weights wx wy (ew, precomputed in FP64: a step's 64 are
+// contiguous), r the coil values of up to 8 CT coils in the entry's sample row
+// (re and im as separate columns, lane j holding floats CT j .. CT j + CT - 1)
+// and AA_l its weights of up to NL segments, so a chunk is NL segments of 8 CT
+// coils; the rows are those of k_spread_rows (stride S: nc coil values, then
+// L weights, and for MODE 2 their L imaginary parts: conj(AA) r).  MODE 0: no
+// weights, the rows hold the nc = B grid values themselves (L = 1).
+// A patch of 65 .. 64 W entries is split over gs = 2 .. W consecutive
+// wavefronts of a block (bgs[block] = gs, the same for all groups of a block),
+// whose sums are added through LDS in a fixed tree order; the group's first
+// wavefront writes the patch, or its partial slot when the patch is one of the
+// parts of a heavier patch (added by k_spread_heavy_combine).  No atomics, no
+// zero-fill, deterministic.
+//
+// Why this form.  With a lane per grid and the 16 sums of a patch in registers
+// (the rows staged in LDS) an entry took 32 FMAs and some 18 more vector
+// instructions per 64 grids, 200 clocks, and five LDS broadcasts; here it takes
+// 64 clocks of the matrix cores and some 60 of the vector units.  The patches
+// of a strip of 16 points along y belong to one block and leave the L2 as
+// whole lines (in any order of patches 32-byte pieces reach 0.75 TB/s: 8.6 ms
+// for the 6.4 GB of the planes below), and the chunks of a block follow each
+// other on one XCD, whose L2 then holds their shared rows and weights (6.0 ->
+// 0.55 GB read).  Measured: 384 grids on 32 planes of 256^2, 524288 samples
+// (32 coils, 12 segments): 4.92 ms -> 3.03 with the lane per grid in these
+// orders -> 2.45 (6.9 GB, 2.8 TB/s; matrix cores 34% busy, vector units 36%);
+// 64 grids of 256^2, 32768 samples (8 coils, 8 segments): 30.6 -> 26 us; 4 grids
+// of 128^2, 4096 samples: 13.0 -> 4.7 us.
 using pg::kSpreadWaves;
-
-// ROWS = 1 (2: complex weights): the entries' values are formed from the
-// compact rows of k_spread_rows (stride S floats, nc coils, L segments):
-// lane b = c L + l reads r_c at row + 2c and AA_l at row + 2 nc + l, and
-// forms AA_l r_c with spread_value's products (conj(AA) r for complex AA).
-template <int ROWS>
-__global__ void __launch_bounds__(64 * kSpreadWaves) k_spread_patch(
-    const int4* __restrict__ witems, const int* __restrict__ bgs, const int* __restrict__ entries,
-    const float4* __restrict__ ew, int npy, const float2* __restrict__ V, int B,
-    float2* __restrict__ grids, long long G, int Gy, float2* __restrict__ partial, int n_slots,
-    int npp, long long pstride, int L, int S)
-{
-    __shared__ float2 red[kSpreadWaves / 2][16][64];
-    __shared__ float4 sw[kSpreadWaves][64][4];
-    // wave-uniform (scalar) work item: its loop bounds live in SGPRs
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int4 it = witems[blockIdx.x * kSpreadWaves + wv];
-    const int gs = bgs[blockIdx.x];
-    const int b = blockIdx.y * 64 + lane;
-    const bool active = b < B;
-    const int bb = active ? b : B - 1;
-
-    float2 acc[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = make_float2(0.f, 0.f);
-    const float2* Vb = V + bb;
-    // compact rows: this lane's coil and segment offsets within a row
-    const int lc = ROWS ? bb / L : 0, ll = ROWS ? bb - lc * L : 0;
-    const int nc = ROWS ? B / L : 0;
-    const float* Rf = reinterpret_cast<const float*>(V);
-    const int roff = 2 * lc, aoff = 2 * nc + ll;
-    constexpr int U = 8;  // entries per group
-    float4(*mw)[4] = sw[wv];
-    for (int s0 = it.y; s0 < it.z; s0 += 64) {
-        const int n = min(64, it.z - s0);
-        // stage weights and indices; the weights of rows past n are zero (the
-        // sums below read every row of a group of 8 and mask only the values,
-        // so a stale row would otherwise enter as 0 * stale)
-        const bool ok = lane < n;
-        const int e = ok ? s0 + lane : s0;
-        const int ei = entries[e];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float4 q = ew[4 * e + r];
-            mw[lane][r] = ok ? q : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        pgf::wave_lds_sync();
-        // rows of group k0; entries past n load the last entry's row, which
-        // is zeroed with a bit mask where it is used (no branch around the
-        // loads, so that the next group's loads stay in flight while this
-        // group is summed)
-        auto load_group = [&](int k0, float2 (&v)[U], float (&a)[U], float (&ai)[U]) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = __builtin_amdgcn_readlane(ei, min(k0 + u, n - 1));
-                if (ROWS) {
-                    const float* row = Rf + (long long)i * S;
-                    v[u] = *reinterpret_cast<const float2*>(row + roff);
-                    a[u] = row[aoff];
-                    if (ROWS == 2) ai[u] = row[aoff + L];
-                } else {
-                    v[u] = Vb[(long long)i * B];
-                }
-            }
-        };
-        // sum group k0 (rows in v) into the patch
-        auto sum_group = [&](int k0, float2 (&v)[U], float (&a)[U], float (&ai)[U]) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int m = (k0 + u < n) ? -1 : 0;
-                float2 val = v[u];
-                if (ROWS == 1) val = make_float2(a[u] * val.x, a[u] * val.y);
-                if (ROWS == 2)
-                    val = row_conj_weight(a[u], ai[u], val);
-                const float2 vu = make_float2(__int_as_float(__float_as_int(val.x) & m),
-                                              __int_as_float(__float_as_int(val.y) & m));
-                const int k = min(k0 + u, 63);
-                float w[16];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float4 q4 = mw[k][r];
-                    w[4 * r] = q4.x;
-                    w[4 * r + 1] = q4.y;
-                    w[4 * r + 2] = q4.z;
-                    w[4 * r + 3] = q4.w;
-                }
-#pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    acc[q].x += w[q] * vu.x;
-                    acc[q].y += w[q] * vu.y;
-                }
-            }
-        };
-        // two row buffers in turn (the scheduling barriers keep each group's
-        // loads ahead of the sums; the second group is summed
-        // unconditionally, masked past n, so that its loads are not sunk next
-        // to their use)
-        float2 va[U], vb[U];
-        float aa[U], ab[U], aia[U], aib[U];
-        load_group(0, va, aa, aia);
-        for (int k0 = 0; k0 < n; k0 += 2 * U) {
-            load_group(k0 + U, vb, ab, aib);
-            __builtin_amdgcn_sched_barrier(0);
-            sum_group(k0, va, aa, aia);
-            load_group(k0 + 2 * U, va, aa, aia);
-            __builtin_amdgcn_sched_barrier(0);
-            sum_group(k0 + U, vb, ab, aib);
-        }
-        pgf::wave_lds_sync();  // the weights of the next stage replace these
-    }
-    // groups of gs wavefronts: tree sum, wavefront w + r into w
-    for (int r = 1; r < gs; r *= 2) {
-        __syncthreads();
-        if ((wv & (2 * r - 1)) == r)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) red[wv >> 1][q][lane] = acc[q];
-        __syncthreads();
-        if ((wv & (2 * r - 1)) == 0)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const float2 o = red[(wv + r) >> 1][q][lane];
-                acc[q].x += o.x;
-                acc[q].y += o.y;
-            }
-    }
-    if (!active || it.x < 0 || (wv & (gs - 1)) != 0) return;
-    if (it.w >= 0) {
-        float2* pp = partial + ((long long)blockIdx.y * n_slots + it.w) * 16 * 64 + lane;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) pp[q * 64] = acc[q];
-        return;
-    }
-    // patch it.x = plane * npp + q (plane 0 for a 2-D plan)
-    const int pln = it.x / npp, q0 = it.x - pln * npp;
-    const int px0 = (q0 / npy) * pg::kPatch, py0 = (q0 % npy) * pg::kPatch;
-    float2* g = grids + pln * pstride + (long long)b * G + (long long)px0 * Gy + py0;
-#pragma unroll
-    for (int a = 0; a < pg::kPatch; ++a)
-#pragma unroll
-        for (int q = 0; q < pg::kPatch; ++q) g[(long long)a * Gy + q] = acc[a * 4 + q];
-}
-
-// The same patch spread from compact rows with each stage's row slices
-// staged in LDS.  A stage takes up to kStEntries entries; the wavefront's
-// 64 grids b0 .. b0+63 use coils c_lo .. c_hi and all L segments, i.e. the
-// float runs [2 c_lo, 2 c_hi + 2) and [2 nc, 2 nc + F2) of each entry's row
-// (F2 = L, or 2L for complex weights, rounded up to even).  The lanes load
-// those F = F1 + F2 floats of every entry of the stage as float2 units, all
-// in flight together, and store them to LDS; the sums then read each
-// entry's coil value and segment weight from LDS (a broadcast for the lanes
-// of one coil) instead of from global memory, so a stage waits for memory
-// once instead of once per group of entries.  Same values, products and
-// summation order as k_spread_patch.  FM (32 or 48) bounds the floats staged
-// per entry; the 32-float form keeps 48 KB of LDS and 80 VGPRs per block of
-// 8 wavefronts, so six wavefronts per SIMD.  Requires F <= FM for every
-// 64-grid chunk (checked by the launch).
-constexpr int kStEntries = 32;
-constexpr int kStFloats = 48;  // the largest row slice staged per entry
-
-template <int ROWS, int FM>
-__global__ void __launch_bounds__(64 * kSpreadWaves, FM <= 32 ? 6 : 4) k_spread_patch_st(
-    const int4* __restrict__ witems, const int* __restrict__ bgs, const int* __restrict__ entries,
-    const float4* __restrict__ ew, int npy, const float2* __restrict__ V, int B,
-    float2* __restrict__ grids, long long G, int Gy, float2* __restrict__ partial, int n_slots,
-    int npp, long long pstride, int L, int S)
-{
-    static_assert(ROWS == 1 || ROWS == 2, "compact rows only");
-    constexpr int NE = kStEntries;
-    constexpr int NU = (NE * FM / 2 + 63) / 64;  // float2 row loads per lane per stage
-    // the stage rows of the block's wavefronts, reused for the tree sum after the
-    // last stage (red: [kSpreadWaves / 2][16][64] float2)
-    constexpr int POOL = kSpreadWaves * NE * FM > kSpreadWaves / 2 * 16 * 64 * 2
-                             ? kSpreadWaves * NE * FM
-                             : kSpreadWaves / 2 * 16 * 64 * 2;
-    __shared__ __align__(16) float pool[POOL];
-    __shared__ float4 sw[kSpreadWaves][NE][4];
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    // blocks (patch block, 64-grid chunk), patch blocks fastest: the blocks
-    // that run together write different patches, spread over the memory
-    // channels (the chunks of one patch block write 64-grid-apart rows of
-    // the same addresses, which run together measured 40% slower)
-    const int chunk = blockIdx.y;
-    const int4 it = witems[blockIdx.x * kSpreadWaves + wv];
-    const int gs = bgs[blockIdx.x];
-    const int b0 = chunk * 64;
-    const int b = b0 + lane;
-    const bool active = b < B;
-    const int bb = active ? b : B - 1;
-    const int nc = B / L;
-    const int lc = bb / L, ll = bb - lc * L;
-    const int c_lo = b0 / L, c_hi = (min(b0 + 64, B) - 1) / L;
-    const int F1 = 2 * (c_hi - c_lo + 1);
-    const int F2 = ((ROWS == 2 ? 2 * L : L) + 1) & ~1;
-    const int U2 = (F1 + F2) / 2;        // float2 units per entry
-    const int F = 2 * U2;                // LDS floats per entry
-    const int qd = 64 / U2, qr = 64 - qd * U2;
-    float* rows = pool + wv * NE * FM;
-    float4(*mw)[4] = sw[wv];
-    const float* Rf = reinterpret_cast<const float*>(V);
-    const int voff = 2 * (lc - c_lo), aoff = F1 + ll;
-
-    float2 acc[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = make_float2(0.f, 0.f);
-    for (int s0 = it.y; s0 < it.z; s0 += NE) {
-        const int n = min(NE, it.z - s0);
-        const bool ok = lane < n;
-        const int e = ok ? s0 + lane : s0;
-        const int ei = entries[e];
-        // the stage's weights: lane k < n loads entry k's 64 bytes through a
-        // buffer resource of n entries (other lanes read zeros), all four
-        // loads issued before the rows' (no branch, no wait between them)
-        float4 wq[4];
-        {
-            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-                (void*)(ew + 4 * (long long)s0), (short)0, n * 64, kBufferWord3);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                wq[r] = __builtin_bit_cast(
-                    float4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 64 + r * 16, 0, 0));
-        }
-        // unit t = lane + 64 j of the stage: entry k = t / U2, unit u = t % U2
-        float2 rv[NU];
-        {
-            // the rows through one buffer resource (32-bit byte offsets: the
-            // launch keeps M S 4 below 2^31)
-            const __amdgpu_buffer_rsrc_t rrow = __builtin_amdgcn_make_buffer_rsrc(
-                (void*)Rf, (short)0, 0x7fffffff, kBufferWord3);
-            int k = lane / U2, u = lane - (lane / U2) * U2;
-            // formed anew per stage (kept out of registers across stages)
-            asm volatile("" : "+v"(k), "+v"(u));
-#pragma unroll
-            for (int j = 0; j < NU; ++j) {
-                const int src = __shfl(ei, min(k, n - 1), 64);
-                const int off = u < U2 - F2 / 2 ? 2 * c_lo + 2 * u : 2 * nc + 2 * (u - (U2 - F2 / 2));
-                rv[j] = __builtin_bit_cast(
-                    float2, __builtin_amdgcn_raw_buffer_load_b64(rrow, (src * S + off) * 4, 0, 0));
-                k += qd;
-                u += qr;
-                if (u >= U2) {
-                    u -= U2;
-                    ++k;
-                }
-            }
-        }
-        if (lane < NE) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mw[lane][r] = wq[r];
-        }
-        // every unit t < 64 NU <= NE FM / 2 lies in the wavefront's rows;
-        // those past n U2 are never read
-        static_assert(64 * NU <= NE * FM / 2, "stage rows");
-#pragma unroll
-        for (int j = 0; j < NU; ++j)
-            *reinterpret_cast<float2*>(rows + 2 * (lane + 64 * j)) = rv[j];
-        pgf::wave_lds_sync();
-#pragma unroll 1
-        for (int k = 0; k < n; ++k) {
-            const float* row = rows + k * F;
-            float2 val = *reinterpret_cast<const float2*>(row + voff);
-            const float a = row[aoff];
-            if (ROWS == 1) val = make_float2(a * val.x, a * val.y);
-            if (ROWS == 2) {
-                const float ai = row[aoff + L];
-                val = row_conj_weight(a, ai, val);
-            }
-            float w[16];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float4 q4 = mw[k][r];
-                w[4 * r] = q4.x;
-                w[4 * r + 1] = q4.y;
-                w[4 * r + 2] = q4.z;
-                w[4 * r + 3] = q4.w;
-            }
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                acc[q].x += w[q] * val.x;
-                acc[q].y += w[q] * val.y;
-            }
-        }
-        pgf::wave_lds_sync();  // the next stage replaces these rows and weights
-    }
-    float2(*red)[16][64] = reinterpret_cast<float2(*)[16][64]>(pool);
-    for (int r = 1; r < gs; r *= 2) {
-        __syncthreads();
-        if ((wv & (2 * r - 1)) == r)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) red[wv >> 1][q][lane] = acc[q];
-        __syncthreads();
-        if ((wv & (2 * r - 1)) == 0)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const float2 o = red[(wv + r) >> 1][q][lane];
-                acc[q].x += o.x;
-                acc[q].y += o.y;
-            }
-    }
-    if (!active || it.x < 0 || (wv & (gs - 1)) != 0) return;
-    if (it.w >= 0) {
-        float2* pp = partial + ((long long)chunk * n_slots + it.w) * 16 * 64 + lane;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) pp[q * 64] = acc[q];
-        return;
-    }
-    const int pln = it.x / npp, q0 = it.x - pln * npp;
-    const int px0 = (q0 / npy) * pg::kPatch, py0 = (q0 % npy) * pg::kPatch;
-    // each patch row is 32 contiguous bytes at a 32-byte boundary (py0, Gy
-    // and the plane and grid strides are multiples of 4 points): two
-    // 16-byte stores per row
-    float2* g = grids + pln * pstride + (long long)b * G + (long long)px0 * Gy + py0;
-#pragma unroll
-    for (int a = 0; a < pg::kPatch; ++a) {
-        float4* g4 = reinterpret_cast<float4*>(g + (long long)a * Gy);
-        g4[0] = make_float4(acc[a * 4].x, acc[a * 4].y, acc[a * 4 + 1].x, acc[a * 4 + 1].y);
-        g4[1] = make_float4(acc[a * 4 + 2].x, acc[a * 4 + 2].y, acc[a * 4 + 3].x, acc[a * 4 + 3].y);
-    }
-}
-
-// the largest staged floats per entry of a launch's 64-grid chunks
-int spread_st_floats(int B, int L, bool cpx)
-{
-    int fm = 0;
-    for (int b0 = 0; b0 < B; b0 += 64) {
-        const int f1 = 2 * ((std::min(b0 + 64, B) - 1) / L - b0 / L + 1);
-        fm = std::max(fm, f1 + (((cpx ? 2 * L : L) + 1) & ~1));
-    }
-    return fm;
-}
-
-// The same work list on the matrix cores (B a multiple of 4).  For a chunk of
-// 4 entries the patch update is a product
-//   acc[16 points][128 floats] += W[16 points][4 entries] * V[4 entries][128 floats]
-// of the entries' weights and their rows of grid values (re and im as
-// separate columns), done as 8 v_mfma_f32_16x16x4f32, one per 16-column
-// tile.  Tile t, column j holds row float 8j + t, so that each lane's share
-// of a row is 8 consecutive floats (two 16-byte loads).  Lane layouts of the
-// 16x16x4 f32 product (one block): A[i][k] in lane i + 16k, B[k][j] in lane
-// j + 16k, D[i][j] in lane j + 16(i/4), register i % 4.
 typedef float pg_f4 __attribute__((ext_vector_type(4)));
+typedef float pg_f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float pg_f2u __attribute__((ext_vector_type(2), aligned(4)));
 
-__global__ void __launch_bounds__(64 * kSpreadWaves) k_spread_patch_mfma(
-    const int4* __restrict__ witems, const int* __restrict__ bgs, const int* __restrict__ entries,
-    const float4* __restrict__ ew, int npy, const float2* __restrict__ V, int B,
-    float2* __restrict__ grids, long long G, int Gy, float2* __restrict__ partial, int n_slots,
-    int npp, long long pstride)
+// a lane's neighbour in its pair (quad_perm [1,0,3,2])
+__device__ __forceinline__ float pair_swap(float v)
 {
-    __shared__ float red[kSpreadWaves / 2][32][64];
-    __shared__ float sw[kSpreadWaves][64][16];
-    __shared__ int si[kSpreadWaves][64];
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int4 it = witems[blockIdx.x * kSpreadWaves + wv];
-    const int gs = bgs[blockIdx.x];
-    const int cw = min(64, B - 64 * (int)blockIdx.y);  // grids in this chunk (multiple of 4)
-    const int kq = lane >> 4, jq = lane & 15;          // MFMA k (entry) and j (column) of this lane
-    const bool colok = 4 * jq < cw;                     // this lane's 4 grids exist
-    // this lane's 8 floats of a row: grids 4jq .. 4jq+3 of the chunk
-    const float* Vc = reinterpret_cast<const float*>(V) + 2 * 64 * (long long)blockIdx.y +
-                      8 * (colok ? jq : 0);
-    const long long rowf = 2LL * B;  // floats per sample row
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
+}
 
-    pg_f4 acc[8];
+template <int N>
+__device__ __forceinline__ void load_floats(const float* p, float (&v)[N])
+{
+    if constexpr (N == 1) {
+        v[0] = p[0];
+    } else if constexpr (N == 2) {
+        const pg_f2u q = *reinterpret_cast<const pg_f2u*>(p);
+        v[0] = q[0];
+        v[1] = q[1];
+    } else {
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = pg_f4{0.f, 0.f, 0.f, 0.f};
-    float(*mw)[16] = sw[wv];
-    int* mi = si[wv];
-    for (int s0 = it.y; s0 < it.z; s0 += 64) {
-        const int n = min(64, it.z - s0);
-        {
-            // stage weights and indices; entries past n get zero weights
-            const bool ok = lane < n;
-            const int e = ok ? s0 + lane : s0;
-            mi[lane] = entries[e];
+        for (int u = 0; u < N / 4; ++u) {
+            const pg_f4u q = *reinterpret_cast<const pg_f4u*>(p + 4 * u);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float4 q = ew[4 * e + r];
-                mw[lane][4 * r] = ok ? q.x : 0.f;
-                mw[lane][4 * r + 1] = ok ? q.y : 0.f;
-                mw[lane][4 * r + 2] = ok ? q.z : 0.f;
-                mw[lane][4 * r + 3] = ok ? q.w : 0.f;
-            }
+            for (int t = 0; t < 4; ++t) v[4 * u + t] = q[t];
         }
-        pgf::wave_lds_sync();
-        // rows of chunk k0 for this lane (entry k0 + kq; past n: zeroed)
-        auto load_chunk = [&](int k0, float4 (&v)[2]) {
-            const int k = min(k0 + kq, 63);
-            const float4* src = reinterpret_cast<const float4*>(Vc + rowf * mi[k]);
-            v[0] = src[0];
-            v[1] = src[1];
-        };
-        auto mma_chunk = [&](int k0, float4 (&v)[2]) {
-            const int m = (k0 + kq < n && colok) ? -1 : 0;
-            const float a = mw[min(k0 + kq, 63)][jq];  // A[point jq][entry kq]
-            float b[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
+    }
+}
+
+template <int CT, int NL, int MODE>
+__global__ void __launch_bounds__(64 * kSpreadWaves) k_spread2(
+    const int4* __restrict__ witems, const int* __restrict__ bgs, const int* __restrict__ entries,
+    const float* __restrict__ ew, int npy, const float* __restrict__ rows, int S, int nc, int L,
+    int ncc, int nch, float2* __restrict__ grids, long long G, int Gy,
+    float2* __restrict__ partial, int B, int npp, long long pstride, int gather)
+{
+    static_assert(MODE || NL == 1, "value rows have no segments");
+    constexpr int NA = 4 * NL * CT;  // floats of the patch per lane
+    // the block's strips on their way out: LP segments at a time, per coil 4
+    // rows of 16 points (the coils' 128 floats 4 apart, against bank conflicts)
+    constexpr int LP = NL * CT > 4 ? 4 / CT : NL;
+    constexpr int CP = 132;
+    constexpr int NS = kSpreadWaves / 4;  // strips of a block (gs = 1)
+    constexpr int POOL = NA * 64 * kSpreadWaves / 2 > NS * LP * 8 * CT * CP
+                             ? NA * 64 * kSpreadWaves / 2
+                             : NS * LP * 8 * CT * CP;
+    __shared__ __align__(16) float pool[POOL];
+    float(*red)[NA][64] = reinterpret_cast<float(*)[NA][64]>(pool);
+    // wave-uniform (scalar) work item
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    // block id: XCD, chunk, block of that XCD (chunks fastest)
+    const int pr = blockIdx.x >> 3, chunk = pr % nch;
+    const int blk = (pr / nch) * 8 + (blockIdx.x & 7);
+    const int4 it = witems[blk * kSpreadWaves + wv];
+    const int gs = bgs[blk];
+    const int c0 = (chunk % ncc) * 8 * CT, l0 = (chunk / ncc) * NL;
+    const int nf = 2 * min(8 * CT, nc - c0), nl = min(NL, L - l0);
+    const int i = lane & 15, k = lane >> 4;
+    // this lane's floats of a row; past the chunk's its last ones (those
+    // columns are never stored), an odd coil's last pair moved into place (CT
+    // 4, nf % 4 == 2; a last chunk of one coil reads from the coil before it)
+    const int ro = 2 * c0 + min(CT * i, nf - CT);
+    const bool shifted = CT == 4 && CT * i + CT > nf && CT * i < nf;
+    pg_f4 acc[NL][CT];
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const float bt = __int_as_float(__float_as_int(b[t]) & m);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bt, acc[t], 0, 0, 0);
+    for (int l = 0; l < NL; ++l)
+#pragma unroll
+        for (int t = 0; t < CT; ++t) acc[l][t] = pg_f4{0.f, 0.f, 0.f, 0.f};
+
+    // groups of U steps, the next group's loads in flight during this group's
+    // products
+    constexpr int U = 2;
+    const int n = it.z - it.y;  // <= 64
+    float w[2][U], v[2][U][CT], a[2][U][NL], ai[2][U][MODE == 2 ? NL : 1];
+    if (n > 0) {
+        const int es = entries[it.y + min(lane, n - 1)];
+        const float* ewl = ew + 16LL * it.y + lane;
+        auto load_group = [&](int s, int q) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                // (steps past the end: the last step's weights, the last entry)
+                w[q][u] = ewl[64 * min(s + u, (n - 1) >> 2)];
+                const int si = __shfl(es, min(4 * (s + u) + k, n - 1), 64);
+                const float* row = rows + (long long)si * S;
+                load_floats<CT>(row + ro, v[q][u]);
+                if (MODE) load_floats<NL>(row + 2 * nc + l0, a[q][u]);
+                if constexpr (MODE == 2) load_floats<NL>(row + 2 * nc + L + l0, ai[q][u]);
             }
         };
-        float4 va[2], vb[2];
-        load_chunk(0, va);
-        for (int k0 = 0; k0 < n; k0 += 8) {
-            load_chunk(k0 + 4, vb);
+        auto sum_group = [&](int s, int q) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                // entries past the end (the last one again): zero weights
+                const float wm = 4 * (s + u) + k < n ? w[q][u] : 0.f;
+                float vm[CT];
+#pragma unroll
+                for (int t = 0; t < CT; ++t) {
+                    vm[t] = v[q][u][t];
+                    if (CT == 4 && t < 2) vm[t] = shifted ? v[q][u][(t + 2) % CT] : vm[t];
+                }
+                // conj(a + i ai) r: the partner of each float, signed
+                float vx[MODE == 2 ? CT : 1];
+                if constexpr (MODE == 2) {
+#pragma unroll
+                    for (int t = 0; t < CT; ++t) {
+                        const float o = CT == 1 ? pair_swap(vm[0]) : vm[(t ^ 1) % CT];
+                        vx[t] = (CT == 1 ? (i & 1) : (t & 1)) ? -o : o;
+                    }
+                }
+#pragma unroll
+                for (int l = 0; l < NL; ++l) {
+                    if (NL > 1 && l >= nl) break;
+#pragma unroll
+                    for (int t = 0; t < CT; ++t) {
+                        float b = vm[t];
+                        if (MODE == 1) b = a[q][u][l] * b;
+                        if constexpr (MODE == 2)
+                            b = __builtin_fmaf(a[q][u][l], b, ai[q][u][l] * vx[t]);
+                        acc[l][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wm, b, acc[l][t], 0, 0, 0);
+                    }
+                }
+            }
+        };
+        load_group(0, 0);
+        for (int s = 0; 4 * s < n; s += 2 * U) {
+            load_group(s + U, 1);
             __builtin_amdgcn_sched_barrier(0);
-            mma_chunk(k0, va);
-            load_chunk(k0 + 8, va);
+            sum_group(s, 0);
+            load_group(s + 2 * U, 0);
             __builtin_amdgcn_sched_barrier(0);
-            mma_chunk(k0 + 4, vb);
+            sum_group(s + U, 1);
         }
-        pgf::wave_lds_sync();  // the next stage's weights replace these
     }
     // groups of gs wavefronts: tree sum, wavefront w + r into w
     for (int r = 1; r < gs; r *= 2) {
         __syncthreads();
         if ((wv & (2 * r - 1)) == r)
 #pragma unroll
-            for (int t = 0; t < 8; ++t)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) red[wv >> 1][4 * t + q][lane] = acc[t][q];
+            for (int q = 0; q < NA; ++q) red[wv >> 1][q][lane] = acc[q / (4 * CT)][q / 4 % CT][q % 4];
         __syncthreads();
         if ((wv & (2 * r - 1)) == 0)
 #pragma unroll
-            for (int t = 0; t < 8; ++t)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc[t][q] += red[(wv + r) >> 1][4 * t + q][lane];
+            for (int q = 0; q < NA; ++q)
+                acc[q / (4 * CT)][q / 4 % CT][q % 4] += red[(wv + r) >> 1][q][lane];
     }
-    if (it.x < 0 || (wv & (gs - 1)) != 0 || !colok) return;
-    // lane holds points p = 4 kq + q and grids b = 4 jq + u (re: tile 2u, im: tile 2u+1)
-    const int b0 = 64 * blockIdx.y + 4 * jq;
-    if (it.w >= 0) {
-        float2* pp = partial + ((long long)blockIdx.y * n_slots + it.w) * 16 * 64;
+    // lane: points (row k, y = 0 .. 3), floats CT i + t of the chunk's coils
+    const bool owner = it.x >= 0 && (wv & (gs - 1)) == 0 && CT * i < nf;
+    if (gather && 4 * gs <= kSpreadWaves) {
+        // strips: four patches along y, of gs wavefronts each, gathered in LDS
+        // and stored as whole 128-byte rows, 8 lanes a row
+        const int lgs = gs >> 1;  // log2 gs (1 or 2)
+        const int st = wv >> (2 + lgs), pi = wv >> lgs & 3;
+        // where this thread's piece of a row lies in a grid, per strip (-1:
+        // its patch is not of this block)
+        const int y2 = threadIdx.x & 7, row = threadIdx.x >> 3 & 3;
+        static_assert(NS <= 2, "two strips to a block");
+        long long off[NS];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int t = 0; t < NS; ++t) {
+            const int at = (4 * t + (y2 >> 1)) << lgs;
+            const int pt = at < kSpreadWaves ? witems[blk * kSpreadWaves + at].x : -1;
+            const int pln = pt / npp, p0 = pt - pln * npp;
+            off[t] = pt < 0 ? -1
+                            : pln * pstride + (long long)((p0 / npy) * pg::kPatch + row) * Gy +
+                                  (p0 % npy) * pg::kPatch + 2 * (y2 & 1);
+        }
+        for (int lb = 0; lb < nl; lb += LP) {
+            __syncthreads();
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                pp[(4 * kq + q) * 64 + 4 * jq + u] = make_float2(acc[2 * u][q], acc[2 * u + 1][q]);
+            for (int l = 0; l < NL; ++l) {
+                if (l < lb || l >= lb + LP || l >= nl || !owner) continue;
+                float* sp = pool + (st * LP + l - lb) * 8 * CT * CP + k * 32 + 8 * pi;
+                if constexpr (CT == 1) {
+                    // a pair of lanes holds a coil: the even one takes points
+                    // 0 and 1, the odd one 2 and 3
+                    const bool odd = i & 1;
+                    const pg_f4 o = acc[l][0];
+                    const float p0 = pair_swap(odd ? o[0] : o[2]);
+                    const float p1 = pair_swap(odd ? o[1] : o[3]);
+                    reinterpret_cast<float4*>(sp + (i >> 1) * CP)[i & 1] =
+                        odd ? make_float4(p0, o[2], p1, o[3]) : make_float4(o[0], p0, o[1], p1);
+                } else {
+#pragma unroll
+                    for (int h = 0; h < CT / 2; ++h) {
+                        const pg_f4 re = acc[l][(2 * h) % CT], im = acc[l][(2 * h + 1) % CT];
+                        float4* g4 = reinterpret_cast<float4*>(sp + ((CT / 2) * i + h) * CP);
+                        g4[0] = make_float4(re[0], im[0], re[1], im[1]);
+                        g4[1] = make_float4(re[2], im[2], re[3], im[3]);
+                    }
+                }
+            }
+            __syncthreads();
+            // pieces of 16 bytes: 8 to a row, 4 rows to a coil (thread % 32);
+            // the coils, LP segments and the block's strips in turn
+            constexpr int NC = 8 * CT, NQ = NS * LP * NC, QS = 2 * kSpreadWaves;
+#pragma unroll
+            for (int q0 = 0; q0 < NQ; q0 += QS) {
+                const int q = q0 + (int)(threadIdx.x >> 5);
+                const int c = q % NC, ll = q / NC % LP, t = q / (NC * LP);
+                const long long o = t ? off[NS - 1] : off[0];
+                if (q < NQ && t < NS / gs && 2 * c < nf && lb + ll < nl && o >= 0)
+                    *reinterpret_cast<float4*>(grids + o +
+                                               ((long long)(c0 + c) * L + l0 + lb + ll) * G) =
+                        *reinterpret_cast<const float4*>(
+                            pool + ((t * LP + ll) * NC + c) * CP + row * 32 + 4 * y2);
+            }
+        }
         return;
     }
+    if (!owner) return;
     const int pln = it.x / npp, q0 = it.x - pln * npp;
     const int px0 = (q0 / npy) * pg::kPatch, py0 = (q0 % npy) * pg::kPatch;
+    float2* gp = grids + pln * pstride + (long long)(px0 + k) * Gy + py0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int p = 4 * kq + q;
-        const long long off = pln * pstride + (long long)(px0 + p / pg::kPatch) * Gy + py0 +
-                              p % pg::kPatch;
+    for (int l = 0; l < NL; ++l) {
+        if (l >= nl) break;
+        if constexpr (CT == 1) {
+            const bool odd = i & 1;
+            const pg_f4 o = acc[l][0];
+            const float p0 = pair_swap(odd ? o[0] : o[2]), p1 = pair_swap(odd ? o[1] : o[3]);
+            const float4 d = odd ? make_float4(p0, o[2], p1, o[3]) : make_float4(o[0], p0, o[1], p1);
+            const long long b = (long long)(c0 + (i >> 1)) * L + l0 + l;
+            if (it.w >= 0) {
+                float2* pp = partial + ((long long)it.w * 16 + 4 * k + 2 * (i & 1)) * B + b;
+                pp[0] = make_float2(d.x, d.y);
+                pp[B] = make_float2(d.z, d.w);
+            } else {
+                reinterpret_cast<float4*>(gp + b * G)[i & 1] = d;
+            }
+        } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            grids[(long long)(b0 + u) * G + off] = make_float2(acc[2 * u][q], acc[2 * u + 1][q]);
-    }
-}
-
-// The matrix-core patch spread from compact rows: k_spread_patch_mfma's
-// products (8 v_mfma_f32_16x16x4f32 per chunk of 4 entries, the same lane
-// layouts) with the B operand formed from the row slices that
-// k_spread_patch_st stages in LDS.  Lane (kq, jq) supplies, for entry
-// k0 + kq, the re and im parts of grids b0 + 4 jq + u (u < 4): the value
-// AA_l r_c (conj(AA_l) r_c for complex weights) of coil c = b / L, segment
-// l = b % L, the products of k_spread_values, so the operands, and with the
-// same chunks of 4 entries the sums, are those of the value-row kernel.
-// B a multiple of 4; F <= kStFloats for every 64-grid chunk.
-template <int ROWS>
-__global__ void __launch_bounds__(64 * kSpreadWaves) k_spread_patch_mfma_st(
-    const int4* __restrict__ witems, const int* __restrict__ bgs, const int* __restrict__ entries,
-    const float4* __restrict__ ew, int npy, const float2* __restrict__ V, int B,
-    float2* __restrict__ grids, long long G, int Gy, float2* __restrict__ partial, int n_slots,
-    int npp, long long pstride, int L, int S)
-{
-    static_assert(ROWS == 1 || ROWS == 2, "compact rows only");
-    constexpr int NE = kStEntries, FM = kStFloats;
-    constexpr int NU = (NE * FM / 2 + 63) / 64;
-    constexpr int POOL = kSpreadWaves * NE * FM > kSpreadWaves / 2 * 32 * 64
-                             ? kSpreadWaves * NE * FM
-                             : kSpreadWaves / 2 * 32 * 64;
-    __shared__ __align__(16) float pool[POOL];
-    __shared__ float sw[kSpreadWaves][NE][16];
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int4 it = witems[blockIdx.x * kSpreadWaves + wv];
-    const int gs = bgs[blockIdx.x];
-    const int b0 = blockIdx.y * 64;
-    const int cw = min(64, B - b0);                     // grids in this chunk (multiple of 4)
-    const int kq = lane >> 4, jq = lane & 15;          // MFMA k (entry) and j (column) of this lane
-    const bool colok = 4 * jq < cw;                     // this lane's 4 grids exist
-    const int nc = B / L;
-    const int c_lo = b0 / L, c_hi = (b0 + cw - 1) / L;
-    const int F1 = 2 * (c_hi - c_lo + 1);
-    const int F2 = ((ROWS == 2 ? 2 * L : L) + 1) & ~1;
-    const int U2 = (F1 + F2) / 2;
-    const int F = 2 * U2;
-    const int qd = 64 / U2, qr = 64 - qd * U2;
-    float* rows = pool + wv * NE * FM;
-    float(*mw)[16] = sw[wv];
-    const float* Rf = reinterpret_cast<const float*>(V);
-    // this lane's four grids: coil value and segment weight offsets in a
-    // staged row
-    int vo[4], ao[4];
+            for (int h = 0; h < CT / 2; ++h) {
+                const int c = (CT / 2) * i + h;
+                if (2 * c >= nf) break;
+                const pg_f4 re = acc[l][(2 * h) % CT], im = acc[l][(2 * h + 1) % CT];
+                const long long b = (long long)(c0 + c) * L + l0 + l;
+                if (it.w >= 0) {
+                    float2* pp = partial + ((long long)it.w * 16 + 4 * k) * B + b;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int bq = min(b0 + 4 * jq + u, B - 1);
-        const int cq = bq / L, lq = bq - cq * L;
-        vo[u] = 2 * (cq - c_lo);
-        ao[u] = F1 + lq;
-    }
-
-    pg_f4 acc[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = pg_f4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = it.y; s0 < it.z; s0 += NE) {
-        const int n = min(NE, it.z - s0);
-        const bool ok = lane < n;
-        const int e = ok ? s0 + lane : s0;
-        const int ei = entries[e];
-        float2 rv[NU];
-        {
-            int k = lane / U2, u = lane - (lane / U2) * U2;
-            asm volatile("" : "+v"(k), "+v"(u));
-#pragma unroll
-            for (int j = 0; j < NU; ++j) {
-                const int src = __shfl(ei, min(k, n - 1), 64);
-                const int off = u < U2 - F2 / 2 ? 2 * c_lo + 2 * u : 2 * nc + 2 * (u - (U2 - F2 / 2));
-                rv[j] = *reinterpret_cast<const float2*>(Rf + (long long)src * S + off);
-                k += qd;
-                u += qr;
-                if (u >= U2) {
-                    u -= U2;
-                    ++k;
+                    for (int r = 0; r < 4; ++r) pp[(long long)r * B] = make_float2(re[r], im[r]);
+                } else {
+                    float4* g4 = reinterpret_cast<float4*>(gp + b * G);
+                    g4[0] = make_float4(re[0], im[0], re[1], im[1]);
+                    g4[1] = make_float4(re[2], im[2], re[3], im[3]);
                 }
             }
         }
-        if (lane < NE) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float4 q = ew[4 * e + r];
-                mw[lane][4 * r] = ok ? q.x : 0.f;
-                mw[lane][4 * r + 1] = ok ? q.y : 0.f;
-                mw[lane][4 * r + 2] = ok ? q.z : 0.f;
-                mw[lane][4 * r + 3] = ok ? q.w : 0.f;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < NU; ++j) {
-            const int t = lane + 64 * j;
-            if (t < n * U2) *reinterpret_cast<float2*>(rows + 2 * t) = rv[j];
-        }
-        pgf::wave_lds_sync();
-        for (int k0 = 0; k0 < n; k0 += 4) {
-            const int ke = k0 + kq;
-            const int m = (ke < n && colok) ? -1 : 0;
-            const float a = mw[min(ke, NE - 1)][jq];  // A[point jq][entry kq]
-            const float* row = rows + min(ke, n - 1) * F;
-            float b[8];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                float2 val = *reinterpret_cast<const float2*>(row + vo[u]);
-                const float w = row[ao[u]];
-                if (ROWS == 1) val = make_float2(w * val.x, w * val.y);
-                if (ROWS == 2) val = row_conj_weight(w, row[ao[u] + L], val);
-                b[2 * u] = __int_as_float(__float_as_int(val.x) & m);
-                b[2 * u + 1] = __int_as_float(__float_as_int(val.y) & m);
-            }
-#pragma unroll
-            for (int t = 0; t < 8; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[t], acc[t], 0, 0, 0);
-        }
-        pgf::wave_lds_sync();  // the next stage replaces these rows and weights
-    }
-    float(*red)[32][64] = reinterpret_cast<float(*)[32][64]>(pool);
-    for (int r = 1; r < gs; r *= 2) {
-        __syncthreads();
-        if ((wv & (2 * r - 1)) == r)
-#pragma unroll
-            for (int t = 0; t < 8; ++t)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) red[wv >> 1][4 * t + q][lane] = acc[t][q];
-        __syncthreads();
-        if ((wv & (2 * r - 1)) == 0)
-#pragma unroll
-            for (int t = 0; t < 8; ++t)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc[t][q] += red[(wv + r) >> 1][4 * t + q][lane];
-    }
-    if (it.x < 0 || (wv & (gs - 1)) != 0 || !colok) return;
-    const int bl = b0 + 4 * jq;
-    if (it.w >= 0) {
-        float2* pp = partial + ((long long)blockIdx.y * n_slots + it.w) * 16 * 64;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                pp[(4 * kq + q) * 64 + 4 * jq + u] = make_float2(acc[2 * u][q], acc[2 * u + 1][q]);
-        return;
-    }
-    const int pln = it.x / npp, q0 = it.x - pln * npp;
-    const int px0 = (q0 / npy) * pg::kPatch, py0 = (q0 % npy) * pg::kPatch;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int p = 4 * kq + q;
-        const long long off = pln * pstride + (long long)(px0 + p / pg::kPatch) * Gy + py0 +
-                              p % pg::kPatch;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            grids[(long long)(bl + u) * G + off] = make_float2(acc[2 * u][q], acc[2 * u + 1][q]);
     }
 }
 
-// patches summed in parts: add the parts' slots in slot order; block
-// (patch, grid chunk, point)
-__global__ void __launch_bounds__(64) k_spread_heavy_combine(const int4* __restrict__ comb, int npy,
-                                                             const float2* __restrict__ partial,
-                                                             int n_slots, int B,
-                                                             float2* __restrict__ grids,
-                                                             long long G, int Gy, int npp,
-                                                             long long pstride)
+// patches summed in parts: add the parts' slots (16 points x B grids) in slot
+// order; block (patch, 256 of its 16 B sums)
+__global__ void __launch_bounds__(256) k_spread_heavy_combine(
+    const int4* __restrict__ comb, int npy, const float2* __restrict__ partial, int B,
+    float2* __restrict__ grids, long long G, int Gy, int npp, long long pstride)
 {
     const int4 cb = comb[blockIdx.x];
-    const int q = blockIdx.z;
-    const int b = blockIdx.y * 64 + threadIdx.x;
-    if (b >= B) return;
-    const float2* pp = partial + ((long long)blockIdx.y * n_slots + cb.y) * 16 * 64 + q * 64 +
-                       threadIdx.x;
+    const int e = blockIdx.y * 256 + threadIdx.x;
+    if (e >= 16 * B) return;
+    const int q = e / B, b = e - q * B;
+    const float2* pp = partial + (long long)cb.y * 16 * B + e;
     float2 t = pp[0];
+#pragma unroll 4
     for (int k = 1; k < cb.z; ++k) {
-        const float2 v = pp[(long long)k * 16 * 64];
+        const float2 v = pp[(long long)k * 16 * B];
         t.x += v.x;
         t.y += v.y;
     }
@@ -1417,6 +1072,47 @@ __global__ void __launch_bounds__(64) k_spread_heavy_combine(const int4* __restr
     const int px0 = (q0 / npy) * pg::kPatch, py0 = (q0 % npy) * pg::kPatch;
     grids[pln * pstride + (long long)b * G + (long long)(px0 + q / pg::kPatch) * Gy + py0 +
           q % pg::kPatch] = t;
+}
+
+// the 2-D patches (of every z-class plane) of nc coils x L segments from rows
+// of S floats; mode as k_spread2
+void launch_spread2(const pg::Gnufft& G, const float* rows, int S, int nc, int L, int mode,
+                    float2* grids, long long gsz, long long pstride, float2* partial,
+                    hipStream_t s)
+{
+    const pg::Geometry& g = G.geo;
+    const int B = nc * L, npy = g.Gy / pg::kPatch;
+    // Whole rows through LDS where the grids outgrow the caches: written as
+    // each lane's 16 bytes, a request each, they keep the L2 busy (4e8 of them
+    // at the larger size above: 3.36 against 2.45 ms; 64 grids of 128^2 on 16
+    // planes, 134 MB: 70 against 67 us); below, the barriers cost more (34 MB:
+    // 28.6 against 30.6 us).
+    const int gather = (G.nzc > 0 && pstride ? G.nzc : 1) * (double)B * gsz * 8 > 64e6;
+    auto launch = [&](auto kern, int ct, int nseg) {
+        const int ncc = (nc + 8 * ct - 1) / (8 * ct), nch = ncc * ((L + nseg - 1) / nseg);
+        hipLaunchKernelGGL(kern, dim3((unsigned)(G.n_sblocks * nch)), dim3(64 * kSpreadWaves), 0, s,
+                           G.witems, G.bgs, G.entries, G.ent_w, npy, rows, S, nc, L, ncc, nch, grids,
+                           gsz, g.Gy, partial, B, G.npp, pstride, gather);
+    };
+    // columns for the coils there are, 8, 16 or chunks of 32, and segments for
+    // 16 or 32 sums a lane (8 coils: 4 segments at a time measured 26.2 us,
+    // 8 at a time 28.6, at the smaller size above)
+    if (mode == 0) {
+        if (nc <= 8) launch(k_spread2<1, 1, 0>, 1, 1);
+        else if (nc <= 16) launch(k_spread2<2, 1, 0>, 2, 1);
+        else launch(k_spread2<4, 1, 0>, 4, 1);
+    } else if (mode == 1) {
+        if (nc <= 8) launch(k_spread2<1, 4, 1>, 1, 4);
+        else if (nc <= 16) launch(k_spread2<2, 4, 1>, 2, 4);
+        else launch(k_spread2<4, 2, 1>, 4, 2);
+    } else {
+        if (nc <= 8) launch(k_spread2<1, 4, 2>, 1, 4);
+        else if (nc <= 16) launch(k_spread2<2, 4, 2>, 2, 4);
+        else launch(k_spread2<4, 2, 2>, 4, 2);
+    }
+    if (G.n_comb > 0)
+        hipLaunchKernelGGL(k_spread_heavy_combine, dim3(G.n_comb, (16 * B + 255) / 256), dim3(256), 0,
+                           s, G.comb, npy, partial, B, grids, gsz, g.Gy, G.npp, pstride);
 }
 
 // ------------------------------------------- 3-D patch spread ------------
@@ -1448,9 +1144,6 @@ __global__ void __launch_bounds__(64) k_spread_heavy_combine(const int4* __restr
 // with the rest of the adjoint.
 // Deterministic: entries in sample order, parts in order.  A value that is
 // not finite reaches every point of the patches its window meets.
-typedef float pg_f4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef float pg_f2u __attribute__((ext_vector_type(2), aligned(4)));
-
 constexpr int kP3Waves = 4;
 
 template <int NTP>
@@ -1791,53 +1484,11 @@ void spread_dispatch(const pg::Gnufft& G, const float2* in, long long in_cstride
         // (p*B + b)*Gx*Gy
         const long long gsz = planes ? (long long)g.Gx * g.Gy : g.G();
         const long long pstride = planes ? (long long)B * gsz : 0;
-        const int nch = (B + 63) / 64;
-        const int npy = g.Gy / pg::kPatch;
-        const pg::Gnufft::Tuned* tn = G.tuned_for(B);
-        const bool mfma =
-            B % 4 == 0 &&
-            (tn ? tn->mfma != 0 : pgk::g_spread_mfma.load(std::memory_order_relaxed) != 0);
-        if (mfma && S) {
-            // compact rows reach the matrix cores only through the staged form
-            auto launch = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3(G.n_sblocks, nch), dim3(64 * kSpreadWaves), 0, s,
-                                   G.witems, G.bgs, G.entries, (const float4*)G.ent_w, npy, vals,
-                                   B, grids, gsz, g.Gy, partial, G.n_slots, G.npp, pstride, L, S);
-            };
-            AAi ? launch(k_spread_patch_mfma_st<2>) : launch(k_spread_patch_mfma_st<1>);
-        } else if (mfma)
-            hipLaunchKernelGGL(k_spread_patch_mfma, dim3(G.n_sblocks, nch), dim3(64 * kSpreadWaves),
-                               0, s, G.witems, G.bgs, G.entries, (const float4*)G.ent_w, npy, vals,
-                               B, grids, gsz, g.Gy, partial, G.n_slots, G.npp, pstride);
-        else {
-            auto launch = [&](auto kern, int L_, int S_) {
-                hipLaunchKernelGGL(kern, dim3(G.n_sblocks, nch), dim3(64 * kSpreadWaves), 0, s,
-                                   G.witems, G.bgs, G.entries, (const float4*)G.ent_w, npy, vals,
-                                   B, grids, gsz, g.Gy, partial, G.n_slots, G.npp, pstride, L_, S_);
-            };
-            const bool st = S && pgk::g_spread_stage.load(std::memory_order_relaxed) != 0 &&
-                            spread_st_floats(B, L, AAi != nullptr) <= kStFloats &&
-                            (long long)G.M * S * 4 < (1LL << 31);
-            auto launch_st = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3(G.n_sblocks, nch), dim3(64 * kSpreadWaves), 0, s,
-                                   G.witems, G.bgs, G.entries, (const float4*)G.ent_w, npy, vals,
-                                   B, grids, gsz, g.Gy, partial, G.n_slots, G.npp, pstride, L, S);
-            };
-            const bool small = spread_st_floats(B, L, AAi != nullptr) <= 32;
-            if (st && AAi)
-                small ? launch_st(k_spread_patch_st<2, 32>) : launch_st(k_spread_patch_st<2, 48>);
-            else if (st)
-                small ? launch_st(k_spread_patch_st<1, 32>) : launch_st(k_spread_patch_st<1, 48>);
-            else if (S && AAi)
-                launch(k_spread_patch<2>, L, S);
-            else if (S)
-                launch(k_spread_patch<1>, L, S);
-            else
-                launch(k_spread_patch<0>, L, 0);
-        }
-        if (G.n_comb > 0)
-            hipLaunchKernelGGL(k_spread_heavy_combine, dim3(G.n_comb, nch, 16), dim3(64), 0, s, G.comb,
-                               npy, partial, G.n_slots, B, grids, gsz, g.Gy, G.npp, pstride);
+        const float* rows = reinterpret_cast<const float*>(vals);
+        if (S)
+            launch_spread2(G, rows, S, nc, L, AAi ? 2 : 1, grids, gsz, pstride, partial, s);
+        else
+            launch_spread2(G, rows, 2 * B, B, 1, 0, grids, gsz, pstride, partial, s);
         return;
     }
     if (NT == 12)
@@ -1850,7 +1501,6 @@ void spread_dispatch(const pg::Gnufft& G, const float2* in, long long in_cstride
 
 namespace pgk {
 
-std::atomic<int> g_spread_mfma{0};
 std::atomic<int> g_zclass{1};
 std::atomic<int> g_interp4{1};
 std::atomic<int> g_spread_rows{1};
@@ -1858,19 +1508,12 @@ std::atomic<int> g_zfuse{1};
 std::atomic<int> g_zmfma{1};
 std::atomic<int> g_zamfma{1};
 std::atomic<int> g_zfwd{1};
-std::atomic<int> g_spread_stage{1};
 
 int spread_row_floats(const pg::Gnufft& G, int nc, int L, const float* AA, const float* AAi)
 {
     const int B = nc * L;
     if (!g_spread_rows.load(std::memory_order_relaxed) || !AA || L < 2) return 0;
     if (G.geo.dims == 3 && !zclass_active(G, B)) return 0;
-    const pg::Gnufft::Tuned* tn = G.tuned_for(B);
-    // the matrix-core spread reads compact rows only in its staged form
-    if (B % 4 == 0 && (tn ? tn->mfma != 0 : g_spread_mfma.load(std::memory_order_relaxed) != 0) &&
-        !(g_spread_stage.load(std::memory_order_relaxed) &&
-          spread_st_floats(B, L, AAi != nullptr) <= kStFloats))
-        return 0;
     const int S = (2 * nc + (AAi ? 2 : 1) * L + 3) & ~3;
     // the rows live in the plan's value buffer (M x B float2) and a block of
     // 64 rows in LDS

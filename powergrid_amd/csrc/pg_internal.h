@@ -105,9 +105,6 @@ inline void grid_y_runs(long long n, F launch)
 // (defined in the .hip files; all asynchronous on `stream`)
 namespace pgk {
 
-// 2-D batched spread on the matrix cores (k_spread_patch_mfma) when set and
-// the grid count is a multiple of 4; the vector-unit kernel otherwise
-extern std::atomic<int> g_spread_mfma;
 // plans of 3-D trajectories with few distinct z windows are built for the
 // z-class planes (pg_gnufft.h) when set (the default); 0 builds them for the
 // full 3-D grid
@@ -137,10 +134,6 @@ extern std::atomic<int> g_zamfma;
 // the forward z stage of z-class planes on the matrix cores runs fused with
 // the planes' y FFT (Ny 64 or 128 at gridos 2) when set (default)
 extern std::atomic<int> g_zfwd;
-
-// the compact-row patch spread stages each stage's row slices in LDS
-// (k_spread_patch_st) when set (default), else reads them per entry
-extern std::atomic<int> g_spread_stage;
 
 // whether a batched launch of B grids of plan G runs on its z-class planes
 bool zclass_active(const pg::Gnufft& G, int B);

@@ -1,0 +1,49 @@
+"""GPU: the 2-D spread on the matrix cores against the FP64 restatement
+(oracle): every width of its coil chunks and remainder of its segment chunks,
+complex segment weights, value rows (no segments), patches of one to eight
+wavefronts and in parts, grids whose rows end in a partial strip, and grids
+large enough for the rows gathered in LDS.
+
+Tolerance 2e-6: FP32 sums of products of two taps and a weight (each rounded,
+eps = 6e-8) and a 2-D FFT, below 1e-6 in relative 2-norm."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-6
+
+
+def _complex(rng, *shape):
+    return (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64)
+
+
+@pytest.mark.parametrize("N,M,nc,L,interp,centre", [
+    (16, 300, 1, 1, 1, 0.0), (16, 300, 5, 3, 1, 0.0), (18, 300, 8, 4, 1, 0.3),
+    (16, 300, 9, 5, 1, 0.0), (22, 900, 16, 7, 1, 0.6), (16, 300, 17, 1, 1, 0.0),
+    (16, 300, 17, 3, 1, 0.0), (16, 300, 33, 2, 1, 0.0), (16, 300, 40, 1, 1, 0.0),
+    (16, 300, 3, 4, 2, 0.0), (16, 300, 11, 3, 2, 0.0), (16, 300, 19, 4, 3, 0.0),
+    (16, 9000, 4, 2, 1, 0.7), (66, 2000, 33, 16, 1, 0.2), (110, 1500, 7, 24, 1, 0.5)])
+def test_adjoint(orc, N, M, nc, L, interp, centre):
+    import powergrid_amd as P
+    rng = np.random.default_rng(M + nc + L)
+    kx, ky = rng.uniform(-N / 2, N / 2, M), rng.uniform(-N / 2, N / 2, M)
+    kx[:int(centre * M)] *= 0.08  # crowd the central patches
+    ky[:int(centre * M)] *= 0.08
+    kx, ky, kz = kx.astype(np.float32), ky.astype(np.float32), np.zeros(M, np.float32)
+    n = N * N
+    t = np.linspace(1e-3, 9e-3, M).astype(np.float32)
+    fm = rng.uniform(-700, 700, n).astype(np.float32)
+    sens, y = _complex(rng, nc, n), _complex(rng, nc * M)
+    A = P.SENSE(P.TimeSegmentation(P.Gnufft(M, 2.0, N, N, 1, kx, ky, kz), fm, t, M, n, L,
+                                   interptype=interp), sens, M, n, nc)
+    G = orc.Gnufft(M, 2.0, N, N, 1, kx, ky, kz, prec="d")
+    O = orc.SENSE(orc.TimeSegmentation(G, fm, t, M, n, L, interptype=interp),
+                  sens.astype(complex).ravel(), M, n, nc)
+    x = A / y
+    orc.set_threads(8)
+    try:
+        ref = O / y.astype(complex)
+    finally:
+        orc.set_threads(1)
+    assert np.linalg.norm(x - ref) / np.linalg.norm(ref) < TOL
+    assert np.array_equal(x, A / y)  # deterministic
