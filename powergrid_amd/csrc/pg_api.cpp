@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -187,17 +188,34 @@ void free_fft_plan(FftPlan1D& p)
     p.tw = nullptr;
 }
 
-// fn(begin, end) over [0, n) on up to 4 host threads (set-up loops whose
-// iterations are independent), at least `grain` iterations each
+// fn(begin, end) over [0, n) on up to 8 host threads (set-up loops whose
+// iterations are independent), at least `grain` iterations each; the threads'
+// ranges are in order.  An exception of any of them is thrown here, once all
+// have ended.
 template <class F>
 static void host_parallel(size_t n, size_t grain, F fn)
 {
-    const size_t hw = std::max(1u, std::min(4u, std::thread::hardware_concurrency()));
+    const size_t hw = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
     const size_t nth = std::max<size_t>(1, std::min(hw, n / std::max<size_t>(grain, 1)));
+    std::vector<std::exception_ptr> err(nth);
+    auto run = [&](size_t t) {
+        try {
+            fn(n * t / nth, n * (t + 1) / nth);
+        } catch (...) {
+            err[t] = std::current_exception();
+        }
+    };
     std::vector<std::thread> th;
-    for (size_t t = 1; t < nth; ++t) th.emplace_back(fn, n * t / nth, n * (t + 1) / nth);
-    fn(0, n / nth);
+    try {
+        for (size_t t = 1; t < nth; ++t) th.emplace_back(run, t);
+    } catch (...) {  // no more threads: the rest runs here
+    }
+    const size_t made = th.size();
+    run(0);
+    for (size_t t = made + 1; t < nth; ++t) run(t);
     for (std::thread& x : th) x.join();
+    for (const std::exception_ptr& e : err)
+        if (e) std::rethrow_exception(e);
 }
 
 template <class T>
@@ -625,7 +643,8 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
             std::vector<float> rw((size_t)2 * 8 * M, 0.0f);
             std::vector<int> tcnt(nbin + 1, 0), tof(M);
             const int Gd[2] = {g.Gx, g.Gy};
-            for (size_t i = 0; i < M; ++i) {
+            host_parallel(M, 8192, [&](size_t ib, size_t ie) {
+              for (size_t i = ib; i < ie; ++i) {
                 int tt[2];
                 for (int d = 0; d < 2; ++d) {
                     int l0 = lo[(size_t)d * M + i];
@@ -647,13 +666,13 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                     tt[d] = (l0 + padl) / kIT;
                 }
                 tof[i] = plane(i) * nt + tt[0] * G.ity + tt[1];
-                tcnt[tof[i] + 1]++;
-            }
+              }
+            });
+            for (size_t i = 0; i < M; ++i) tcnt[tof[i] + 1]++;
             for (long long t = 0; t < nbin; ++t) tcnt[t + 1] += tcnt[t];
             std::vector<int> pos(tcnt.begin(), tcnt.end() - 1), order(M);
             for (size_t i = 0; i < M; ++i) order[pos[tof[i]]++] = (int)i;
             std::vector<float4> rec((size_t)5 * M), rec4((size_t)5 * M);
-            std::vector<int4> its, its4;
             // LDS bank balance.  A wavefront of k_interp_lds reads, per tap,
             // one 8-byte point per (sample, segment) lane at index
             //   ((ox + x) LP + l) R + oy + y   (R = kIR, LP = 8 segment slots)
@@ -706,7 +725,14 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                 r[(size_t)5 * k + 3] = make_float4(wy[0], wy[1], wy[2], wy[3]);
                 r[(size_t)5 * k + 4] = make_float4(wy[4], wy[5], wy[6], wy[7]);
             };
-            for (long long tb = 0; tb < nbin; ++tb) {
+            // (bins are independent; the host threads' items are put together in
+            // bin order)
+            std::vector<std::vector<int4>> pits, pits4;
+            std::mutex pm;
+            std::vector<std::pair<size_t, size_t>> pruns;  // first bin, place in pits
+            host_parallel((size_t)nbin, M >= 4096 ? 16 : (size_t)nbin, [&](size_t bb, size_t be) {
+             std::vector<int4> its, its4;
+             for (long long tb = (long long)bb; tb < (long long)be; ++tb) {
                 const int p = (int)(tb / nt), t = (int)(tb - (long long)p * nt);
                 const int tx = t / G.ity, ty = t % G.ity;
                 const int rx0 = tx * kIT - padl, ry0 = ty * kIT - padl;
@@ -753,6 +779,17 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                     put(rec, k, i8, rlo[i8] - rx0, rlo[M + i8] - ry0);
                     put(rec4, k, i4, rlo[i4] - rx0, rlo[M + i4] - ry0);
                 }
+             }
+             std::lock_guard<std::mutex> lk(pm);
+             pruns.push_back({bb, pits.size()});
+             pits.push_back(std::move(its));
+             pits4.push_back(std::move(its4));
+            });
+            std::sort(pruns.begin(), pruns.end());
+            std::vector<int4> its, its4;
+            for (const auto& r : pruns) {
+                its.insert(its.end(), pits[r.second].begin(), pits[r.second].end());
+                its4.insert(its4.end(), pits4[r.second].begin(), pits4[r.second].end());
             }
             // items stay in (plane, tile raster) order: neighbouring tiles,
             // whose staged regions overlap, run at about the same time and
@@ -782,18 +819,22 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                 pos.assign(cnt.begin(), cnt.end() - 1);
                 ent.resize(std::max<long long>(1, cnt[npall]));
             }
-            for (size_t i = 0; i < M; ++i) {
-                if (empty(i)) continue;
-                const long long pb = (long long)plane(i) * np;
-                const int x0 = vlo[i] / kPatch, x1 = vhi[i] / kPatch;
-                const int y0 = vlo[M + i] / kPatch, y1 = vhi[M + i] / kPatch;
-                for (int a = x0; a <= x1; ++a)
-                    for (int c = y0; c <= y1; ++c) {
-                        const long long q = pb + (long long)a * npy + c;
-                        if (pass == 0) cnt[q + 1]++;
-                        else ent[pos[q]++] = (int)i;
-                    }
-            }
+            // each host thread counts and fills a run of patch rows (plane, x)
+            host_parallel((size_t)npl * npx, M >= 4096 ? 8 : (size_t)npl * npx, [&](size_t rb, size_t re) {
+                for (size_t i = 0; i < M; ++i) {
+                    const long long r0 = (long long)plane(i) * npx;
+                    const long long x0 = std::max<long long>(vlo[i] / kPatch, (long long)rb - r0);
+                    const long long x1 = std::min<long long>(vhi[i] / kPatch, (long long)re - 1 - r0);
+                    if (x1 < x0 || empty(i)) continue;
+                    const int y0 = vlo[M + i] / kPatch, y1 = vhi[M + i] / kPatch;
+                    for (long long a = x0; a <= x1; ++a)
+                        for (int c = y0; c <= y1; ++c) {
+                            const long long q = (r0 + a) * npy + c;
+                            if (pass == 0) cnt[q + 1]++;
+                            else ent[pos[q]++] = (int)i;
+                        }
+                }
+            });
             if (pass == 1) {
                 // weights of entry k (patch q, sample i) on the patch's 16 points,
                 // wx * wy formed in FP64 and rounded once
