@@ -328,7 +328,8 @@ int pg_recon_solve_batch(size_t K, const pg_op* A, const pg_penalty* R, const vo
  * has one form, on the matrix cores).
  * "autotune" 1: when an operator is first prepared for a batch of B grids,
  * its Gnufft plan times each variant of the 2-D (or z-class plane) batched
- * interpolation (gather, or LDS-staged tiles with sample bins of 128 or 64)
+ * interpolation (gather, LDS-staged tiles with sample bins of 128 or 64, or
+ * by patches on the matrix cores where that form serves the batch)
  * on its own workspaces and keeps the fastest for that B, overriding
  * "interp_lds4";
  * 0 (default): the fixed choice.  The variants differ in
@@ -344,6 +345,9 @@ int pg_recon_solve_batch(size_t K, const pg_op* A, const pg_penalty* R, const vo
  * segments at a time (256-thread blocks, items of <= 64 samples) when a
  * batch has 4 segments or more; 2: always; 0: never (all segments at once,
  * 512-thread blocks, items of <= 128 samples).  Same sums, FP32 order aside.
+ * With 1, batches of 8 coils, 6 segments and 64 grids or more on plans of 16
+ * samples a 4 x 4 patch are interpolated by patches on the matrix cores
+ * instead, where the partial sums fit the plan's workspace.
  * "batch_streams" n (0..8, default 4): streams of pg_recon_solve_batch.
  * "spread_rows" 1 (default): the 2-D (and z-class plane) spread of a
  * time-segmented batch forms each grid's value from a compact sample row
@@ -373,7 +377,8 @@ int pg_gnufft_zclasses(pg_op h, size_t* nzc);
 /* the variants the autotuner chose for the Gnufft plan under h (a Gnufft,
  * or a TimeSegmentation or SENSE over one) at B grids: interp_lds 1 =
  * LDS-staged tiles with every segment at once over bins of <= 128 samples,
- * 2 = four segments at a time over bins of <= 64 samples, 0 = gather;
+ * 2 = four segments at a time over bins of <= 64 samples, 0 = gather (the
+ * best of these, whether or not the patch form was faster still);
  * spread_mfma 1 = matrix cores (the one form); both -1 when the plan was not
  * tuned for B */
 int pg_op_tuning(pg_op h, int B, int* interp_lds, int* spread_mfma);

@@ -330,6 +330,8 @@ void Gnufft::release()
     dev_free(irec);
     dev_free(irec4);
     dev_free(ent_w);
+    dev_free(islots);
+    dev_free(soff);
     dev_free(items3);
     dev_free(entries3);
     dev_free(wpad3);
@@ -877,6 +879,15 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                 for (std::thread& x : th) x.join();
                 G.entries = dev_copy(ent.data(), ent.size());
                 G.ent_w = dev_copy(ew.data(), ew.size());
+                // the entries' places among their samples'
+                std::vector<int> soff(M + 1, 0), slots(std::max<long long>(1, cnt[npall]));
+                for (long long k = 0; k < cnt[npall]; ++k) ++soff[ent[k] + 1];
+                for (size_t i = 0; i < M; ++i) soff[i + 1] += soff[i];
+                std::vector<int> at(soff.begin(), soff.end() - 1);
+                for (long long k = 0; k < cnt[npall]; ++k) slots[k] = at[ent[k]]++;
+                G.islots = dev_copy(slots.data(), slots.size());
+                G.soff = dev_copy(soff.data(), soff.size());
+                G.n_entries = (size_t)cnt[npall];
             }
         }
         // Strips of four patches that follow each other along y: 128
@@ -1513,13 +1524,16 @@ static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi
         PG_HIP(hipEventElapsedTime(&ms, e[0], e[1]));
         return ms;
     };
-    G.tuned.push_back(Gnufft::Tuned{B, 1});
+    G.tuned.push_back(Gnufft::Tuned{B, 1, false});
     Gnufft::Tuned& t = G.tuned.back();
+    const bool mm = (G.geo.dims == 2 || planes) &&
+                    pgk::interp_mm_possible(G, nc, L, AA != nullptr, G.tbuf_floats());
     if (pgk::interp_lds_possible(G, L, AA != nullptr)) {
         // gather (0), all segments staged over bins of <= 128 samples (1),
         // four segments per stage over bins of <= 64 samples (2)
         auto interp = [&] {
-            pgk::launch_interp(G, G.grids, nc, L, AA, AAi, G.vals, G.M, ss, planes);
+            pgk::launch_interp(G, G.grids, nc, L, AA, AAi, G.vals, G.M, ss, planes,
+                               reinterpret_cast<float*>(G.tbuf), G.tbuf_floats());
         };
         float best = 0.f;
         int pick = 1;
@@ -1533,8 +1547,13 @@ static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi
             }
         }
         t.lds = pick;
+        if (mm) {
+            t.mm = true;
+            t.mm = timed(interp) < best;
+        }
     } else {
         t.lds = 0;
+        t.mm = mm;
     }
     PG_HIP(hipGetLastError());
     // the fills (and any timing launch) are done before the caller's stream
@@ -1578,8 +1597,9 @@ static void fused_forward(const Fused& f, const float2* x, float2* y, hipStream_
     }
     {
         Prof p("interp", s);
+        // (tbuf, the y FFT's output, is free once the x FFT has run)
         pgk::launch_interp(G, G.grids, f.nc, f.L, f.AA, f.AAi, y, y_cstride < 0 ? G.M : y_cstride,
-                           s, planes);
+                           s, planes, reinterpret_cast<float*>(G.tbuf), G.tbuf_floats());
     }
 }
 

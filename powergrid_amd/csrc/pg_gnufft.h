@@ -74,6 +74,12 @@ struct Gnufft {
     // entry's sample (ent_w[16k + 4a + q], point (a, q)), 0 outside its
     // clamped window
     float* ent_w = nullptr;
+    // the transposed use of the same entries (2-D interpolation by patches):
+    // entry k's share of its sample is partial sum islots[k], sample i's are
+    // soff[i] .. soff[i + 1], in patch order
+    int* islots = nullptr;
+    int* soff = nullptr;
+    size_t n_entries = 0;
     // 2-D interp through LDS: samples binned by the kIT x kIT tile of their
     // (re-based) window start; work items {tile, rec begin, rec end, 0} of at
     // most kIChunk samples; per binned sample a record of 5 float4:
@@ -132,9 +138,11 @@ struct Gnufft {
     // kernel variants chosen by the autotuner for a batch of B grids: the
     // interpolation as a gather (0), LDS-staged with all segments at once over
     // bins of <= kIChunk samples (1) or four segments at a time over bins of
-    // <= kIChunk4 samples (2); no entry: the default
+    // <= kIChunk4 samples (2); mm: by patches on the matrix cores instead, where
+    // that form serves the batch; no entry: the default
     struct Tuned {
         int B, lds;
+        bool mm;
     };
     std::vector<Tuned> tuned;
     const Tuned* tuned_for(int B) const
@@ -152,6 +160,11 @@ struct Gnufft {
     float2* img_tmp = nullptr;
     float2* dat_tmp = nullptr;
 
+    // floats of tbuf (cap_batch transforms of the y pass)
+    size_t tbuf_floats() const
+    {
+        return (size_t)2 * cap_batch * (geo.Nz > nzc ? geo.Nz : nzc) * geo.Nx * geo.Gy;
+    }
     void ensure_batch(int B);
     void release();
 };

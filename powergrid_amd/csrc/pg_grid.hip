@@ -1115,6 +1115,265 @@ void launch_spread2(const pg::Gnufft& G, const float* rows, int S, int nc, int L
                            s, G.comb, npy, partial, B, grids, gsz, g.Gy, G.npp, pstride);
 }
 
+// ------------------------------------------- 2-D interpolation by patches --
+// The transpose of k_spread2: the same work items (a patch, at most 64 of its
+// entries), for one chunk of 8 CT coils and all L segments:
+//   acc[64 entries][16 CT floats] += AA_l (W[entries][16 points] g_l[16 points][16 CT floats])
+// over the segments (the weights by FMA: a product's own sum is short, and a
+// segment's sum is rounded into acc once), v_mfma_f32_16x16x4f32 with the entries as rows: lane (i,
+// k) = (lane % 16, lane / 16) holds entry 16 g + i's weights of patch row k
+// (four floats of ew: a group's 1 KB in one load), B[k][j] the values of row
+// k of coil j's grid (32 contiguous bytes per lane and segment, the next
+// segment's in flight during this one's products).  So every grid point is
+// read once, by one block per strip of 128-byte rows; a patch's share of each
+// sample goes to part[slot of the entry][coil], the slots of a sample in
+// consecutive places, and k_interp_sum adds them in patch order (in FP64: an
+// add at the full sum's size for every patch would show in the result).
+// Why this form.  The tiled interpolation (k_interp_lds4) reads a tap of 8
+// bytes from LDS per FMA pair and is bound by that, by its bank conflicts and
+// by the 2.1-fold staged regions; here a value read from memory serves up to 64
+// samples, and 64 clocks of the matrix cores take the place of 128 FMAs and 64
+// LDS reads per (entry, 64 grids).  Measured: 384 grids on
+// 32 planes of 256^2, 524288 samples (32 coils, 12 segments): 3.21 ms -> 1.97 + 0.21
+// for the sums (6.4 GB of grids once, 3.3 TB/s; the shares' 0.7 GB at 3.2 TB/s);
+// 384 grids of 384^2, 65536 samples: 380 us -> 214 + 25; 64 grids of 256^2, 32768
+// samples (8 coils, 8 segments): 35.8 us -> 27.4 + 5.2.  Slower: 32 entries at a
+// time (two passes over the values, 2.37 ms), 16 or 8 coils a chunk (2.08, 2.62).
+// CT = 1 (up to 8 coils): column j holds the re (j < 8) or im of coil j % 8;
+// else tile 2 h holds the re and 2 h + 1 the im of coils 16 h + j.
+constexpr int kIpWaves = 4;   // a spread block's items run in blocks of 4 (a strip)
+static_assert(kSpreadWaves % kIpWaves == 0, "whole parts of a block");
+
+constexpr int NG = 4;  // 16-entry groups of an item
+
+template <int CT, bool CPLX>
+__global__ void __launch_bounds__(64 * kIpWaves) k_interp_mm(
+    const int4* __restrict__ witems, const int* __restrict__ entries, const float* __restrict__ ew,
+    const int* __restrict__ slots, int npy, const float2* __restrict__ grids, long long G, int Gy,
+    int nc, int L, const float* __restrict__ AA, const float* __restrict__ AAi, int M, int ncc,
+    float* __restrict__ part, int npp, long long pstride)
+{
+    constexpr int NH = CT == 1 ? 1 : CT / 2;  // coils per lane
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int pr = blockIdx.x >> 3, cc = pr % ncc;
+    constexpr int NP = kSpreadWaves / kIpWaves;
+    const int blk = pr / ncc / NP * 8 + (blockIdx.x & 7);
+    const int4 it = witems[blk * kSpreadWaves + pr / ncc % NP * kIpWaves + wv];
+    const int n = it.z - it.y;  // <= 64
+    if (it.x < 0 || n <= 0) return;
+    const int i = lane & 15, k = lane >> 4;
+    const int es = entries[it.y + min(lane, n - 1)], sl = slots[it.y + min(lane, n - 1)];
+    const int ng = (n + 15) >> 4;
+    float w[NG][4];
+#pragma unroll
+    for (int q = 0; q < NG; ++q) {
+        // (past the end: the last entry's, with zero weights)
+        const int e = 16 * q + i;
+        const float4 u = *reinterpret_cast<const float4*>(ew + 16LL * (it.y + min(e, n - 1)) + 4 * k);
+        w[q][0] = e < n ? u.x : 0.f;
+        w[q][1] = e < n ? u.y : 0.f;
+        w[q][2] = e < n ? u.z : 0.f;
+        w[q][3] = e < n ? u.w : 0.f;
+    }
+    const int pln = it.x / npp, q0 = it.x - pln * npp;
+    const int px0 = (q0 / npy) * pg::kPatch, py0 = (q0 % npy) * pg::kPatch;
+    const float2* gp = grids + pln * pstride + (long long)(px0 + k) * Gy + py0;
+    const float2* gc[NH];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+        const int c = cc * 8 * CT + (CT == 1 ? (i & 7) : 16 * h + i);
+        gc[h] = gp + (long long)min(c, nc - 1) * L * G;
+    }
+    float4 v[2][NH][2];
+    float a[2], ai[2];
+    auto load = [&](int l, int q) {
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const float4* p = reinterpret_cast<const float4*>(gc[h] + l * G);
+            v[q][h][0] = p[0];
+            v[q][h][1] = p[1];
+        }
+        a[q] = AA[(long long)l * M + es];
+        if (CPLX) ai[q] = AAi[(long long)l * M + es];
+    };
+    pg_f4 acc[NG][CT];
+#pragma unroll
+    for (int q = 0; q < NG; ++q)
+#pragma unroll
+        for (int t = 0; t < CT; ++t) acc[q][t] = pg_f4{0.f, 0.f, 0.f, 0.f};
+    auto sum = [&](int q) {
+        // b[t][s]: column i of tile t, point (row k, y = s)
+        float b[CT][4];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const float4 lo = v[q][h][0], hi = v[q][h][1];
+            if (CT == 1) {
+                const bool im = i >= 8;
+                b[0][0] = im ? lo.y : lo.x;
+                b[0][1] = im ? lo.w : lo.z;
+                b[0][2] = im ? hi.y : hi.x;
+                b[0][3] = im ? hi.w : hi.z;
+            } else {
+                b[(2 * h) % CT][0] = lo.x;
+                b[(2 * h) % CT][1] = lo.z;
+                b[(2 * h) % CT][2] = hi.x;
+                b[(2 * h) % CT][3] = hi.z;
+                b[(2 * h + 1) % CT][0] = lo.y;
+                b[(2 * h + 1) % CT][1] = lo.w;
+                b[(2 * h + 1) % CT][2] = hi.y;
+                b[(2 * h + 1) % CT][3] = hi.w;
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            if (g >= ng) break;
+            pg_f4 t4[CT];
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                t4[t] = pg_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    t4[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[g][s], b[t][s], t4[t], 0, 0, 0);
+            }
+            // times the segment's weight of entry 16 g + 4 k + r
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float ar = __shfl(a[q], 16 * g + 4 * k + r, 64);
+#pragma unroll
+                for (int t = 0; t < CT; ++t) acc[g][t][r] = __builtin_fmaf(ar, t4[t][r], acc[g][t][r]);
+                if constexpr (CPLX) {
+                    const float br = __shfl(ai[q], 16 * g + 4 * k + r, 64);
+                    if (CT == 1) {
+                        // (the other part is 8 columns away: row_ror 8)
+                        const float o = __int_as_float(__builtin_amdgcn_update_dpp(
+                            0, __float_as_int(t4[0][r]), 0x128, 0xF, 0xF, false));
+                        acc[g][0][r] = __builtin_fmaf(i >= 8 ? br : -br, o, acc[g][0][r]);
+                    } else {
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) {
+                            const int u = (2 * h) % CT, v1 = (2 * h + 1) % CT;
+                            acc[g][u][r] = __builtin_fmaf(-br, t4[v1][r], acc[g][u][r]);
+                            acc[g][v1][r] = __builtin_fmaf(br, t4[u][r], acc[g][v1][r]);
+                        }
+                    }
+                }
+            }
+        }
+    };
+    // the next segment's values in flight during this one's products (two
+    // or three segments ahead measured no faster)
+    load(0, 0);
+    for (int l = 0; l < L; l += 2) {
+        load(min(l + 1, L - 1), 1);
+        __builtin_amdgcn_sched_barrier(0);
+        sum(0);
+        if (l + 1 >= L) break;
+        load(min(l + 2, L - 1), 0);
+        __builtin_amdgcn_sched_barrier(0);
+        sum(1);
+    }
+    // lane: entries 16 g + 4 k + r, column i of every tile
+    float* pp = part + (long long)cc * 16 * CT;
+    const long long ps = 16LL * CT * ncc;  // floats per slot
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g >= ng) break;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = 16 * g + 4 * k + r;
+            const long long o = __shfl(sl, e, 64) * ps;
+            if (e >= n) continue;
+            if constexpr (CT == 1) {
+                pp[o + i] = acc[g][0][r];
+            } else {
+#pragma unroll
+                for (int h = 0; h < NH; ++h)
+                    *reinterpret_cast<float2*>(pp + o + 32 * h + 2 * i) =
+                        make_float2(acc[g][(2 * h) % CT][r], acc[g][(2 * h + 1) % CT][r]);
+            }
+        }
+    }
+}
+
+// the samples' sums over their slots soff[i] .. soff[i + 1], in slot order:
+// block of 32 samples, lanes over the coils (contiguous), the sums turned
+// through LDS into runs of samples.  PLANAR: a chunk's 8 re, then 8 im.
+// PLANAR: one chunk of 8 re, then 8 im; else a chunk's coils in pairs of floats.
+template <bool PLANAR>
+__global__ void __launch_bounds__(256) k_interp_sum(const int* __restrict__ soff,
+                                                    const float* __restrict__ part, int nc, int rf,
+                                                    int M, float2* __restrict__ out,
+                                                    long long out_cstride)
+{
+    // a sample's slots: rows of rf floats; NL lanes of float4 a row
+    constexpr int NL = PLANAR ? 4 : 8, NS = 256 / NL;
+    __shared__ float buf[4 * NL][NS + 1];
+    const int i0 = blockIdx.x * NS, c0 = blockIdx.y * 2 * NL;
+    const int s = threadIdx.x / NL, ln = threadIdx.x % NL;
+    if (i0 + s < M) {
+        const int b = soff[i0 + s], n = soff[i0 + s + 1] - b;
+        const float* p = part + (long long)b * rf + 2 * c0 + 4 * ln;
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+        // (a window meets at most 9 or 16 patches; six loads in flight)
+        for (int q = 0; q < n; q += 6) {
+            float4 v[6];
+#pragma unroll
+            for (int u = 0; u < 6; ++u)
+                v[u] = *reinterpret_cast<const float4*>(p + (long long)min(q + u, n - 1) * rf);
+#pragma unroll
+            for (int u = 0; u < 6; ++u)
+                if (q + u < n) {
+                    t[0] += v[u].x;
+                    t[1] += v[u].y;
+                    t[2] += v[u].z;
+                    t[3] += v[u].w;
+                }
+        }
+        buf[4 * ln + 0][s] = (float)t[0];
+        buf[4 * ln + 1][s] = (float)t[1];
+        buf[4 * ln + 2][s] = (float)t[2];
+        buf[4 * ln + 3][s] = (float)t[3];
+    }
+    __syncthreads();
+    const int so = threadIdx.x % NS;
+#pragma unroll
+    for (int co = threadIdx.x / NS; co < 2 * NL; co += NL)
+        if (i0 + so < M && c0 + co < nc)
+            out[(c0 + co) * out_cstride + i0 + so] =
+                PLANAR ? make_float2(buf[co][so], buf[(8 + co) % (4 * NL)][so])
+                       : make_float2(buf[2 * co][so], buf[2 * co + 1][so]);
+}
+
+// the coil columns of a chunk (the widest that the coils fill)
+int interp_mm_width(int nc) { return nc <= 8 ? 8 : nc <= 16 ? 16 : 32; }
+
+void launch_interp_mm(const pg::Gnufft& G, const float2* grids, long long gsz, long long pstride,
+                      int nc, int L, int w, const float* AA, const float* AAi, float* part,
+                      float2* out, long long out_cstride, hipStream_t s)
+{
+    const pg::Geometry& g = G.geo;
+    const int npy = g.Gy / pg::kPatch, ncc = (nc + w - 1) / w;
+    auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)(G.n_sblocks * ncc * (kSpreadWaves / kIpWaves))),
+                           dim3(64 * kIpWaves), 0, s, G.witems, G.entries, G.ent_w, G.islots, npy, grids, gsz, g.Gy, nc, L, AA,
+                           AAi, G.M, ncc, part, G.npp, pstride);
+    };
+    if (AAi)
+        w == 8    ? launch(k_interp_mm<1, true>)
+        : w == 16 ? launch(k_interp_mm<2, true>)
+                  : launch(k_interp_mm<4, true>);
+    else
+        w == 8    ? launch(k_interp_mm<1, false>)
+        : w == 16 ? launch(k_interp_mm<2, false>)
+                  : launch(k_interp_mm<4, false>);
+    if (w == 8)
+        hipLaunchKernelGGL(k_interp_sum<true>, dim3((G.M + 63) / 64), dim3(256), 0, s, G.soff, part,
+                           nc, 16, G.M, out, out_cstride);
+    else
+        hipLaunchKernelGGL(k_interp_sum<false>, dim3((G.M + 31) / 32, (nc + 15) / 16), dim3(256), 0,
+                           s, G.soff, part, nc, 2 * ncc * w, G.M, out, out_cstride);
+}
+
 // ------------------------------------------- 3-D patch spread ------------
 // The full 3-D grid (trajectories that are not stacks of 2-D ones), any
 // number of grids.  A wavefront runs the work item items3[] = {patch (-1:
@@ -1389,13 +1648,19 @@ __global__ void __launch_bounds__(256) k_spread_atomic(
 template <int NT, bool D3>
 void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, const float* AA,
                      const float* AAi, float2* out, long long out_cstride, hipStream_t s,
-                     bool planes)
+                     bool planes, float* part, size_t part_cap)
 {
     const pg::Geometry& g = G.geo;
     const pg::Gnufft::Tuned* tn = G.tuned_for(nc * L);
     // z-class planes: a 2-D interpolation on the plane of each sample's class
     const long long gsz = planes ? (long long)g.Gx * g.Gy : g.G();
     const long long pstride = planes ? (long long)nc * L * gsz : 0;
+    if ((!D3 || planes) && part && pgk::interp_mm_possible(G, nc, L, AA != nullptr, part_cap) &&
+        (tn ? tn->mm : pgk::g_interp4.load(std::memory_order_relaxed) == 1)) {
+        launch_interp_mm(G, grids, gsz, pstride, nc, L, interp_mm_width(nc), AA, AAi, part, out,
+                         out_cstride, s);
+        return;
+    }
     if ((!D3 || planes) && NT <= 8 && pgk::interp_lds_possible(G, L, AA != nullptr) &&
         (!tn || tn->lds)) {
         // four segments per stage when the autotuner chose it, or else from
@@ -1525,6 +1790,23 @@ bool zclass_active(const pg::Gnufft& G, int B)
     return G.nzc > 0 && B >= 16 && (long long)B * G.nzc < (1LL << 31);
 }
 
+// The patch interpolation takes batches whose columns and products are worth
+// its second pass over the partial sums (part_cap floats must hold them): 8
+// coils (fewer leave matrix columns idle), 6 segments (a partial sum is written
+// and read once for all of them) and 64 grids, and patches of 16 entries on the
+// average (one group of the products).  Tiled / by patches, whole forward
+// operator: 128^2, 16384 samples: 8 x 8 (coils x segments) 46.0 / 44.0 us, 12 x
+// 6 55.3 / 53.5, 6 x 6 38.7 / 39.4, 16 x 4 43.6 / 46.6; 256^2, 32768 samples (10
+// entries a patch): 8 x 8 106.7 / 110.9, 4 x 4 38.8 / 52.6; 64^2, 2048 samples (10
+// entries): 8 x 8 20.8 / 23.9.
+bool interp_mm_possible(const pg::Gnufft& G, int nc, int L, bool aa, size_t part_cap)
+{
+    if (!aa || !G.islots || nc < 8 || L < 6 || nc * L < 64) return false;
+    const size_t patches = (size_t)G.npp * (G.nzc > 0 ? G.nzc : 1);
+    const int w = interp_mm_width(nc);
+    return G.n_entries >= 16 * patches && G.n_entries * 2 * ((nc + w - 1) / w * w) <= part_cap;
+}
+
 bool interp_lds_possible(const pg::Gnufft& G, int L, bool aa)
 {
     const pg::Geometry& g = G.geo;
@@ -1533,22 +1815,23 @@ bool interp_lds_possible(const pg::Gnufft& G, int L, bool aa)
 }
 
 void launch_interp(const pg::Gnufft& G, const float2* grids, int nc, int L, const float* AA,
-                   const float* AAi, float2* out, long long out_cstride, hipStream_t s, bool planes)
+                   const float* AAi, float2* out, long long out_cstride, hipStream_t s, bool planes,
+                   float* part, size_t part_cap)
 {
     PG_REQUIRE(!planes || zclass_active(G, nc * L), PG_ERR_STATE, "no z-class planes for this batch");
     const bool d3 = G.geo.dims == 3;
     switch (G.geo.ntaps) {
     case 8:
-        d3 ? interp_dispatch<8, true>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes)
-           : interp_dispatch<8, false>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes);
+        d3 ? interp_dispatch<8, true>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes, part, part_cap)
+           : interp_dispatch<8, false>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes, part, part_cap);
         break;
     case 6:
-        d3 ? interp_dispatch<6, true>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes)
-           : interp_dispatch<6, false>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes);
+        d3 ? interp_dispatch<6, true>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes, part, part_cap)
+           : interp_dispatch<6, false>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes, part, part_cap);
         break;
     case 12:
-        d3 ? interp_dispatch<12, true>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes)
-           : interp_dispatch<12, false>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes);
+        d3 ? interp_dispatch<12, true>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes, part, part_cap)
+           : interp_dispatch<12, false>(G, grids, nc, L, AA, AAi, out, out_cstride, s, planes, part, part_cap);
         break;
     default:
         throw pg::Error{PG_ERR_UNSUPPORTED, "kernel width * gridos must give 6, 8 or 12 taps"};

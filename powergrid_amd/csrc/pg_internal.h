@@ -151,6 +151,10 @@ struct WeightArgs {
     const float* AA;
 };
 
+// whether interpolation by patches on the matrix cores (k_interp_mm) serves a
+// batch, given part_cap floats for its partial sums
+bool interp_mm_possible(const pg::Gnufft& G, int nc, int L, bool aa, size_t part_cap);
+
 // forward: image(s) -> batched grids  (deapod, pad, fftshift, FFT, ifftshift;
 // with `planes`, the z-class planes of the grids: the z taps applied in the
 // z pass)
@@ -158,10 +162,12 @@ void launch_fwd_prep_fft(const pg::Gnufft& G, const float2* img, long long img_c
                          WeightArgs w, int nc, int L, float2* tbuf, float2* tbuf2, float2* grids,
                          hipStream_t s, bool planes = false);
 // forward: batched grids (or z-class planes) -> samples (KB interpolation,
-// sum over segments)
+// sum over segments).  part: workspace of part_cap floats for the patch
+// interpolation, which serves time-segmented batches whose partial sums fit it
+// (none: the tiled forms)
 void launch_interp(const pg::Gnufft& G, const float2* grids, int nc, int L, const float* AA,
                    const float* AAi, float2* out, long long out_cstride, hipStream_t s,
-                   bool planes = false);
+                   bool planes = false, float* part = nullptr, size_t part_cap = 0);
 // adjoint: samples -> batched grids (KB spread, deterministic tiles)
 // (with resid_y set, the samples are W (resid_y - ax64), ax64 the FP64 Ax of
 // the CG, and `in` is unused; with vals_ready the per-sample values
