@@ -726,22 +726,29 @@ def kernel_times(P, Sg, x_host, stream, nrep, M, Gsz, B, nc, L, d, plane_g=None)
 
 
 def roofline(kinfo, L, summary, plane_bytes=None):
-    """the roofline object of the dominant gridding kernel.  The interpolation
-    stages all L segments of a tile (k_interp_lds) below 4 segments and four
-    at a time (k_interp_lds4) from 4 up; the spread of a time-segmented batch
-    of 32 coils is k_spread2<4, 2, 1>, that of 8 coils k_spread2<1, 8, 1> (or
-    <1, 4, 1>).  plane_bytes: on z-class planes the
+    """the roofline object of the dominant gridding pass.  At 32 coils and L
+    >= 6 the interpolation is k_interp_mm<4, false> and its sums, at 8 coils and
+    L = 8 k_interp_mm<1, false>; below, tiles of all L segments (k_interp_lds)
+    or of four at a time (k_interp_lds4, from 4 up); the spread of a
+    time-segmented batch is k_spread2<4, 2, 1> at 32 coils, k_spread2<1, 4, 1>
+    at 8.  plane_bytes: on z-class planes the
     launch moves 4*2*M + B*(8*M + 8*nzc*Gx*Gy) bytes (its x-y grids are the
     nzc planes, the z taps having been applied in the z stage), reported
     beside the full-grid figure of 4*d*M + B*(8*M + 8*G)."""
     dom = max(("interp", "spread"), key=lambda k: kinfo[k]["ms"])
-    kname = {"interp": "k_interp_lds4<false>" if L >= 4 else "k_interp_lds<8, false>",
-             "spread": "k_spread2<4, 2, 1>"}[dom]
-    tr = pmc_traffic(summary, kname)
-    for other in ("k_spread2<1, 8, 1>", "k_spread2<1, 4, 1>"):
-        if tr is None and dom == "spread":  # 8 coils
-            kname = other
-            tr = pmc_traffic(summary, kname)
+    forms = {"interp": [("k_interp_mm<4, false>", "k_interp_sum<false>"),
+                        ("k_interp_mm<1, false>", "k_interp_sum<true>")],
+             "spread": [("k_spread2<4, 2, 1>", "k_spread_heavy_combine"),
+                        ("k_spread2<1, 4, 1>", "k_spread_heavy_combine")]}[dom]
+    if dom == "interp" and L < 6:
+        forms = [("k_interp_lds4<false>" if L >= 4 else "k_interp_lds<8, false>",)]
+    # the form that the summary holds (main kernel and second pass)
+    kname, tr = forms[0][0], None
+    for names in forms:
+        rows = [pmc_traffic(summary, k) for k in names]
+        if rows[0] is not None:
+            kname, tr = names[0], sum(r or 0.0 for r in rows)
+            break
     out = dict(bound="hbm", achieved=round(kinfo[dom]["GBs"], 1), peak=HBM_PEAK_GBS,
                unit="GB/s", frac=round(kinfo[dom]["frac"], 4),
                traffic=None if tr is None else round(tr), kernel=kname,

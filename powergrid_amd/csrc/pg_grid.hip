@@ -1135,7 +1135,8 @@ void launch_spread2(const pg::Gnufft& G, const float* rows, int S, int nc, int L
 // samples, and 64 clocks of the matrix cores take the place of 128 FMAs and 64
 // LDS reads per (entry, 64 grids).  Measured: 384 grids on
 // 32 planes of 256^2, 524288 samples (32 coils, 12 segments): 3.21 ms -> 1.97 + 0.21
-// for the sums (6.4 GB of grids once, 3.3 TB/s; the shares' 0.7 GB at 3.2 TB/s);
+// for the sums (6.4 GB of grids read, 1.0 of shares written, 3.8 TB/s; 1.15 GB
+// in the second pass, 5.4 TB/s);
 // 384 grids of 384^2, 65536 samples: 380 us -> 214 + 25; 64 grids of 256^2, 32768
 // samples (8 coils, 8 segments): 35.8 us -> 27.4 + 5.2.  Slower: 32 entries at a
 // time (two passes over the values, 2.37 ms), 16 or 8 coils a chunk (2.08, 2.62).
