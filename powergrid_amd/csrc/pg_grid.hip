@@ -1120,32 +1120,30 @@ void launch_spread2(const pg::Gnufft& G, const float* rows, int S, int nc, int L
 // entries), for one chunk of 8 CT coils and all L segments:
 //   acc[64 entries][16 CT floats] += AA_l (W[entries][16 points] g_l[16 points][16 CT floats])
 // over the segments (the weights by FMA: a product's own sum is short, and a
-// segment's sum is rounded into acc once), v_mfma_f32_16x16x4f32 with the entries as rows: lane (i,
-// k) = (lane % 16, lane / 16) holds entry 16 g + i's weights of patch row k
-// (four floats of ew: a group's 1 KB in one load), B[k][j] the values of row
-// k of coil j's grid (32 contiguous bytes per lane and segment, the next
-// segment's in flight during this one's products).  So every grid point is
-// read once, by one block per strip of 128-byte rows; a patch's share of each
-// sample goes to part[slot of the entry][coil], the slots of a sample in
-// consecutive places, and k_interp_sum adds them in patch order (in FP64: an
-// add at the full sum's size for every patch would show in the result).
+// segment's sum is rounded into acc once), v_mfma_f32_16x16x4f32 with the
+// entries as rows: lane (i, k) = (lane % 16, lane / 16) holds entry 16 g + i's
+// weights of patch row k (four floats of ew: a group's 1 KB in one load),
+// B[k][j] the values of row k of coil j's grid (32 contiguous bytes per lane and
+// segment, the next segment's in flight during this one's products).  So every
+// grid point is read once, by one block per strip of 128-byte rows; a patch's
+// share of each sample goes to part[slot of the entry][coil], the slots of a
+// sample in consecutive places, and k_interp_sum adds them in patch order (in
+// FP64: an add at the full sum's size for every patch would show in the result).
 // Why this form.  The tiled interpolation (k_interp_lds4) reads a tap of 8
 // bytes from LDS per FMA pair and is bound by that, by its bank conflicts and
 // by the 2.1-fold staged regions; here a value read from memory serves up to 64
 // samples, and 64 clocks of the matrix cores take the place of 128 FMAs and 64
-// LDS reads per (entry, 64 grids).  Measured: 384 grids on
-// 32 planes of 256^2, 524288 samples (32 coils, 12 segments): 3.21 ms -> 1.97 + 0.21
-// for the sums (6.4 GB of grids read, 1.0 of shares written, 3.8 TB/s; 1.15 GB
-// in the second pass, 5.4 TB/s);
-// 384 grids of 384^2, 65536 samples: 380 us -> 214 + 25; 64 grids of 256^2, 32768
-// samples (8 coils, 8 segments): 35.8 us -> 27.4 + 5.2.  Slower: 32 entries at a
-// time (two passes over the values, 2.37 ms), 16 or 8 coils a chunk (2.08, 2.62).
+// LDS reads per (entry, 64 grids).  Bound by memory requests.  Measured: 384
+// grids on 32 planes of 256^2, 524288 samples (32 coils, 12 segments): 3.21 ms ->
+// 1.97 + 0.21 for the sums (6.4 GB of grids read and 1.0 of shares written, 3.8
+// TB/s; 1.15 GB in the second pass, 5.4 TB/s); 384 grids of 384^2, 65536 samples:
+// 380 us -> 214 + 25; 64 grids of 256^2, 32768 samples (8 coils, 8 segments): 35.8
+// us -> 27.4 + 5.2.  Slower at the first of these: 32 entries at a time (two
+// passes over the values, 2.37 ms), 16 or 8 coils a chunk (2.08, 2.62).
 // CT = 1 (up to 8 coils): column j holds the re (j < 8) or im of coil j % 8;
 // else tile 2 h holds the re and 2 h + 1 the im of coils 16 h + j.
-constexpr int kIpWaves = 4;   // a spread block's items run in blocks of 4 (a strip)
+constexpr int kIpWaves = 4;  // a spread block's items run in blocks of 4 (a strip)
 static_assert(kSpreadWaves % kIpWaves == 0, "whole parts of a block");
-
-constexpr int NG = 4;  // 16-entry groups of an item
 
 template <int CT, bool CPLX>
 __global__ void __launch_bounds__(64 * kIpWaves) k_interp_mm(
@@ -1155,6 +1153,7 @@ __global__ void __launch_bounds__(64 * kIpWaves) k_interp_mm(
     float* __restrict__ part, int npp, long long pstride)
 {
     constexpr int NH = CT == 1 ? 1 : CT / 2;  // coils per lane
+    constexpr int NG = 4;                     // 16-entry groups of an item
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int pr = blockIdx.x >> 3, cc = pr % ncc;
     constexpr int NP = kSpreadWaves / kIpWaves;

@@ -112,7 +112,8 @@ extern std::atomic<int> g_zclass;
 // the LDS-staged interpolation stages four segments at a time in 256-thread
 // blocks over items of <= 64 samples (k_interp_lds4): 2 always, 1 (the
 // default) from 4 segments up, 0 never (all segments at once in
-// 512-thread blocks over items of <= 128 samples)
+// 512-thread blocks over items of <= 128 samples).  With 1, batches that
+// interp_mm_possible() accepts are interpolated by patches instead
 extern std::atomic<int> g_interp4;
 
 // the 2-D (and z-class plane) spread of a time-segmented batch forms each
