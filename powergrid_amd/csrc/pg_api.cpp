@@ -1527,13 +1527,13 @@ static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi
     G.tuned.push_back(Gnufft::Tuned{B, 1, false});
     Gnufft::Tuned& t = G.tuned.back();
     const bool mm = (G.geo.dims == 2 || planes) &&
-                    pgk::interp_mm_possible(G, nc, L, AA != nullptr, G.tbuf_floats());
+                    pgk::interp_mm_possible(G, nc, L, AA != nullptr, G.tbuf_floats(B));
     if (pgk::interp_lds_possible(G, L, AA != nullptr)) {
         // gather (0), all segments staged over bins of <= 128 samples (1),
         // four segments per stage over bins of <= 64 samples (2)
         auto interp = [&] {
             pgk::launch_interp(G, G.grids, nc, L, AA, AAi, G.vals, G.M, ss, planes,
-                               reinterpret_cast<float*>(G.tbuf), G.tbuf_floats());
+                               reinterpret_cast<float*>(G.tbuf), G.tbuf_floats(B));
         };
         float best = 0.f;
         int pick = 1;
@@ -1599,7 +1599,8 @@ static void fused_forward(const Fused& f, const float2* x, float2* y, hipStream_
         Prof p("interp", s);
         // (tbuf, the y FFT's output, is free once the x FFT has run)
         pgk::launch_interp(G, G.grids, f.nc, f.L, f.AA, f.AAi, y, y_cstride < 0 ? G.M : y_cstride,
-                           s, planes, reinterpret_cast<float*>(G.tbuf), G.tbuf_floats());
+                           s, planes, reinterpret_cast<float*>(G.tbuf),
+                           G.tbuf_floats(f.nc * f.L));
     }
 }
 

@@ -160,10 +160,12 @@ struct Gnufft {
     float2* img_tmp = nullptr;
     float2* dat_tmp = nullptr;
 
-    // floats of tbuf (cap_batch transforms of the y pass)
-    size_t tbuf_floats() const
+    // floats that a batch of B grids has in tbuf (its transforms of the y pass;
+    // what a larger batch made of tbuf does not count, so that a kernel chosen
+    // by this does not depend on the plan's earlier calls)
+    size_t tbuf_floats(int B) const
     {
-        return (size_t)2 * cap_batch * (geo.Nz > nzc ? geo.Nz : nzc) * geo.Nx * geo.Gy;
+        return (size_t)2 * B * (geo.Nz > nzc ? geo.Nz : nzc) * geo.Nx * geo.Gy;
     }
     void ensure_batch(int B);
     void release();

@@ -62,3 +62,22 @@ def test_forward(orc, N, Nz, M, nc, L, interp, centre, patches):
     finally:
         P.set_tuning("interp_lds4", 1)
     assert np.array_equal(y, tiled) != patches
+
+
+def test_form_independent_of_earlier_calls():
+    """a batch whose partial sums do not fit its own share of the plan's
+    workspace keeps its form, and so its bits, when a larger batch on the same
+    plan has grown that workspace"""
+    import powergrid_amd as P
+    rng = np.random.default_rng(5)
+    N, M, nc, L = 32, 1500, 12, 6
+    n = N * N
+    kx, ky = (rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(2))
+    t = np.linspace(1e-3, 9e-3, M).astype(np.float32)
+    fm = rng.uniform(-700, 700, n).astype(np.float32)
+    x, sens = _complex(rng, n), _complex(rng, 32, n)
+    G = P.Gnufft(M, 2.0, N, N, 1, kx, ky, np.zeros(M, np.float32))
+    A = P.SENSE(P.TimeSegmentation(G, fm, t, M, n, L), sens[:nc], M, n, nc)
+    fresh = A * x
+    P.SENSE(P.TimeSegmentation(G, fm, t, M, n, 8), sens, M, n, 32) * x
+    assert np.array_equal(A * x, fresh)
