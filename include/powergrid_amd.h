@@ -326,11 +326,11 @@ int pg_recon_solve_batch(size_t K, const pg_op* A, const pg_penalty* R, const vo
 /* ---- tuning (no counterpart in the reference) ----------------------------
  * "spread_mfma", "spread_stage": accepted and without effect (the 2-D spread
  * has one form, on the matrix cores).
- * "autotune" 1: when an operator is first prepared for a batch of B grids,
- * its Gnufft plan times each variant of the 2-D (or z-class plane) batched
+ * "autotune" 1: when an operator is first prepared for a batch of B grids
+ * (coils x segments), its Gnufft plan times each variant of the 2-D (or z-class plane) batched
  * interpolation (gather, LDS-staged tiles with sample bins of 128 or 64, or
  * by patches on the matrix cores where that form serves the batch)
- * on its own workspaces and keeps the fastest for that B, overriding
+ * on its own workspaces and keeps the fastest for that batch, overriding
  * "interp_lds4";
  * 0 (default): the fixed choice.  The variants differ in
  * FP32 summation order only, but with autotuning on, which one runs -- and
@@ -380,7 +380,8 @@ int pg_gnufft_zclasses(pg_op h, size_t* nzc);
  * 2 = four segments at a time over bins of <= 64 samples, 0 = gather (the
  * best of these, whether or not the patch form was faster still);
  * spread_mfma 1 = matrix cores (the one form); both -1 when the plan was not
- * tuned for B */
+ * tuned for B.  A plan is tuned for each number of coils and segments and kind
+ * of weights by itself; of several with B grids the last one is reported */
 int pg_op_tuning(pg_op h, int B, int* interp_lds, int* spread_mfma);
 
 /* ---- measurement --------------------------------------------------------

@@ -1484,13 +1484,15 @@ static std::atomic<int> g_autotune{0};
 
 // Times each variant of plan G's batched interpolation (LDS-staged or
 // gather) for nc x L grids, on the plan's own workspaces (their contents do
-// not matter for timing), and keeps the fastest.  Set-up work on the thread's set-up stream, before any
-// capture; a plan is tuned once per grid count.
+// not matter for timing), and keeps the fastest.  Set-up work on the thread's
+// set-up stream, before any capture; a plan is tuned once per nc, L and kind
+// of weights.
 static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi)
 {
     const int B = nc * L;
     const bool planes = pgk::zclass_active(G, B);
-    if ((G.geo.dims != 2 && !planes) || !G.fft_ok || G.tuned_for(B)) return;
+    if ((G.geo.dims != 2 && !planes) || !G.fft_ok || G.tuned_for(nc, L, AAi != nullptr))
+        return;
     G.ensure_batch(B);
     const hipStream_t ss = setup_stream();
     hipEvent_t e[2] = {nullptr, nullptr};
@@ -1524,7 +1526,7 @@ static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi
         PG_HIP(hipEventElapsedTime(&ms, e[0], e[1]));
         return ms;
     };
-    G.tuned.push_back(Gnufft::Tuned{B, 1, false});
+    G.tuned.push_back(Gnufft::Tuned{nc, L, AAi != nullptr, 1, false});
     Gnufft::Tuned& t = G.tuned.back();
     const bool mm = (G.geo.dims == 2 || planes) &&
                     pgk::interp_mm_possible(G, nc, L, AA != nullptr, G.tbuf_floats(B));
@@ -1564,11 +1566,11 @@ static void autotune(Gnufft& G, int nc, int L, const float* AA, const float* AAi
 }
 
 // autotune the plan of a fused launch on stream s, unless already tuned for
-// its grid count or s is capturing; s is drained first, since the timing
+// its batch or s is capturing; s is drained first, since the timing
 // runs overwrite the plan's workspaces
 static void maybe_autotune(const Fused& f, hipStream_t s)
 {
-    if (!g_autotune.load() || f.G->tuned_for(f.nc * f.L)) return;
+    if (!g_autotune.load() || f.G->tuned_for(f.nc, f.L, f.AAi != nullptr)) return;
     if (s) {
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         PG_HIP(hipStreamIsCapturing(s, &st));
@@ -3629,7 +3631,7 @@ int pg_op_tuning(pg_op h, int B, int* interp_lds, int* spread_mfma)
     if (op->kind == K_SENSE) op = static_cast<SenseOp*>(op)->inner;
     if (op->kind == K_TS) op = static_cast<TsOp*>(op)->inner;
     PG_REQUIRE(op->kind == K_NUFFT, PG_ERR_ARG, "not a Gnufft or an operator over one");
-    const Gnufft::Tuned* t = static_cast<NufftOp*>(op)->G.tuned_for(B);
+    const Gnufft::Tuned* t = static_cast<NufftOp*>(op)->G.tuned_last(B);
     *interp_lds = t ? t->lds : -1;
     *spread_mfma = t ? 1 : -1;  // the one form of the spread
     PG_CATCH

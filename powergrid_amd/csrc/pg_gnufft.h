@@ -135,20 +135,31 @@ struct Gnufft {
     int4* iitems3 = nullptr;
     int n_iitems3 = 0;
     int4* irec3 = nullptr;
-    // kernel variants chosen by the autotuner for a batch of B grids: the
-    // interpolation as a gather (0), LDS-staged with all segments at once over
+    // kernel variants chosen by the autotuner for a batch of nc coils x L
+    // segments, cplx: complex segment weights (which variants serve a batch
+    // and how fast they are depends on all three): the interpolation as a
+    // gather (0), LDS-staged with all segments at once over
     // bins of <= kIChunk samples (1) or four segments at a time over bins of
     // <= kIChunk4 samples (2); mm: by patches on the matrix cores instead, where
     // that form serves the batch; no entry: the default
     struct Tuned {
-        int B, lds;
+        int nc, L;
+        bool cplx;
+        int lds;
         bool mm;
     };
     std::vector<Tuned> tuned;
-    const Tuned* tuned_for(int B) const
+    const Tuned* tuned_for(int nc, int L, bool cplx) const
     {
         for (const Tuned& t : tuned)
-            if (t.B == B) return &t;
+            if (t.nc == nc && t.L == L && t.cplx == cplx) return &t;
+        return nullptr;
+    }
+    // the last batch of B grids that was tuned
+    const Tuned* tuned_last(int B) const
+    {
+        for (size_t k = tuned.size(); k-- > 0;)
+            if (tuned[k].nc * tuned[k].L == B) return &tuned[k];
         return nullptr;
     }
     // workspace for batched transforms (grown on demand)

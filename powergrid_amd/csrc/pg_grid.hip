@@ -1651,7 +1651,7 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
                      bool planes, float* part, size_t part_cap)
 {
     const pg::Geometry& g = G.geo;
-    const pg::Gnufft::Tuned* tn = G.tuned_for(nc * L);
+    const pg::Gnufft::Tuned* tn = G.tuned_for(nc, L, AAi != nullptr);
     // z-class planes: a 2-D interpolation on the plane of each sample's class
     const long long gsz = planes ? (long long)g.Gx * g.Gy : g.G();
     const long long pstride = planes ? (long long)nc * L * gsz : 0;

@@ -146,3 +146,27 @@ def test_cached_solve_follows_mode_and_tuning_changes():
     assert rel(xi, xb) < 1e-5
     xb3, _ = P.reconSolve(y, ops_b[2], R, niter=5)
     assert np.array_equal(xb3, xb)
+
+
+def test_tuned_by_coils_and_segments():
+    # a plan tuned at 2 coils x 32 segments (more than 16 segments have the
+    # gather alone) tunes 8 x 8, the same number of grids, by itself, and finds
+    # a staged form faster
+    print("[autotune per batch]", flush=True)
+    N = 128
+    _, G, A = ops(N, 16, 2048, 2, 32)
+    kx, ky, kz = S.spiral(N, 16, 2048)
+    M = len(kx)
+    t = S.readout_times(16, 2048, dwell=5e-6, te=5e-4)
+    fm = S.field_map(N, peak_hz=120.0).astype(np.float32)
+    sens = S.coil_maps(N, 8).astype(np.complex64)
+    x = S.ellipse_phantom(N, seed=3).astype(np.complex64)
+    P.set_tuning("autotune", 1)
+    try:
+        A * x
+        assert P.op_tuning(A, 64)[0] == 0
+        B = P.SENSE(P.TimeSegmentation(G, fm, t, M, N * N, 8), sens, M, N * N, 8)
+        B * x
+        assert P.op_tuning(B, 64)[0] in (1, 2)
+    finally:
+        P.set_tuning("autotune", 0)
