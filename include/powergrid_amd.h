@@ -346,8 +346,9 @@ int pg_recon_solve_batch(size_t K, const pg_op* A, const pg_penalty* R, const vo
  * batch has 4 segments or more; 2: always; 0: never (all segments at once,
  * 512-thread blocks, items of <= 128 samples).  Same sums, FP32 order aside.
  * With 1, batches of 8 coils, 6 segments and 64 grids or more on plans of 16
- * samples a 4 x 4 patch are interpolated by patches on the matrix cores
- * instead, where the partial sums fit the plan's workspace.
+ * (sample, 4 x 4 patch) pairs a patch are interpolated by patches on the matrix
+ * cores instead, where the partial sums fit the batch's workspace and the size
+ * makes that the faster form; 3: wherever they fit, whatever the size.
  * "batch_streams" n (0..8, default 4): streams of pg_recon_solve_batch.
  * "spread_rows" 1 (default): the 2-D (and z-class plane) spread of a
  * time-segmented batch forms each grid's value from a compact sample row

@@ -3671,7 +3671,7 @@ int pg_set_tuning(const char* key, int value)
     else if (k == "batch_streams")
         g_batch_streams.store(value < 0 ? 0 : (value > 8 ? 8 : value));
     else if (k == "interp_lds4")
-        pgk::g_interp4.store(value < 0 ? 0 : (value > 2 ? 2 : value));
+        pgk::g_interp4.store(value < 0 ? 0 : (value > 3 ? 3 : value));
     else if (k == "autotune")
         g_autotune.store(value ? 1 : 0);
     else

@@ -25,6 +25,8 @@
 //            grids of a plan of z-class planes, one thread per sample with
 //            hardware float atomics into a zeroed grid (the reference's
 //            OpenACC spread, gridding.cpp:102-106).
+#include <cmath>
+
 #include "pg_gnufft.h"
 #include "pg_internal.h"
 #include "pg_fftreg.h"
@@ -1655,8 +1657,9 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
     // z-class planes: a 2-D interpolation on the plane of each sample's class
     const long long gsz = planes ? (long long)g.Gx * g.Gy : g.G();
     const long long pstride = planes ? (long long)nc * L * gsz : 0;
+    const int v4 = pgk::g_interp4.load(std::memory_order_relaxed);
     if ((!D3 || planes) && part && pgk::interp_mm_possible(G, nc, L, AA != nullptr, part_cap) &&
-        (tn ? tn->mm : pgk::g_interp4.load(std::memory_order_relaxed) == 1)) {
+        (tn ? tn->mm : v4 == 3 || (v4 == 1 && pgk::interp_mm_pays(G, nc, L, AAi != nullptr)))) {
         launch_interp_mm(G, grids, gsz, pstride, nc, L, interp_mm_width(nc), AA, AAi, part, out,
                          out_cstride, s);
         return;
@@ -1666,8 +1669,7 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
         // four segments per stage when the autotuner chose it, or else from
         // four segments up (measured faster there: the smaller blocks and
         // LDS footprint keep more of them per CU)
-        const int v4 = pgk::g_interp4.load(std::memory_order_relaxed);
-        const bool four = tn ? tn->lds == 2 : (v4 == 2 || (v4 == 1 && L >= 4));
+        const bool four = tn ? tn->lds == 2 : (v4 == 2 || (v4 != 0 && L >= 4));
         // (its staging and weight offsets are 32-bit byte offsets)
         if (G.n_iitems4 > 0 && four && gsz * 4 * 8 < (1LL << 31) &&
             (long long)L * G.M * 4 < (1LL << 31)) {
@@ -1790,21 +1792,40 @@ bool zclass_active(const pg::Gnufft& G, int B)
     return G.nzc > 0 && B >= 16 && (long long)B * G.nzc < (1LL << 31);
 }
 
-// The patch interpolation takes batches whose columns and products are worth
-// its second pass over the partial sums (part_cap floats must hold them): 8
-// coils (fewer leave matrix columns idle), 6 segments (a partial sum is written
-// and read once for all of them) and 64 grids, and patches of 16 entries on the
-// average (one group of the products).  Tiled / by patches, whole forward
-// operator: 128^2, 16384 samples: 8 x 8 (coils x segments) 46.0 / 44.0 us, 12 x
-// 6 55.3 / 53.5, 6 x 6 38.7 / 39.4, 16 x 4 43.6 / 46.6; 256^2, 32768 samples (10
-// entries a patch): 8 x 8 106.7 / 110.9, 4 x 4 38.8 / 52.6; 64^2, 2048 samples (10
-// entries): 8 x 8 20.8 / 23.9.
+// The batches that the patch interpolation can take: 8 coils (fewer leave
+// matrix columns idle), 6 segments (a partial sum is written and read once for
+// all of them) and 64 grids, patches of 16 entries on the average (one group
+// of the products), and partial sums that fit part_cap floats.
 bool interp_mm_possible(const pg::Gnufft& G, int nc, int L, bool aa, size_t part_cap)
 {
     if (!aa || !G.islots || nc < 8 || L < 6 || nc * L < 64) return false;
     const size_t patches = (size_t)G.npp * (G.nzc > 0 ? G.nzc : 1);
     const int w = interp_mm_width(nc);
     return G.n_entries >= 16 * patches && G.n_entries * 2 * ((nc + w - 1) / w * w) <= part_cap;
+}
+
+// Which of them it is the faster form for.  Against it are a wavefront's
+// serial chain over the segments (some 1 us each while the patches' wavefronts
+// do not fill the SIMDs), columns without a coil, the launch of the second pass
+// and, for up to 8 coils, whose products are short, the shuffles of the weights
+// (complex ones above all); the tiled form pays for segments in fours (L4).  So
+// patches x sqrt(entries a patch) x (filled share of the columns)^2 x L4^2 / L
+// has to exceed a bound.  5687 random batches (48^2 .. 256^2 and stacks of 32^2
+// .. 64^2, 8 .. 32 coils, 6 .. 12 segments, whole forward operator): patches in
+// 0.63 to 1.43 times the tiles' time, over 1.05 in 1371.  Of the 3720 that pass
+// the bound 34 are slower by over 5%; 59 of the others would gain as much.  128^2, 32768 samples, 8 coils x 8 segments: 56.8 (tiles) / 56.6
+// us, 32 x 12: 265 / 210; 64^2, 4096 samples, 17 x 8: 34.0 / 47.8.  Batches that
+// have no tiles (12 taps, over 16 segments) would go to the gather kernel.
+bool interp_mm_pays(const pg::Gnufft& G, int nc, int L, bool cplx)
+{
+    if (!interp_lds_possible(G, L, true)) return true;
+    const int w = interp_mm_width(nc), l4 = (L + 3) & ~3;
+    const double patches = (double)G.npp * (G.nzc > 0 ? G.nzc : 1);
+    const double fill = (double)nc / ((nc + w - 1) / w * w);
+    double bound = 8e4;
+    if (w == 8) bound *= 1.5;
+    if (cplx) bound *= w == 8 ? 2.0 : 1.125;
+    return std::sqrt(patches * G.n_entries) * fill * fill * l4 * l4 >= bound * L;
 }
 
 bool interp_lds_possible(const pg::Gnufft& G, int L, bool aa)

@@ -113,7 +113,8 @@ extern std::atomic<int> g_zclass;
 // blocks over items of <= 64 samples (k_interp_lds4): 2 always, 1 (the
 // default) from 4 segments up, 0 never (all segments at once in
 // 512-thread blocks over items of <= 128 samples).  With 1, batches that
-// interp_mm_possible() accepts are interpolated by patches instead
+// interp_mm_possible() and interp_mm_pays() accept are interpolated by patches
+// instead, with 3 all that interp_mm_possible() accepts (the rest as with 1)
 extern std::atomic<int> g_interp4;
 
 // the 2-D (and z-class plane) spread of a time-segmented batch forms each
@@ -155,6 +156,8 @@ struct WeightArgs {
 // whether interpolation by patches on the matrix cores (k_interp_mm) serves a
 // batch, given part_cap floats for its partial sums
 bool interp_mm_possible(const pg::Gnufft& G, int nc, int L, bool aa, size_t part_cap);
+// and whether it is the faster form for one that it serves
+bool interp_mm_pays(const pg::Gnufft& G, int nc, int L, bool cplx);
 
 // forward: image(s) -> batched grids  (deapod, pad, fftshift, FFT, ifftshift;
 // with `planes`, the z-class planes of the grids: the z taps applied in the

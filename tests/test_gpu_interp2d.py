@@ -2,7 +2,9 @@
 restatement (oracle): each width of its coil chunks with partial last ones,
 odd and even segment counts, complex segment weights, patches of one to
 several wavefronts, samples at the grid's edges, class planes, and the calls
-around its rule (fewer coils, segments or samples: the tiled form).
+that it does not serve (fewer coils, segments or samples: the tiled form).  It
+is asked for wherever it can serve (interp_lds4 3): at these sizes the tiles
+are the faster form, as the last test shows.
 
 Tolerance 2e-6: FP32 sums of products of two taps, a grid value and a weight
 (each rounded, eps = 6e-8) after a 2-D FFT, below 1e-6 in relative 2-norm."""
@@ -47,14 +49,18 @@ def test_forward(orc, N, Nz, M, nc, L, interp, centre, patches):
     G = orc.Gnufft(M, 2.0, N, N, Nz, kx, ky, kz, prec="d")
     O = orc.SENSE(orc.TimeSegmentation(G, fm, t, M, n, L, interptype=interp),
                   sens.astype(complex).ravel(), M, n, nc)
-    y = A * x
+    P.set_tuning("interp_lds4", 3)
+    try:
+        y, again = A * x, A * x
+    finally:
+        P.set_tuning("interp_lds4", 1)
     orc.set_threads(8)
     try:
         ref = O * x.astype(complex)
     finally:
         orc.set_threads(1)
     assert np.linalg.norm(y - ref) / np.linalg.norm(ref) < TOL
-    assert np.array_equal(y, A * x)  # deterministic
+    assert np.array_equal(y, again)  # deterministic
     # which form ran: the tiled one alone differs in its last bits
     P.set_tuning("interp_lds4", 2)
     try:
@@ -78,6 +84,38 @@ def test_form_independent_of_earlier_calls():
     x, sens = _complex(rng, n), _complex(rng, 32, n)
     G = P.Gnufft(M, 2.0, N, N, 1, kx, ky, np.zeros(M, np.float32))
     A = P.SENSE(P.TimeSegmentation(G, fm, t, M, n, L), sens[:nc], M, n, nc)
-    fresh = A * x
-    P.SENSE(P.TimeSegmentation(G, fm, t, M, n, 8), sens, M, n, 32) * x
-    assert np.array_equal(A * x, fresh)
+    P.set_tuning("interp_lds4", 3)
+    try:
+        fresh = A * x
+        P.SENSE(P.TimeSegmentation(G, fm, t, M, n, 8), sens, M, n, 32) * x
+        again = A * x
+    finally:
+        P.set_tuning("interp_lds4", 1)
+    assert np.array_equal(again, fresh)
+
+
+@pytest.mark.parametrize("N,M,nc,L,interp,patches", [
+    (64, 4096, 17, 8, 1, False), (64, 8192, 8, 8, 1, False), (128, 16384, 8, 8, 2, False),
+    (128, 32768, 8, 8, 1, True), (128, 16384, 16, 6, 1, True), (96, 16384, 32, 12, 2, True)])
+def test_rule(N, M, nc, L, interp, patches):
+    """which form a batch takes by default; both sides of the rule measured"""
+    import powergrid_amd as P
+    rng = np.random.default_rng(7)
+    n = N * N
+    kx, ky = (rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(2))
+    t = np.linspace(1e-3, 9e-3, M).astype(np.float32)
+    fm = rng.uniform(-4000, 4000, n).astype(np.float32)
+    A = P.SENSE(P.TimeSegmentation(P.Gnufft(M, 2.0, N, N, 1, kx, ky, np.zeros(M, np.float32)),
+                                   fm, t, M, n, L, interptype=interp), _complex(rng, nc, n), M, n,
+                nc)
+    x = _complex(rng, n)
+    y = {}
+    try:
+        for form in (3, 2, 1):
+            P.set_tuning("interp_lds4", form)
+            y[form] = A * x
+    finally:
+        P.set_tuning("interp_lds4", 1)
+    assert not np.array_equal(y[3], y[2])
+    assert np.array_equal(y[1], y[3 if patches else 2])
+    assert np.linalg.norm(y[3] - y[2]) / np.linalg.norm(y[2]) < TOL
