@@ -353,7 +353,8 @@ int pg_recon_solve_batch(size_t K, const pg_op* A, const pg_penalty* R, const vo
  * "spread_rows" 1 (default): the 2-D (and z-class plane) spread of a
  * time-segmented batch forms each grid's value from a compact sample row
  * (the nc coil values and L segment weights) instead of reading a row of
- * nc*L values; 0: value rows.  Same products, same order.
+ * nc*L values, unless few coils leave columns of the matrix products empty;
+ * 0: always value rows.  Same products, same order.
  * "trace" 1: tracing ranges (pg_trace_ranges); 0 (default): none.
  * "zfuse" 1 (default): on z-class planes at gridos 2 the adjoint's y IFFT
  * and z stage run as one kernel; 0: two kernels with the class planes in

@@ -395,7 +395,8 @@ def set_tuning(key, value):
     "zclass" 1 (default) builds 3-D plans of stacked trajectories for z-class
     planes, 0 for the full 3-D grid (plans created afterwards); "spread_rows"
     1 (default) spreads time-segmented batches from compact sample rows (coil
-    values and segment weights), 0 from rows of nc*L values; "trace" 1
+    values and segment weights; few coils: value rows), 0 always from rows of
+    nc*L values; "trace" 1
     pushes roctx tracing ranges (trace()); "zfuse" 1 (default) runs the
     adjoint y IFFT and z stage of z-class planes as one kernel;
     "zstage_mfma" 1 (default)

@@ -1087,9 +1087,16 @@ void launch_spread2(const pg::Gnufft& G, const float* rows, int S, int nc, int L
     // Whole rows through LDS where the grids outgrow the caches: written as
     // each lane's 16 bytes, a request each, they keep the L2 busy (4e8 of them
     // at the larger size above: 3.36 against 2.45 ms; 64 grids of 128^2 on 16
-    // planes, 134 MB: 70 against 67 us); below, the barriers cost more (34 MB:
-    // 28.6 against 30.6 us).
-    const int gather = (G.nzc > 0 && pstride ? G.nzc : 1) * (double)B * gsz * 8 > 64e6;
+    // planes, 134 MB: 168 against 161 us for the adjoint); below, the barriers
+    // cost more (34 MB: 28.6 against 30.6 us).  Value rows have the shorter loop
+    // and gain earlier (16 grids of 512^2, 34 MB, 1000 samples: 55.2 against 51.0
+    // us; 64^2 .. 128^2 up to 13 MB: even or 1 us slower).  A single column tile
+    // has fewer requests to save while coils are missing: 1 x 8 on 1024^2, 67 MB,
+    // 90.8 direct, 98.5 gathered; on 16 planes of 128^2 6 x 8, 101 MB, 128 and 136,
+    // 8 x 4, 67 MB, 81 and 85; on 12 planes of 192^2 8 x 4, 113 MB, 128 and 124; on 32
+    // planes of 256^2 7 x 4, 470 MB, 503 and 484.
+    const double bytes = (G.nzc > 0 && pstride ? G.nzc : 1) * (double)B * gsz * 8;
+    const int gather = nc <= 8 ? mode && bytes * nc * nc > 64 * 96e6 : bytes > (mode ? 64e6 : 16e6);
     auto launch = [&](auto kern, int ct, int nseg) {
         const int ncc = (nc + 8 * ct - 1) / (8 * ct), nch = ncc * ((L + nseg - 1) / nseg);
         hipLaunchKernelGGL(kern, dim3((unsigned)(G.n_sblocks * nch)), dim3(64 * kSpreadWaves), 0, s,
@@ -1781,6 +1788,17 @@ int spread_row_floats(const pg::Gnufft& G, int nc, int L, const float* AA, const
     const int B = nc * L;
     if (!g_spread_rows.load(std::memory_order_relaxed) || !AA || L < 2) return 0;
     if (G.geo.dims == 3 && !zclass_active(G, B)) return 0;
+    // Value rows where the compact ones leave columns of the products empty: a
+    // tile of 16 columns holds 8 coils of one segment there, here 8 grids of any.
+    // They are more memory to write and read, so a fifth of the tiles has to be
+    // saved, past 64 grids a third and the values have to stay in the caches.
+    // Adjoint, compact / value rows (us): 1 coil x 8 segments, 512^2, 8192
+    // samples 125 / 91 (101 with a lane per grid), 3 x 5 229 / 183 (197); 128^2,
+    // 32768 samples: 1 x 8 42 / 27, 11 x 5 70 / 62, 9 x 4 (as many tiles) 53.5 / 55.2;
+    // 17 x 12 (53 MB of values) 161 / 146, 192^2, 65536 samples (107 MB) 340 / 356.
+    auto tiles = [](int cols) { return cols <= 8 ? 1 : cols <= 16 ? 2 : 4 * ((cols + 31) / 32); };
+    const int tv = tiles(B), tc = tiles(nc) * L;
+    if (B <= 64 ? 5 * tv <= 4 * tc : 3 * tv <= 2 * tc && 8.0 * G.M * B <= 54e6) return 0;
     const int S = (2 * nc + (AAi ? 2 : 1) * L + 3) & ~3;
     // the rows live in the plan's value buffer (M x B float2) and a block of
     // 64 rows in LDS
