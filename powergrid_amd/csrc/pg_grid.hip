@@ -1406,7 +1406,11 @@ void launch_interp_mm(const pg::Gnufft& G, const float2* grids, long long gsz, l
 // k_spread3_combine.  32 grids of 128^3, 131072 samples on 1024 spokes: 4860 ->
 // 390 us, and 65 us for the parts.  The products themselves take 150 us (128
 // clocks per entry and 32 grids) and the 0.8 GB written 170; the rest is the
-// latency of each patch's first entries at 3 wavefronts per SIMD.  Few grids
+// latency of each patch's first entries at 3 wavefronts per SIMD.  Runs of four
+// patches that no sample meets are stored as whole rows: lane by lane, 32 bytes
+// each, the empty part of a large grid took most of a sparse trajectory's time
+// (16 grids of 128^3, 1024 samples, whole adjoint: 263 us by the kernel before,
+// 390 without the rows, 261 with them).  Few grids
 // (a single NUFFT, density compensation) leave columns empty; they took the
 // atomic spread before: 6 grids of 60^3, 36080 samples, 11.4 ms -> 0.06 ms
 // with the rest of the adjoint.
@@ -1426,7 +1430,7 @@ __global__ void __launch_bounds__(256) k_wpad3(const float* __restrict__ w, int 
 }
 
 template <int NTP, int NCT>
-__global__ void __launch_bounds__(64 * kP3Waves) k_spread3(
+__global__ void __launch_bounds__(64 * kP3Waves, NCT == 4 ? 3 : 4) k_spread3(
     const int4* __restrict__ items, const int2* __restrict__ entries,
     const float* __restrict__ wpad, const float2* __restrict__ V, int B,
     float2* __restrict__ grids, long long G, int Gx, int Gy, int npx, int npy,
@@ -1434,9 +1438,25 @@ __global__ void __launch_bounds__(64 * kP3Waves) k_spread3(
 {
     constexpr int CW = 8 * NCT;  // grids per chunk
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int4 it = items[blockIdx.x * kP3Waves + wv];
-    if (it.x < 0) return;
+    const int4* bi = items + (long long)blockIdx.x * kP3Waves;
     const int b0 = blockIdx.y * CW;
+    bool none = true;
+#pragma unroll
+    for (int w = 0; w < kP3Waves; ++w) none = none && bi[w].y == bi[w].z;
+    if (none) {
+        // patches (along y) that no sample meets: zeros as whole 128-byte rows,
+        // 8 lanes a row, 16 rows (z, x) a grid
+        const int4 me = bi[(threadIdx.x & 7) >> 1];
+        if (me.x < 0) return;
+        const int r = threadIdx.x >> 3 & 15, q = me.x / npx;
+        const long long o = ((long long)((q / npy) * 4 + (r >> 2)) * Gx + (me.x % npx) * 4 + (r & 3)) * Gy +
+                            (q % npy) * 4 + 2 * (threadIdx.x & 1);
+        for (int b = b0 + (int)(threadIdx.x >> 7); b < min(b0 + CW, B); b += kP3Waves / 2)
+            *reinterpret_cast<float4*>(grids + b * G + o) = make_float4(0.f, 0.f, 0.f, 0.f);
+        return;
+    }
+    const int4 it = bi[wv];
+    if (it.x < 0) return;
     const int nf = 2 * min(CW, B - b0);  // floats of the chunk's rows
     const int px = it.x % npx, pr = it.x / npx;
     const int x0 = px * 4, y0 = (pr % npy) * 4, z0 = (pr / npy) * 4;
