@@ -1729,8 +1729,19 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
         return;
     }
     if constexpr (D3 && NT <= 8) {
+        // A tile costs a block and its whole region whatever it holds, and one
+        // or two segments hide little of its loads: where such a batch has more
+        // blocks than run at a time and few samples in each, the gather is the
+        // faster form (a multiple of 8 coils, each on its XCD's L2, somewhat
+        // earlier).  Spokes of 64 samples, tiles / gather in us: 128^3, 256
+        // spokes (2.6 samples a tile) 1 grid 114 / 95, 4 grids 465 / 392, 2 coils x 2
+        // segments 441 / 394, 1 x 4 432 / 451; 64 spokes 2 x 2 359 / 377; 64^3, 64
+        // spokes (4.6) 1 grid 30 / 41, 8 grids 106 / 90, 17 grids 260 / 270; 256 spokes
+        // (7.9) 1 grid 38 / 43, 4 grids 88 / 107, 8 grids 162 / 154.
+        const bool sparse = L <= 2 && (long long)G.n_iitems3 * nc * L >= (L == 1 ? 4096 : 16384) &&
+                            G.M < (nc % 8 ? 6LL : 8LL) * G.n_iitems3;
         // (32-bit byte offsets within a grid)
-        if (G.n_iitems3 > 0 && g.G() * 8 < (1LL << 31)) {
+        if (G.n_iitems3 > 0 && !sparse && g.G() * 8 < (1LL << 31)) {
             const int per = (G.n_iitems3 + 7) / 8;
             auto launch = [&](auto kern) {
                 hipLaunchKernelGGL(kern, dim3((unsigned)(8 * per * nc)), dim3(8 * kI3Chunk), 0, s, G.iitems3,

@@ -1,7 +1,8 @@
 """GPU: gridding on the full 3-D grid (trajectories that are not stacks of
 2-D ones) against the FP64 restatement (oracle): every chunk width of the
 patch spread, patches summed in parts, runs of patches without a sample,
-ragged items, windows past the grid's edges, 6, 8 and 12 taps.
+ragged items, windows past the grid's edges, 6, 8 and 12 taps, and few samples
+on a large grid (the gather).
 
 Tolerance 2e-6: FP32 sums of products of three taps (each rounded, eps = 6e-8)
 and a 3-D FFT, below 1e-6 in relative 2-norm."""
@@ -34,9 +35,9 @@ def _complex(rng, *shape):
     (12, 10, 301, 1, 1, 4.0, 0.0), (12, 10, 301, 4, 2, 4.0, 0.0), (12, 10, 301, 9, 1, 4.0, 0.0),
     (12, 10, 65, 8, 2, 4.0, 0.0), (12, 10, 301, 17, 1, 4.0, 0.0), (12, 10, 301, 33, 1, 4.0, 0.0),
     (10, 4, 97, 13, 5, 3.0, 0.2), (16, 16, 5000, 6, 3, 4.0, 0.5), (16, 16, 9000, 3, 1, 4.0, 0.5),
-    # most patches met by no sample, in every chunk width
+    # most patches met by no sample, in every chunk width; the last two gathered
     (26, 20, 100, 3, 1, 4.0, 0.8), (26, 20, 100, 11, 1, 4.0, 0.8), (26, 20, 100, 7, 5, 4.0, 0.8),
-    (22, 24, 100, 4, 3, 3.0, 0.8)])
+    (22, 24, 100, 4, 3, 3.0, 0.8), (32, 32, 600, 12, 1, 4.0, 0.0), (32, 32, 600, 24, 2, 3.0, 0.0)])
 def test_operator(orc, N, Nz, M, nc, L, width, centre):
     import powergrid_amd as P
     rng = np.random.default_rng(M + nc)
