@@ -1135,6 +1135,7 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
         std::vector<Blk> blk;
         std::vector<int4> comb, parts;
         int nslots = 0;
+        const int part_n = p3_part_entries(cnt[np]);
         auto morton = [](int x, int y, int z) {
             uint64_t k = 0;
             for (int b = 0; b < 20; ++b)
@@ -1156,19 +1157,20 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                         b.w[w] = make_int4(-1, 0, 0, -1);
                         if (y + w >= npy) continue;
                         const int q = (int)(((long long)z * npy + y + w) * npx + x);
-                        const int e0 = (int)cnt[q], n = (int)(cnt[q + 1] - cnt[q]);
-                        if (n > kP3Entries) {
-                            const int np_ = (n + kP3Entries - 1) / kP3Entries;
+                        const long long e0 = cnt[q], n = cnt[q + 1] - cnt[q];
+                        if (n > part_n) {
+                            const int np_ = (int)((n + part_n - 1) / part_n);
                             comb.push_back(make_int4(q, nslots, np_, 0));
-                            for (int k = 0; k < np_; ++k)
-                                parts.push_back(make_int4(q, e0 + (int)((long long)n * k / np_),
-                                                          e0 + (int)((long long)n * (k + 1) / np_),
+                            for (int k = 0; k < np_; ++k) {
+                                const long long a = n * k / np_;
+                                parts.push_back(make_int4(q, (int)(e0 + a), (int)(e0 + n * (k + 1) / np_),
                                                           nslots + k));
+                            }
                             nslots += np_;
                             continue;
                         }
-                        b.w[w] = make_int4(q, e0, e0 + n, -1);
-                        b.work += n;
+                        b.w[w] = make_int4(q, (int)e0, (int)(e0 + n), -1);
+                        b.work += (int)n;
                         any = true;
                     }
                     if (any) blk.push_back(b);
@@ -1176,7 +1178,7 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
         for (size_t k = 0; k < parts.size(); k += 4) {
             Blk b;
             b.key = patch_key(parts[k].x);
-            b.work = 4 * kP3Entries;
+            b.work = 4 * part_n;
             for (size_t w = 0; w < 4; ++w)
                 b.w[w] = k + w < parts.size() ? parts[k + w] : make_int4(-1, 0, 0, -1);
             blk.push_back(b);

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "pg_internal.h"
+#include "pg_worklist.h"
 
 namespace pg {
 
@@ -28,10 +29,6 @@ constexpr int kI3Chunk = 64;  // and for the full 3-D grid
 // for its kIR x kIR region: kIR .. kIR + kI4Pitches - 1
 constexpr int kI4Pitches = 3;
 
-// 3-D spread: entries of a patch summed by one wavefront.  A lone wavefront
-// takes about 500 clocks per 4 entries, so 256 of them (14 us) keep the
-// longest item short against the whole launch
-constexpr int kP3Entries = 256;
 // a sample's padded weights along one dimension: 3 zeros, the taps, zeros
 inline int wpad3_len(int ntaps) { return ntaps > 8 ? 20 : 16; }
 
@@ -119,7 +116,7 @@ struct Gnufft {
     // begin, entry end, slot or -1}, n_items3 of them (a multiple of the
     // block's wavefronts); entries3 holds {sample, where the patch's origin
     // lies in the sample's padded weights: x | y << 10 | z << 20}, comb,
-    // n_comb and n_slots the patches of more than kP3Entries entries, summed
+    // n_comb and n_slots the patches of more than p3_part_entries() entries, summed
     // in parts;
     // wpad3 each sample's weights with zeros around them:
     // wpad3[(3 i + d) wpad3_len + 3 + j] = w_d[j] of sample i

@@ -69,3 +69,25 @@ def test_spatial_interpolation(orc, gridos, width):
                 orc.grid_forward(grid.astype(complex), *geo, gridos, width)) < TOL
     assert _rel(Gg.adjointSpatialInterp(d),
                 orc.grid_adjoint(d.astype(complex), *geo, Gg.grid_size, gridos, width)) < TOL
+
+
+def test_dense_plan(orc):
+    """more than 8.4 million (sample, patch) entries: longer parts, and a
+    workspace of at most 65536 partial patches (16 KB for 32 grids each; one for
+    every 256 entries would be 5.2 GB here)"""
+    import powergrid_amd as P
+    from powergrid_amd import serve
+    rng = np.random.default_rng(11)
+    N, M = 16, 600_000
+    k = [rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(3)]
+    d = _complex(rng, M)
+    Gg = P.Gnufft(M, 2.0, N, N, N, *k)
+    ref = orc.grid_adjoint(d.astype(complex), *k, N, N, N, Gg.grid_size, 2.0, 4.0)
+    assert _rel(Gg.adjointSpatialInterp(d), ref) < TOL
+    del Gg
+    M = 4_000_000
+    k = [rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(3)]
+    free = serve.mem_info()[0]
+    A = P.SENSE(P.Gnufft(M, 2.0, N, N, N, *k), _complex(rng, 8, N ** 3), M, N ** 3, 8)
+    A / np.ones(8 * M, np.complex64)
+    assert free - serve.mem_info()[0] < 4 << 30
