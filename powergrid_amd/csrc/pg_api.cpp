@@ -1098,7 +1098,7 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
             std::vector<long long> pos;
             if (pass == 1) {
                 for (long long q = 0; q < np; ++q) cnt[q + 1] += cnt[q];
-                PG_REQUIRE(cnt[np] < (1ll << 31), PG_ERR_UNSUPPORTED, "too many patch entries");
+                PG_REQUIRE(cnt[np] < kP3MaxEntries, PG_ERR_UNSUPPORTED, "too many patch entries");
                 pos.assign(cnt.begin(), cnt.end() - 1);
                 ent.resize(std::max<long long>(1, cnt[np]));
             }
@@ -1163,13 +1163,13 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                             comb.push_back(make_int4(q, nslots, np_, 0));
                             for (int k = 0; k < np_; ++k) {
                                 const long long a = n * k / np_;
-                                parts.push_back(make_int4(q, (int)(e0 + a), (int)(e0 + n * (k + 1) / np_),
-                                                          nslots + k));
+                                parts.push_back(make_int4(q, p3_y(e0 + a),
+                                                          p3_z(e0 + a, n * (k + 1) / np_ - a), nslots + k));
                             }
                             nslots += np_;
                             continue;
                         }
-                        b.w[w] = make_int4(q, (int)e0, (int)(e0 + n), -1);
+                        b.w[w] = make_int4(q, p3_y(e0), p3_z(e0, n), -1);
                         b.work += (int)n;
                         any = true;
                     }

@@ -112,9 +112,8 @@ struct Gnufft {
     float* dapxy = nullptr;
     int* zcls = nullptr;
     // 3-D plans without z classes (the full 3-D grid): the spread's work items
-    // over 4x4x4 patches (patch x + npx (y + npy z)), {patch or -1, entry
-    // begin, entry end, slot or -1}, n_items3 of them (a multiple of the
-    // block's wavefronts); entries3 holds {sample, where the patch's origin
+    // over 4x4x4 patches (patch x + npx (y + npy z)), packed as pg_worklist.h says,
+    // n_items3 of them (a multiple of the block's wavefronts); entries3 holds {sample, where the patch's origin
     // lies in the sample's padded weights: x | y << 10 | z << 20}, comb,
     // n_comb and n_slots the patches of more than p3_part_entries() entries, summed
     // in parts;

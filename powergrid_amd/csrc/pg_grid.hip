@@ -1385,8 +1385,8 @@ void launch_interp_mm(const pg::Gnufft& G, const float2* grids, long long gsz, l
 
 // ------------------------------------------- 3-D patch spread ------------
 // The full 3-D grid (trajectories that are not stacks of 2-D ones), any
-// number of grids.  A wavefront runs the work item items3[] = {patch (-1:
-// none), entry begin, entry end, slot or -1}: it forms a 4x4x4 patch of up
+// number of grids.  A wavefront runs the work item items3[] (packed as
+// pg_worklist.h says; patch -1: none): it forms a 4x4x4 patch of up
 // to 8 NCT grids as a product on the matrix cores,
 //   acc[64 points][16 NCT floats] += W[64 points][4 entries] V[4 entries][16 NCT floats]
 // four entries a step: per entry the weights wx wy wz of the patch's points,
@@ -1442,7 +1442,7 @@ __global__ void __launch_bounds__(64 * kP3Waves, NCT == 4 ? 3 : 4) k_spread3(
     const int b0 = blockIdx.y * CW;
     bool none = true;
 #pragma unroll
-    for (int w = 0; w < kP3Waves; ++w) none = none && bi[w].y == bi[w].z;
+    for (int w = 0; w < kP3Waves; ++w) none = none && pg::p3_count(bi[w].z) == 0;
     if (none) {
         // patches (along y) that no sample meets: zeros as whole 128-byte rows,
         // 8 lanes a row, 16 rows (z, x) a grid
@@ -1479,12 +1479,13 @@ __global__ void __launch_bounds__(64 * kP3Waves, NCT == 4 ? 3 : 4) k_spread3(
     // group's products; the lanes hold 64 entries at a time and the next 64
     // are requested a stage ahead
     constexpr int U = 2, GE = 4 * U, PER = 64 / GE;
-    const int n = it.z - it.y;
+    const int n = pg::p3_count(it.z);
     const int ng = (n + GE - 1) / GE;
     float wx[2][U], wy[2][U], v[2][U][NCT];
     pg_f4u wz[2][U];
     int2 cur = make_int2(0, 0), nxt = make_int2(0, 0);
-    auto entry = [&](int st) { return entries[it.y + min(64 * st + lane, n - 1)]; };
+    const int2* ent = entries + pg::p3_first(it.y, it.z);
+    auto entry = [&](int st) { return ent[min(64 * st + lane, n - 1)]; };
     auto load_group = [&](int g, int q) {
         if (g % PER == 0) {
             cur = nxt;

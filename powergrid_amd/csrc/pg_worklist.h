@@ -1,6 +1,14 @@
-// pg_worklist.h -- the spread's work lists: how many entries an
-// item of the 3-D list takes.  Plain C++.
+// pg_worklist.h -- the spread's work lists: how an item of the 3-D list is
+// packed.  Plain C++ besides the device attributes.
 #pragma once
+
+#include <cstdint>
+
+#ifdef __HIPCC__
+#define PG_HD __host__ __device__
+#else
+#define PG_HD
+#endif
 
 namespace pg {
 
@@ -15,6 +23,19 @@ inline int p3_part_entries(long long total)
 {
     const long long n = (total + 32767) / 32768;
     return n > kP3Entries ? (int)n : kP3Entries;
+}
+
+// Its items are {patch or -1, y, z, slot or -1} with the first entry and the
+// number of entries in y and z.  A sample has up to 64 entries, so a plan can
+// hold more than 32 bits count: y and the upper 8 bits of z are the first
+// entry, the lower 24 bits of z the number (p3_part_entries() at most).
+constexpr long long kP3MaxEntries = 1LL << 38;
+inline int p3_y(long long first) { return (int)(uint32_t)first; }
+inline int p3_z(long long first, long long n) { return (int)(uint32_t)(n | first >> 32 << 24); }
+PG_HD inline int p3_count(int z) { return z & 0xFFFFFF; }
+PG_HD inline long long p3_first(int y, int z)
+{
+    return (long long)(uint32_t)y | (long long)((uint32_t)z >> 24) << 32;
 }
 
 }  // namespace pg

@@ -1,5 +1,6 @@
 """The host-side work lists of the spread (powergrid_amd/csrc/pg_worklist.h),
-compiled with g++: the partial slots are bounded.  CPU only."""
+compiled with g++: plans of more than 2^31 (sample, patch) entries keep their
+items, and the partial slots are bounded.  CPU only."""
 import os
 import subprocess
 
