@@ -1056,9 +1056,7 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
             }
         {
             // groups are aligned runs of gs wavefronts with one patch and slot
-            // and consecutive ranges; all ranges of a patch tile its entries
-            std::vector<long long> seen(npall, 0);
-            std::vector<char> met(npall, 0);
+            // and consecutive ranges; all ranges tile the patches' entries
             for (size_t blk = 0; blk < nmax * kXcd; ++blk) {
                 const int gs = bgs[blk];
                 for (int w = 0; w < kW; ++w) {
@@ -1066,17 +1064,10 @@ static void gnufft_setup(Gnufft& G, size_t M, float os, size_t Nx, size_t Ny, si
                     const int4 ld = witems[blk * kW + (w / gs) * gs];
                     PG_REQUIRE(it.x == ld.x && it.w == ld.w, PG_ERR_STATE, "spread work groups");
                     if (w % gs) PG_REQUIRE(witems[blk * kW + w - 1].z == it.y, PG_ERR_STATE, "spread work groups");
-                    if (it.x < 0) continue;
-                    PG_REQUIRE(it.x < npall && it.z >= it.y && it.z <= it.y + 64 &&
-                                   it.y >= cnt[it.x] && it.z <= cnt[it.x + 1],
-                               PG_ERR_STATE, "spread work list");
-                    seen[it.x] += it.z - it.y;
-                    met[it.x] = 1;
                 }
             }
-            for (long long q = 0; q < npall; ++q)
-                PG_REQUIRE(met[q] && seen[q] == cnt[q + 1] - cnt[q], PG_ERR_STATE,
-                           "spread work list coverage");
+            PG_REQUIRE(spread_items_tile(witems.data(), witems.size(), cnt, 64), PG_ERR_STATE,
+                       "spread work list coverage");
         }
         G.n_comb = (int)comb.size();
         G.n_slots = nslots;

@@ -1,8 +1,11 @@
 // pg_worklist.h -- the spread's work lists: how an item of the 3-D list is
-// packed.  Plain C++ besides the device attributes.
+// packed, and whether a 2-D list takes every entry once.  Plain C++ besides
+// the device attributes.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
+#include <vector>
 
 #ifdef __HIPCC__
 #define PG_HD __host__ __device__
@@ -36,6 +39,34 @@ PG_HD inline int p3_count(int z) { return z & 0xFFFFFF; }
 PG_HD inline long long p3_first(int y, int z)
 {
     return (long long)(uint32_t)y | (long long)((uint32_t)z >> 24) << 32;
+}
+
+// Whether the 2-D items {patch or -1, first entry, end, slot} hold every
+// entry of patch q, cnt[q] .. cnt[q + 1], once, at most `longest` to an item,
+// and name every patch.  The patches' entries follow each other, so the items
+// lie within their patches and together tile 0 .. cnt[np].
+template <class Item>
+bool spread_items_tile(const Item* items, size_t n, const std::vector<long long>& cnt, int longest)
+{
+    const long long np = (long long)cnt.size() - 1;
+    std::vector<int> step((size_t)cnt[np] + 1, 0);  // changes of the cover count
+    std::vector<char> met((size_t)np, 0);
+    for (size_t k = 0; k < n; ++k) {
+        const Item& it = items[k];
+        if (it.x < 0) continue;
+        if (it.x >= np || it.z < it.y || it.z - it.y > longest || it.y < cnt[it.x] ||
+            it.z > cnt[it.x + 1])
+            return false;
+        ++step[it.y];
+        --step[it.z];
+        met[it.x] = 1;
+    }
+    int cover = 0;
+    for (long long e = 0; e < cnt[np]; ++e)
+        if ((cover += step[e]) != 1) return false;
+    for (char m : met)
+        if (!m) return false;
+    return true;
 }
 
 }  // namespace pg

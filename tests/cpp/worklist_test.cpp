@@ -1,9 +1,14 @@
 // The spread's work lists (pg_worklist.h) on the CPU: the packing of 3-D items
-// over the whole range of entries and the bound on the partial slots.
+// over the whole range of entries, the bound on the partial slots, and the
+// check of a 2-D list against lists that are wrong.
 #include "../../powergrid_amd/csrc/pg_worklist.h"
 
 #include <cstdio>
 #include <initializer_list>
+
+struct Item {
+    int x, y, z, w;
+};
 
 #define CHECK(c)                                              \
     do {                                                      \
@@ -33,6 +38,27 @@ int main()
         // all in one patch, or in patches one entry too heavy
         CHECK((total + t - 1) / t <= 65536 && 2 * (total / (t + 1)) <= 65536);
     }
+    // three patches of 5, 0 and 130 entries, items of up to 64
+    const std::vector<long long> cnt = {0, 5, 5, 135};
+    const std::vector<Item> good = {{2, 69, 102, -1}, {0, 0, 5, -1}, {-1, 0, 0, -1}, {1, 5, 5, -1},
+                                    {2, 5, 69, -1},   {2, 102, 135, -1}};
+    auto ok = [&](const std::vector<Item>& v) {
+        return spread_items_tile(v.data(), v.size(), cnt, 64);
+    };
+    CHECK(ok(good));
+    auto with = [&](size_t k, Item it) {
+        std::vector<Item> v = good;
+        v[k] = it;
+        return v;
+    };
+    CHECK(!ok(with(0, {2, 68, 101, -1})));   // an overlap matched by a gap
+    CHECK(!ok(with(0, {2, 69, 101, -1})));   // a gap
+    CHECK(!ok(with(0, {2, 68, 102, -1})));   // an overlap
+    CHECK(!ok(with(1, {0, 0, 6, -1})));      // past the patch
+    CHECK(!ok(with(1, {-1, 0, 0, -1})));     // a patch's entries missing
+    CHECK(!ok(with(3, {-1, 0, 0, -1})));     // an empty patch without an item
+    CHECK(!ok(with(4, {2, 5, 70, -1})));     // longer than an item may be
+    CHECK(!ok(with(4, {3, 5, 69, -1})));     // no such patch
     std::printf("ok\n");
     return 0;
 }

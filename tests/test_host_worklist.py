@@ -1,6 +1,7 @@
 """The host-side work lists of the spread (powergrid_amd/csrc/pg_worklist.h),
 compiled with g++: plans of more than 2^31 (sample, patch) entries keep their
-items, and the partial slots are bounded.  CPU only."""
+items, the partial slots are bounded, and a list that misses or repeats an
+entry is noticed.  CPU only."""
 import os
 import subprocess
 
