@@ -102,10 +102,23 @@ def mem_info():
     return f.value, t.value
 
 
+def _plainly_stack(req: ReconRequest) -> bool:
+    """whether the plan surely grids a 3-D request on planes, one for each kz"""
+    gy = req.gridos * req.Ny
+    if req.Nz > 128 or gy not in (16, 32, 64, 128, 256, 512, 1024):
+        return False
+    k = len(np.unique(np.asarray(req.kz, np.float32)))
+    return k <= min(128, req.gridos * req.Nz) and k * req.Nz <= 4096
+
+
 def plan_bytes(req: ReconRequest) -> int:
     """Device bytes of the request's Gnufft plan: its batched grids and FFT
     intermediates (B = nc*L grids of the oversampled size), per-sample spread
-    values and tap tables, with a quarter in reserve."""
+    values, tap tables and work lists, and the partial sums of heavy patches,
+    with a quarter in reserve.  A sample meets (taps + 3) / 4 patches per
+    dimension on the average; how many lie in heavy patches is not known here,
+    so the most is taken, and so are the larger lists of a 3-D trajectory that is
+    not plainly a stack."""
     d = 3 if req.Nz > 1 else 2
     G = 1
     for n in (req.Nx, req.Ny, req.Nz if d == 3 else 1):
@@ -115,8 +128,22 @@ def plan_bytes(req: ReconRequest) -> int:
     taps = int(math.ceil(req.kernel_width * req.gridos))
     grids = 8 * B * G * 2  # grids and the FFT intermediates
     vals = 8 * B * M
-    tables = M * (4 * d + 4 * d * taps + 64 * 4)
-    return int(1.25 * (grids + vals + tables))
+    taps_tables = M * (4 * d + 4 * d * taps)
+    # 2-D, and the planes of a stack: 16 patch weights, a sample index and a
+    # place among its sample's for every entry; two interpolation records, the
+    # first place and the plane of every sample; 16 points of every grid for
+    # parts of 256 .. 512 entries
+    e2 = M * ((taps + 3) / 4) ** 2
+    lists = 72 * e2 + 168 * M
+    parts = (128 * B) * (e2 / 256) if e2 > 512 else 0
+    if d == 3 and not _plainly_stack(req):
+        # the full grid: an entry's sample and place, a sample's padded weights
+        # and interpolation record; 64 points of 32 grids for at most 65536 parts
+        # of 128 .. 256 entries or more
+        e3 = M * ((taps + 3) / 4) ** 3
+        lists = max(lists, 8 * e3 + M * (12 * (20 if taps > 8 else 16) + 16))
+        parts = max(parts, 16384 * -(-B // 32) * min(e3 / 128, 65536) if e3 > 256 else 0)
+    return int(1.25 * (grids + vals + taps_tables + lists + parts))
 
 
 def estimate_bytes(req: ReconRequest) -> int:

@@ -200,3 +200,28 @@ def test_serve_reuses_plans_with_the_same_image():
         assert srv.plan_hits == 2
     for r, o in zip(reqs, outs):
         np.testing.assert_array_equal(o.image, alone[r.tag])
+
+
+@pytest.mark.parametrize("N,Nz,M,nc,L,width,raster", [
+    (32, 1, 1_000_000, 1, 1, 4.0, True), (32, 1, 600_000, 4, 2, 6.0, True),
+    (16, 16, 1_000_000, 2, 1, 4.0, False), (16, 16, 500_000, 3, 2, 6.0, False),
+    (24, 16, 800_000, 2, 8, 4.0, True), (32, 16, 800_000, 2, 8, 4.0, True)])
+def test_estimate_covers_the_memory_held(N, Nz, M, nc, L, width, raster):
+    # dense trajectories, whose plan tables and partial sums outweigh the grids
+    print(f"[serve estimate {N} x {N} x {Nz}, {M} samples, {nc} x {L}]", flush=True)
+    rng = np.random.default_rng(M + N)
+    kx, ky = (rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(2))
+    kz = rng.integers(0, Nz, M) - Nz // 2 if raster else rng.uniform(-Nz / 2, Nz / 2, M)
+    n = N * N * Nz
+    r = SV.ReconRequest(kx, ky, kz.astype(np.float32), np.linspace(0, 9e-3, M).astype(np.float32),
+                        N, N, Nz, nc, L, np.linspace(-300, 300, n).astype(np.float32),
+                        np.ones(nc * n, np.complex64), np.ones(nc * M, np.complex64), niter=1,
+                        kernel_width=width)
+    keep = []
+    free = SV.mem_info()[0]
+    SV.run_request(r, P.Stream(), keep)
+    held = free - SV.mem_info()[0]
+    print(f"  held {held / 1e9:.2f} GB, estimate {SV.estimate_bytes(r) / 1e9:.2f} GB")
+    assert held <= SV.estimate_bytes(r)
+    plan = [k for k in keep if isinstance(k, P.Gnufft)]
+    assert len(plan) == 1 and (P.zclasses(plan[0]) > 0) == (raster and Nz > 1)
