@@ -25,6 +25,7 @@
 //            grids of a plan of z-class planes, one thread per sample with
 //            hardware float atomics into a zeroed grid (the reference's
 //            OpenACC spread, gridding.cpp:102-106).
+#include <algorithm>
 #include <cmath>
 
 #include "pg_gnufft.h"
@@ -34,6 +35,19 @@
 namespace {
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return min(max(v, lo), hi); }
+
+// blocks of `threads` threads that one launch can have (its threads in 32 bits)
+constexpr int max_blocks(int threads) { return (int)(((1LL << 32) - 1) / threads); }
+
+// launch(first, count) over a work list of n blocks (a multiple of 8), each
+// `times` times, in runs that one launch can have; every run a multiple of 8
+// blocks, one for each XCD
+template <class F>
+void block_runs(int n, int times, int threads, F launch)
+{
+    const int run = std::max(1, max_blocks(threads) / times / 8) * 8;
+    for (int o = 0; o < n; o += run) launch(o, std::min(run, n - o));
+}
 
 // ---------------------------------------------------------------- interp --
 // Four lanes per sample: lane q of a sample reads the taps q, q+4, q+8 (as
@@ -1099,9 +1113,12 @@ void launch_spread2(const pg::Gnufft& G, const float* rows, int S, int nc, int L
     const int gather = nc <= 8 ? mode && bytes * nc * nc > 64 * 96e6 : bytes > (mode ? 64e6 : 16e6);
     auto launch = [&](auto kern, int ct, int nseg) {
         const int ncc = (nc + 8 * ct - 1) / (8 * ct), nch = ncc * ((L + nseg - 1) / nseg);
-        hipLaunchKernelGGL(kern, dim3((unsigned)(G.n_sblocks * nch)), dim3(64 * kSpreadWaves), 0, s,
-                           G.witems, G.bgs, G.entries, G.ent_w, npy, rows, S, nc, L, ncc, nch, grids,
-                           gsz, g.Gy, partial, B, G.npp, pstride, gather);
+        block_runs(G.n_sblocks, nch, 64 * kSpreadWaves, [&](int o, int n) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)n * nch), dim3(64 * kSpreadWaves), 0, s,
+                               G.witems + (long long)o * kSpreadWaves, G.bgs + o, G.entries, G.ent_w,
+                               npy, rows, S, nc, L, ncc, nch, grids, gsz, g.Gy, partial, B, G.npp,
+                               pstride, gather);
+        });
     };
     // columns for the coils there are, 8, 16 or chunks of 32, and segments for
     // 16 or 32 sums a lane (8 coils: 4 segments at a time measured 26.2 us,
@@ -1363,9 +1380,12 @@ void launch_interp_mm(const pg::Gnufft& G, const float2* grids, long long gsz, l
     const pg::Geometry& g = G.geo;
     const int npy = g.Gy / pg::kPatch, ncc = (nc + w - 1) / w;
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)(G.n_sblocks * ncc * (kSpreadWaves / kIpWaves))),
-                           dim3(64 * kIpWaves), 0, s, G.witems, G.entries, G.ent_w, G.islots, npy, grids, gsz, g.Gy, nc, L, AA,
-                           AAi, G.M, ncc, part, G.npp, pstride);
+        block_runs(G.n_sblocks, ncc, 64 * kSpreadWaves, [&](int o, int n) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)n * ncc * (kSpreadWaves / kIpWaves)),
+                               dim3(64 * kIpWaves), 0, s, G.witems + (long long)o * kSpreadWaves,
+                               G.entries, G.ent_w, G.islots, npy, grids, gsz, g.Gy, nc, L, AA, AAi,
+                               G.M, ncc, part, G.npp, pstride);
+        });
     };
     if (AAi)
         w == 8    ? launch(k_interp_mm<1, true>)
@@ -1745,10 +1765,13 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
         if (G.n_iitems3 > 0 && !sparse && g.G() * 8 < (1LL << 31)) {
             const int per = (G.n_iitems3 + 7) / 8;
             auto launch = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3((unsigned)(8 * per * nc)), dim3(8 * kI3Chunk), 0, s, G.iitems3,
-                                   G.n_iitems3, G.irec3, G.wpad3, G.itx, G.ity, G.ipadl, grids,
-                                   g.G(), g.Gx, g.Gy, g.Gz, nc, L, AA, AAi, G.M, out, out_cstride,
-                                   per);
+                const int cpl = std::max(1, max_blocks(8 * kI3Chunk) / (8 * per));  // coils a launch
+                for (int c = 0; c < nc; c += cpl)
+                    hipLaunchKernelGGL(kern, dim3((unsigned)(8 * per * std::min(cpl, nc - c))),
+                                       dim3(8 * kI3Chunk), 0, s, G.iitems3, G.n_iitems3, G.irec3,
+                                       G.wpad3, G.itx, G.ity, G.ipadl, grids + (long long)c * L * g.G(),
+                                       g.G(), g.Gx, g.Gy, g.Gz, nc, L, AA, AAi, G.M,
+                                       out + c * out_cstride, out_cstride, per);
             };
             AAi ? launch(k_interp3_lds<NT, true>) : launch(k_interp3_lds<NT, false>);
             return;

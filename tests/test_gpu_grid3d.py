@@ -91,3 +91,18 @@ def test_dense_plan(orc):
     A = P.SENSE(P.Gnufft(M, 2.0, N, N, N, *k), _complex(rng, 8, N ** 3), M, N ** 3, 8)
     A / np.ones(8 * M, np.complex64)
     assert free - serve.mem_info()[0] < 4 << 30
+
+
+def test_many_blocks():
+    """more (tile, coil) blocks than one launch can have"""
+    import powergrid_amd as P
+    rng = np.random.default_rng(13)
+    N, M, nc = 8, 2_200_000, 256
+    k = [rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(3)]
+    n = N ** 3
+    G = P.Gnufft(M, 2.0, N, N, N, *k)
+    maps, x = _complex(rng, 4, n), _complex(rng, n)
+    ref = (P.SENSE(G, maps, M, n, 4) * x).reshape(4, M)
+    y = (P.SENSE(G, np.tile(maps, (nc // 4, 1)), M, n, nc) * x).reshape(nc, M)
+    for c in (*range(8), *range(nc - 8, nc)):
+        assert np.array_equal(y[c], ref[c % 4])
