@@ -26,6 +26,7 @@
 //            hardware float atomics into a zeroed grid (the reference's
 //            OpenACC spread, gridding.cpp:102-106).
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 
 #include "pg_gnufft.h"
@@ -1435,7 +1436,8 @@ void launch_interp_mm(const pg::Gnufft& G, const float2* grids, long long gsz, l
 // atomic spread before: 6 grids of 60^3, 36080 samples, 11.4 ms -> 0.06 ms
 // with the rest of the adjoint.
 // Deterministic: entries in sample order, parts in order.  A value that is
-// not finite reaches every point of the patches its window meets.
+// not finite reaches the points of its window alone (a patch's sums are formed
+// again then, so it costs others nothing).
 constexpr int kP3Waves = 4;
 
 template <int NTP>
@@ -1566,6 +1568,40 @@ __global__ void __launch_bounds__(64 * kP3Waves, NCT == 4 ? 3 : 4) k_spread3(
             load_group(g + 2, 0);
             __builtin_amdgcn_sched_barrier(0);
             sum_group(g + 1, 1);
+        }
+    }
+    // A value that is not finite has met weights of zero: the points in the
+    // windows alone, then, an entry at a time
+    bool bad = false;
+#pragma unroll
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int t = 0; t < NCT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bad = bad || !(fabsf(acc[z][t][r]) <= FLT_MAX);
+    if (__builtin_expect(__any(bad), 0)) {
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+#pragma unroll
+            for (int t = 0; t < NCT; ++t) acc[z][t] = pg_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int e = 0; e < n; ++e) {
+            const int2 en = ent[e];
+            const float* wp = wpad + (long long)en.x * (3 * NTP);
+            const float* row = Vf + 2LL * B * en.x;
+            const float wk = wp[(en.y & 1023) + k];
+#pragma unroll
+            for (int t = 0; t < NCT; ++t) {
+                const float w = row[shifted ? (t + 2) % NCT : t];
+#pragma unroll
+                for (int z = 0; z < 4; ++z)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float q = wk * wp[NTP + ((en.y >> 10) & 1023) + r] *
+                                        wp[2 * NTP + (en.y >> 20) + z];
+                        if (q != 0.f) acc[z][t][r] += q * w;
+                    }
+            }
         }
     }
     // lane: points (x0 + k, y0 + r, z0 + z), floats NCT i + t of the chunk

@@ -71,6 +71,27 @@ def test_spatial_interpolation(orc, gridos, width):
                 orc.grid_adjoint(d.astype(complex), *geo, Gg.grid_size, gridos, width)) < TOL
 
 
+@pytest.mark.parametrize("gridos,width", [(2.0, 4.0), (2.0, 3.0), (3.0, 4.0)])
+def test_values_not_finite(orc, gridos, width):
+    """reach the points of their windows alone, in patches summed whole and in
+    parts; the others keep their sums"""
+    import powergrid_amd as P
+    rng = np.random.default_rng(4)
+    N, Nz, M = 12, 8, 1500
+    k = _traj(rng, N, Nz, M, 0.5)
+    d = _complex(rng, M)
+    d[3], d[700], d[1000], d[1300] = np.nan, 1 + 1j * np.inf, -np.inf, 2 + 1j * np.nan
+    Gg = P.Gnufft(M, gridos, N, N, Nz, *k, kernel_width=width)
+    x = Gg.adjointSpatialInterp(d)
+    ref = orc.grid_adjoint(d.astype(complex), *k, N, N, Nz, Gg.grid_size, gridos, width)
+    for a, b in ((x.real, ref.real), (x.imag, ref.imag)):
+        ok = np.isfinite(b)
+        assert 0 < ok.sum() < ok.size
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        assert np.array_equal(a[np.isinf(b)], b[np.isinf(b)])
+        assert _rel(a[ok], b[ok]) < TOL
+
+
 def test_dense_plan(orc):
     """more than 8.4 million (sample, patch) entries: longer parts, and a
     workspace of at most 65536 partial patches (16 KB for 32 grids each; one for
