@@ -909,13 +909,17 @@ __global__ void __launch_bounds__(64 * kSpreadWaves) k_spread2(
         auto sum_group = [&](int s, int q) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                // entries past the end (the last one again): zero weights
-                const float wm = 4 * (s + u) + k < n ? w[q][u] : 0.f;
+                // entries past the end (the last one again): zero weights, and
+                // where a caller may see the grid (MODE 0, few grids) zero
+                // values, for a sample that is infinite
+                const bool in = 4 * (s + u) + k < n;
+                const float wm = in ? w[q][u] : 0.f;
                 float vm[CT];
 #pragma unroll
                 for (int t = 0; t < CT; ++t) {
                     vm[t] = v[q][u][t];
                     if (CT == 4 && t < 2) vm[t] = shifted ? v[q][u][(t + 2) % CT] : vm[t];
+                    if (CT == 1 && MODE == 0) vm[t] = in ? vm[t] : 0.f;
                 }
                 // conj(a + i ai) r: the partner of each float, signed
                 float vx[MODE == 2 ? CT : 1];

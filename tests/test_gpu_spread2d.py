@@ -58,3 +58,21 @@ def test_adjoint(orc, N, M, nc, L, interp, centre):
         orc.set_threads(1)
     assert np.linalg.norm(x - ref) / np.linalg.norm(ref) < TOL
     assert np.array_equal(x, A / y)  # deterministic
+
+
+@pytest.mark.parametrize("M", [300, 301, 302, 303])
+def test_infinite_sample(orc, M):
+    """the spatial spread of an infinite sample is infinite in its window, also
+    where it is the last entry of a patch"""
+    import powergrid_amd as P
+    rng = np.random.default_rng(M)
+    N = 16
+    kx, ky = (rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(2))
+    kz = np.zeros(M, np.float32)
+    d = _complex(rng, M)
+    d[-1], kx[-1], ky[-1] = np.inf + 1j, 0.3, -0.7
+    G = P.Gnufft(M, 2.0, N, N, 1, kx, ky, kz)
+    x = G.adjointSpatialInterp(d).real
+    ref = orc.grid_adjoint(d.astype(complex), kx, ky, kz, N, N, 1, G.grid_size, 2.0, 4.0).real
+    assert np.isinf(ref).sum() == 64
+    assert np.array_equal(x[np.isinf(ref)], ref[np.isinf(ref)])
