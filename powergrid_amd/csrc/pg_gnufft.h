@@ -25,6 +25,9 @@ constexpr int kIR = kIT + 7;  // staged grid region edge (8 taps)
 constexpr int kIChunk = 128;  // samples per interp work item
 constexpr int kIChunk4 = 64;  // the same for the four-segment staging
 constexpr int kI3Chunk = 64;  // and for the full 3-D grid
+// the 2-D interpolation by patches serves plans of this many entries a patch on
+// the average (one group of its products)
+constexpr long long kIpEntries = 16;
 // row pitches (in points) that an item of the four-segment staging may take
 // for its kIR x kIR region: kIR .. kIR + kI4Pitches - 1
 constexpr int kI4Pitches = 3;
@@ -73,7 +76,7 @@ struct Gnufft {
     float* ent_w = nullptr;
     // the transposed use of the same entries (2-D interpolation by patches):
     // entry k's share of its sample is partial sum islots[k], sample i's are
-    // soff[i] .. soff[i + 1], in patch order
+    // soff[i] .. soff[i + 1], in patch order (plans of kIpEntries entries a patch)
     int* islots = nullptr;
     int* soff = nullptr;
     size_t n_entries = 0;

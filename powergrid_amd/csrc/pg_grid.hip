@@ -1914,7 +1914,7 @@ bool interp_mm_possible(const pg::Gnufft& G, int nc, int L, bool aa, size_t part
     if (!aa || !G.islots || nc < 8 || L < 6 || nc * L < 64) return false;
     const size_t patches = (size_t)G.npp * (G.nzc > 0 ? G.nzc : 1);
     const int w = interp_mm_width(nc);
-    return G.n_entries >= 16 * patches && G.n_entries * 2 * ((nc + w - 1) / w * w) <= part_cap;
+    return G.n_entries >= pg::kIpEntries * patches && G.n_entries * 2 * ((nc + w - 1) / w * w) <= part_cap;
 }
 
 // Which of them it is the faster form for.  Against it are a wavefront's
