@@ -946,6 +946,31 @@ def ts_model_error(P, prob, yd, xe, stream, Ls=(8, 16, 32)):
     return out
 
 
+# the keys of the result line: all of CONTRACT, and of BESIDE, in this order,
+# what LINE_MAX characters hold (whoever keeps the end of the output keeps the
+# line); every measurement is on stderr before it
+CONTRACT = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step",
+            "higher_is_better", "scaling", "vs_baseline", "dtype", "data", "config")
+BESIDE = ("recon_latency_ms", "nrmse_vs_fp64_exact_nudft_cg", "nrmse_plain_vs_batched",
+          "plain_iters_per_s", "speedup_vs_plain", "roofline", "cpu_baseline", "speedup_vs_cpu",
+          "exit_reason", "hbm_copy_GBs", "sense2d_iters_per_s")
+LINE_MAX = 1900
+
+
+def result_line(out):
+    """the one JSON line of the results"""
+    sense2d = out.get("sense2d") or {}
+    have = dict(out, sense2d_iters_per_s=sense2d.get("iters_per_s"))
+    line = {k: out[k] for k in CONTRACT}
+    for k in BESIDE:
+        if have.get(k) is None:
+            continue
+        more = dict(line, **{k: have[k]})
+        if len(json.dumps(more)) <= LINE_MAX:
+            line = more
+    return json.dumps(line)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1130,7 +1155,8 @@ def main():
     if not args.no_rows:
         out["rows"] = rows_rates(P, S, stream, with_cpu=not args.no_cpu)
         log(f"[bench] rows {out['rows']}")
-    print(json.dumps(out), flush=True)
+    log(f"[bench] all measurements: {json.dumps(out)}")
+    print(result_line(out), flush=True)
 
 
 if __name__ == "__main__":
