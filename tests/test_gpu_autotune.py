@@ -1,6 +1,6 @@
-"""The autotuner (pg_set_tuning("autotune", 1)): a plan first used for a grid
-count times its interpolation (LDS-staged or gather) and spread (vector units
-or matrix cores) and keeps the faster.  The tuned operator matches the FP64
+"""The autotuner (pg_set_tuning("autotune", 1)): a plan first used for a number
+of coils and segments times its interpolation (gather, LDS-staged tiles or
+patches) and keeps the fastest.  The tuned operator matches the FP64
 restatement at the usual 5e-6, and a tuned PCG matches the default one."""
 import numpy as np
 import pytest
@@ -45,9 +45,8 @@ def test_autotuned_operator_matches_oracle(orc, autotune, N, nshot, ns, nc, L):
     x = S.ellipse_phantom(N, seed=3).astype(np.complex64)
     y = Sg * x
     lds, mfma = P.op_tuning(Sg, nc * L)
-    print(f"  chose interp {['gather', 'lds bins 128', 'lds 4-segment bins 64'][lds]}, "
-          f"spread {'mfma' if mfma else 'valu'}")
-    assert lds in (0, 1, 2) and mfma in (0, 1)
+    print(f"  best tiled form {['gather', 'lds bins 128', 'lds 4-segment bins 64'][lds]}")
+    assert lds in (0, 1, 2) and mfma == 1  # (the spread has one form)
     Gd = orc.Gnufft(M, 2.0, N, N, 1, kx, ky, kz, prec="d")
     Sd = orc.SENSE(orc.TimeSegmentation(Gd, fm, t, M, N * N, L), sens.ravel(), M, N * N, nc)
     if N >= 128:
@@ -79,9 +78,8 @@ def test_autotuned_pcg_matches_default(autotune):
 
 
 def test_autotune_untunable_shape_matches_default():
-    # 3 coils without segments: no LDS interpolation and a grid count that
-    # is not a multiple of 4, so nothing is timed; the zeroed timing
-    # workspaces must not race the first forward/adjoint
+    # 3 coils without segments: no LDS interpolation, so nothing is timed; the
+    # zeroed timing workspaces must not race the first forward/adjoint
     print("[autotune untunable nc=3 L=1]", flush=True)
     N, nc = 64, 3
     kx, ky, kz = S.spiral(N, 8, 512)

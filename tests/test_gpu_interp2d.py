@@ -70,6 +70,36 @@ def test_forward(orc, N, Nz, M, nc, L, interp, centre, patches):
     assert np.array_equal(y, tiled) != patches
 
 
+@pytest.mark.parametrize("M,nc,L,interp,width", [
+    (900, 8, 8, 1, 3.0), (900, 16, 6, 2, 3.0), (600, 8, 8, 1, 6.0), (600, 16, 6, 2, 6.0)])
+def test_widths(orc, M, nc, L, interp, width):
+    """6 taps, and 12, whose windows meet up to 16 patches"""
+    import powergrid_amd as P
+    rng = np.random.default_rng(M + nc)
+    N = 32
+    n = N * N
+    kx, ky = (rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(2))
+    kz = np.zeros(M, np.float32)
+    t = np.linspace(1e-3, 9e-3, M).astype(np.float32)
+    fm = rng.uniform(-4000, 4000, n).astype(np.float32)
+    sens, x = _complex(rng, nc, n), _complex(rng, n)
+    A = P.SENSE(P.TimeSegmentation(P.Gnufft(M, 2.0, N, N, 1, kx, ky, kz, kernel_width=width), fm,
+                                   t, M, n, L, interptype=interp), sens, M, n, nc)
+    G = orc.Gnufft(M, 2.0, N, N, 1, kx, ky, kz, width, prec="d")
+    O = orc.SENSE(orc.TimeSegmentation(G, fm, t, M, n, L, interptype=interp),
+                  sens.astype(complex).ravel(), M, n, nc)
+    y = {}
+    try:
+        for form in (3, 2):
+            P.set_tuning("interp_lds4", form)
+            y[form] = A * x
+    finally:
+        P.set_tuning("interp_lds4", 1)
+    ref = O * x.astype(complex)
+    assert not np.array_equal(y[3], y[2])  # by patches
+    assert np.linalg.norm(y[3] - ref) / np.linalg.norm(ref) < TOL
+
+
 def test_form_independent_of_earlier_calls():
     """a batch whose partial sums do not fit its own share of the plan's
     workspace keeps its form, and so its bits, when a larger batch on the same

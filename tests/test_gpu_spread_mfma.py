@@ -1,8 +1,7 @@
-"""The 2-D batched spread on the matrix cores (pg_set_tuning("spread_mfma", 1),
-k_spread_patch_mfma: 16x16x4 FP32 products of the entries' patch weights and
-their rows of grid values) against the FP64 restatement at 5e-6, on the
-shapes that exercise it: 64 grids (the 2-D SENSE workload), 72 grids (two
-lane chunks) and a dense k-space centre (patches summed in parts)."""
+"""The 2-D batched spread (k_spread2: 16x16x4 FP32 products on the matrix cores
+of the entries' patch weights and their rows) against the FP64 restatement at
+5e-6: 64 grids (the 2-D SENSE workload), 72 grids of nine coils, and a dense
+k-space centre (patches summed in parts)."""
 import numpy as np
 import pytest
 
@@ -19,18 +18,9 @@ def rel(a, b):
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
 
 
-@pytest.fixture
-def mfma():
-    P.set_tuning("spread_mfma", 1)
-    try:
-        yield
-    finally:
-        P.set_tuning("spread_mfma", 0)
-
-
 @pytest.mark.parametrize("N,nshot,ns,nc,L", [(128, 16, 2048, 8, 8), (32, 8, 512, 9, 8),
                                              (32, 16, 2048, 4, 4)])
-def test_spread_matrix_cores_matches_oracle(orc, mfma, N, nshot, ns, nc, L):
+def test_spread_matrix_cores_matches_oracle(orc, N, nshot, ns, nc, L):
     print(f"[spread mfma N={N} grids={nc * L}]", flush=True)
     kx, ky, kz = S.spiral(N, nshot, ns)
     M = len(kx)
