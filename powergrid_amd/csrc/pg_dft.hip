@@ -250,9 +250,9 @@ __global__ void __launch_bounds__(kT) k_gdft_adj(
 // tiles t, which is the A operand A[i][k] of v_mfma_f32_16x16x4f32; column j
 // of the B operand B[k][j] (lane j + 16 k) is float j of input k's row of
 // 16 CT values (8 CT coils, re and im), the second one its neighbour's with
-// the sign.  The phase arithmetic is that of the FP64-free kernels above
-// (the same products, reduced to [-1/2, 1/2] revolutions, v_sin and v_cos)
-// and the sums are FP32.  Per 64 pairs: 16 vector instructions, sine and cosine
+// the sign.  The phase arithmetic is that of precision 0
+// above (FP32, reduced to [-1/2, 1/2] revolutions, v_sin and v_cos) and the
+// sums are FP32.  Per 64 pairs: 16 vector instructions, sine and cosine
 // at a quarter of the rate (88 clocks, the bound), beside 2 CT products of 32
 // clocks on the matrix cores; forming the sums on the vector units took 32 more
 // instructions and 5 LDS broadcasts for 8 coils.

@@ -103,12 +103,14 @@ __host__ __device__ __forceinline__ void dft(float2 (&v)[R])
 // The supported lengths and their factors, f(N, A, B): A a multiple of 4 (the
 // zero-padded or cropped half of a gridos-2 line is then whole entries of the
 // length-A level, see half_live), both near sqrt(N) and at most 28, so that a
-// thread holds at most 56 floats of the line.  The passes serve the gridos-2
+// thread holds at most 56 floats of the line.  The lengths are those of images
+// of even size up to 240 with factors like these; 324, 420, 440 and longer ones
+// that have such factors (500 ... 784) are not listed and take the Stockham form.  The
+// passes serve the gridos-2
 // layout alone: image row i of N/2 at position (i + 3N/4) mod N.
-#define PG_MIX_LENGTHS_SMALL(f)                                                                  \
+#define PG_MIX_LENGTHS(f)                                                                        \
     f(20, 4, 5) f(24, 8, 3) f(28, 4, 7) f(36, 12, 3) f(40, 8, 5) f(44, 4, 11) f(48, 8, 6)       \
-    f(52, 4, 13) f(56, 8, 7) f(60, 12, 5)
-#define PG_MIX_LENGTHS_LARGE(f)                                                                  \
+    f(52, 4, 13) f(56, 8, 7) f(60, 12, 5)                                                        \
     f(72, 12, 6) f(80, 16, 5) f(84, 12, 7) f(88, 8, 11) f(96, 12, 8) f(100, 20, 5)              \
     f(104, 8, 13) f(108, 12, 9) f(112, 16, 7) f(120, 12, 10) f(132, 12, 11) f(140, 20, 7)       \
     f(144, 12, 12) f(156, 12, 13) f(160, 16, 10) f(168, 24, 7) f(176, 16, 11) f(180, 20, 9)     \
@@ -117,7 +119,6 @@ __host__ __device__ __forceinline__ void dft(float2 (&v)[R])
     f(288, 24, 12) f(300, 20, 15) f(308, 28, 11) f(312, 24, 13) f(320, 20, 16) f(336, 24, 14)   \
     f(352, 16, 22) f(360, 24, 15) f(364, 28, 13) f(384, 24, 16) f(392, 28, 14) f(400, 20, 20)   \
     f(416, 16, 26) f(432, 24, 18) f(448, 28, 16) f(480, 24, 20)
-#define PG_MIX_LENGTHS(f) PG_MIX_LENGTHS_SMALL(f) PG_MIX_LENGTHS_LARGE(f)
 
 template <int R1, int R2>
 constexpr int line_threads()

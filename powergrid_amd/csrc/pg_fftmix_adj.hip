@@ -7,11 +7,7 @@
 namespace {
 
 // lines (columns x segments) of a block
-template <int R1, int R2>
-constexpr int post_lines()
-{
-    return 8;
-}
+constexpr int kPostLines = 8;
 
 // The adjoint tail of image column col and coil c: for every segment l the
 // IFFT along y of column col of grid c L + l (ifftshift on load), the Ny
@@ -22,7 +18,7 @@ constexpr int post_lines()
 // entries, so half of level 2 and of the weights drop out and a thread's
 // running sums are R2 / 2 points.  Bound by the read of T.
 template <int R1, int R2>
-__global__ void __launch_bounds__((pgm::line_threads<R1, R2>() * post_lines<R1, R2>()))
+__global__ void __launch_bounds__((pgm::line_threads<R1, R2>() * kPostLines))
     k_adj_post_mix(const float2* __restrict__ T, const float2* __restrict__ S,
                    const float2* __restrict__ WoH, const float* __restrict__ dap, int ncol, int L,
                    int npc, int ng, const float2* __restrict__ tw, float2* __restrict__ out,
@@ -32,7 +28,7 @@ __global__ void __launch_bounds__((pgm::line_threads<R1, R2>() * post_lines<R1, 
     constexpr int P = pgm::row_pitch<R2>();
     constexpr int H = R2 / 2;  // image rows per thread: y = t + R1 i
     static_assert(R2 % 4 == 0, "gridos-2 layout");
-    __shared__ float2 lds[post_lines<R1, R2>() * R1 * P];
+    __shared__ float2 lds[kPostLines * R1 * P];
     const int t = threadIdx.x % TL, ln = threadIdx.x / TL;
     const int g = ln / npc, jl = ln - g * npc;
     const int c = blockIdx.y;
@@ -112,7 +108,7 @@ template <int R1, int R2>
 void launch(const float2* T, const float2* S, const float2* WoH, const float* dap, int ncol, int nc,
             int L, const float2* tw, float2* out, long long out_cstride, hipStream_t s)
 {
-    constexpr int TL = pgm::line_threads<R1, R2>(), NL = post_lines<R1, R2>();
+    constexpr int TL = pgm::line_threads<R1, R2>(), NL = kPostLines;
     // as many segments in flight as a block holds, in equal rounds (12
     // segments: 6 + 6), then columns up to two wavefronts
     const int rounds = (L + NL - 1) / NL;

@@ -5,8 +5,8 @@
 namespace {
 
 // lines per block: consecutive inner indices, so that every global access is
-// a run of that many points.  32 (256 bytes) while the block's rows stay
-// within 40 KB of LDS and 512 threads, else 16.
+// a run of that many points.  32 (256 bytes) up to length 144, where the block's
+// rows stay within 40 KB of LDS (512 threads at most, 640 at 100 and 140), else 16.
 template <int N>
 constexpr int lpb()
 {

@@ -5,14 +5,16 @@
 // clamped window of gridding.cpp:67-73 carry weight 0 and their addresses
 // are clamped into the grid, so no tap wraps around.
 //
-// interp  -- 2-D with 2..16 segments: the grid region under a tile of
-//            samples is staged in LDS for all segments of a coil and each
-//            sample is one wavefront (lane = segment x y-tap).  Otherwise
-//            four lanes per (sample, coil) gather from global memory.  In
-//            both, the L segment grids of a coil are read with the same
-//            weights and summed with the AA weights (TimeSegmentation.cpp:
-//            279-295), and coils are mapped to XCDs so that each XCD's L2
-//            holds its coils' grids.
+// interp  -- 2-D, large batches: by 4x4 grid patches on the matrix cores, the
+//            samples' shares added in a second pass (k_interp_mm).  2-D with
+//            2..16 segments otherwise: the grid region under a tile of
+//            samples is staged in LDS for all or four segments of a coil.
+//            3-D: the region under an 8^3 tile, a segment at a time
+//            (k_interp3_lds).  Else four lanes per (sample, coil) gather from
+//            global memory.  In all, the L segment grids of a coil are read
+//            with the same weights and summed with the AA weights
+//            (TimeSegmentation.cpp:279-295); the staged forms map coils to
+//            XCDs so that each XCD's L2 holds its coils' grids.
 // spread  -- first the value of every (sample, grid) pair is formed once
 //            (AA weight, CG residual), sample-major.
 //            2-D: 4x4 grid patches as products on the matrix cores (patch
@@ -539,8 +541,8 @@ __global__ void __launch_bounds__(kI4Threads, CPX ? 6 : 7) k_interp_lds4(
 // Measured on 32 grids of 128^3, 131072 samples on 1024 spokes: 2130 us for
 // the gather kernel above (four lanes per sample: 16 cache lines per load),
 // 1830 us for a wavefront per sample gathering 8 rows of 64 bytes per load,
-// 680 us here.  Bound by the LDS reads (43% of its time with their bank
-// conflicts) and the vector units (36%) in turn.
+// 690 us here.  Bound by the LDS, busy for 71% of the time (27% in bank
+// conflicts), beside the vector units' 41%.
 using pg::kI3Chunk;
 
 template <int NT, bool CPX>
@@ -1328,8 +1330,8 @@ __global__ void __launch_bounds__(64 * kIpWaves) k_interp_mm(
 
 // the samples' sums over their slots soff[i] .. soff[i + 1], in slot order:
 // block of 32 samples, lanes over the coils (contiguous), the sums turned
-// through LDS into runs of samples.  PLANAR: a chunk's 8 re, then 8 im.
-// PLANAR: one chunk of 8 re, then 8 im; else a chunk's coils in pairs of floats.
+// through LDS into runs of samples.  PLANAR: one chunk of 8 re, then 8 im; else
+// a chunk's coils in pairs of floats.
 template <bool PLANAR>
 __global__ void __launch_bounds__(256) k_interp_sum(const int* __restrict__ soff,
                                                     const float* __restrict__ part, int nc, int rf,
@@ -1375,7 +1377,8 @@ __global__ void __launch_bounds__(256) k_interp_sum(const int* __restrict__ soff
                        : make_float2(buf[2 * co][so], buf[2 * co + 1][so]);
 }
 
-// the coil columns of a chunk (the widest that the coils fill)
+// the coil columns of a chunk: one chunk for up to 32 coils (9 or 17 fill about
+// half of it), chunks of 32 for more
 int interp_mm_width(int nc) { return nc <= 8 ? 8 : nc <= 16 ? 16 : 32; }
 
 void launch_interp_mm(const pg::Gnufft& G, const float2* grids, long long gsz, long long pstride,
