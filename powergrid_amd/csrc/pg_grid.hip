@@ -27,7 +27,6 @@
 //            grids of a plan of z-class planes, one thread per sample with
 //            hardware float atomics into a zeroed grid (the reference's
 //            OpenACC spread, gridding.cpp:102-106).
-#include <algorithm>
 #include <cfloat>
 #include <cmath>
 
@@ -38,19 +37,6 @@
 namespace {
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return min(max(v, lo), hi); }
-
-// blocks of `threads` threads that one launch can have (its threads in 32 bits)
-constexpr int max_blocks(int threads) { return (int)(((1LL << 32) - 1) / threads); }
-
-// launch(first, count) over a work list of n blocks (a multiple of 8), each
-// `times` times, in runs that one launch can have; every run a multiple of 8
-// blocks, one for each XCD
-template <class F>
-void block_runs(int n, int times, int threads, F launch)
-{
-    const int run = std::max(1, max_blocks(threads) / times / 8) * 8;
-    for (int o = 0; o < n; o += run) launch(o, std::min(run, n - o));
-}
 
 // ---------------------------------------------------------------- interp --
 // Four lanes per sample: lane q of a sample reads the taps q, q+4, q+8 (as
@@ -1120,7 +1106,7 @@ void launch_spread2(const pg::Gnufft& G, const float* rows, int S, int nc, int L
     const int gather = nc <= 8 ? mode && bytes * nc * nc > 64 * 96e6 : bytes > (mode ? 64e6 : 16e6);
     auto launch = [&](auto kern, int ct, int nseg) {
         const int ncc = (nc + 8 * ct - 1) / (8 * ct), nch = ncc * ((L + nseg - 1) / nseg);
-        block_runs(G.n_sblocks, nch, 64 * kSpreadWaves, [&](int o, int n) {
+        pg::block_runs(G.n_sblocks, nch, 64 * kSpreadWaves, [&](int o, int n) {
             hipLaunchKernelGGL(kern, dim3((unsigned)n * nch), dim3(64 * kSpreadWaves), 0, s,
                                G.witems + (long long)o * kSpreadWaves, G.bgs + o, G.entries, G.ent_w,
                                npy, rows, S, nc, L, ncc, nch, grids, gsz, g.Gy, partial, B, G.npp,
@@ -1388,7 +1374,7 @@ void launch_interp_mm(const pg::Gnufft& G, const float2* grids, long long gsz, l
     const pg::Geometry& g = G.geo;
     const int npy = g.Gy / pg::kPatch, ncc = (nc + w - 1) / w;
     auto launch = [&](auto kern) {
-        block_runs(G.n_sblocks, ncc, 64 * kSpreadWaves, [&](int o, int n) {
+        pg::block_runs(G.n_sblocks, ncc, 64 * kSpreadWaves, [&](int o, int n) {
             hipLaunchKernelGGL(kern, dim3((unsigned)n * ncc * (kSpreadWaves / kIpWaves)),
                                dim3(64 * kIpWaves), 0, s, G.witems + (long long)o * kSpreadWaves,
                                G.entries, G.ent_w, G.islots, npy, grids, gsz, g.Gy, nc, L, AA, AAi,
@@ -1764,19 +1750,24 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
         // (its staging and weight offsets are 32-bit byte offsets)
         if (G.n_iitems4 > 0 && four && gsz * 4 * 8 < (1LL << 31) &&
             (long long)L * G.M * 4 < (1LL << 31)) {
-            const dim3 grid((unsigned)G.n_iitems4 * nc), block(kI4Threads);
             auto launch = [&](auto kern) {
-                hipLaunchKernelGGL(kern, grid, block, 0, s, G.iitems4, G.irec4, G.ity, G.ipadl,
-                                   grids, gsz, g.Gx, g.Gy, nc, L, AA, AAi, G.M, out, out_cstride,
-                                   pstride);
+                pg::coil_runs(nc, G.n_iitems4, kI4Threads, [&](int c, int n) {
+                    hipLaunchKernelGGL(kern, dim3((unsigned)G.n_iitems4 * n), dim3(kI4Threads), 0, s,
+                                       G.iitems4, G.irec4, G.ity, G.ipadl, grids + c * L * gsz, gsz,
+                                       g.Gx, g.Gy, n, L, AA, AAi, G.M, out + c * out_cstride,
+                                       out_cstride, pstride);
+                });
             };
             AAi ? launch(k_interp_lds4<true>) : launch(k_interp_lds4<false>);
             return;
         }
-        const dim3 grid((unsigned)G.n_iitems * nc), block(64 * kInterpWaves);
         auto launch = [&](auto kern) {
-            hipLaunchKernelGGL(kern, grid, block, 0, s, G.iitems, G.irec, G.ity, G.ipadl, grids,
-                               gsz, g.Gx, g.Gy, nc, L, AA, AAi, G.M, out, out_cstride, pstride);
+            pg::coil_runs(nc, G.n_iitems, 64 * kInterpWaves, [&](int c, int n) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)G.n_iitems * n), dim3(64 * kInterpWaves), 0,
+                                   s, G.iitems, G.irec, G.ity, G.ipadl, grids + c * L * gsz, gsz,
+                                   g.Gx, g.Gy, n, L, AA, AAi, G.M, out + c * out_cstride,
+                                   out_cstride, pstride);
+            });
         };
         if (L <= 8)
             AAi ? launch(k_interp_lds<8, true>) : launch(k_interp_lds<8, false>);
@@ -1785,13 +1776,15 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
         return;
     }
     const int nsb = (G.M + 63) / 64;  // 64 samples (4 lanes each) per block
-    const int xmap = (nc % 8 == 0) ? 1 : 0;
-    if (planes) {
-        hipLaunchKernelGGL((k_interp<NT, false>), dim3(nsb * nc), dim3(256), 0, s, G.lo, G.w, G.M,
-                           g.Gx, g.Gy, 1, grids, gsz, nc, L, AA, AAi, out, out_cstride, nsb, xmap,
-                           (const int*)G.zcls, pstride);
-        return;
-    }
+    auto gather = [&](auto kern, int Gz, const int* zcls) {
+        pg::coil_runs(nc, nsb, 256, [&](int c, int n) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)nsb * n), dim3(256), 0, s, G.lo, G.w, G.M, g.Gx,
+                               g.Gy, Gz, grids + c * L * gsz, gsz, n, L, AA, AAi,
+                               out + c * out_cstride, out_cstride, nsb, n % 8 == 0 ? 1 : 0, zcls,
+                               pstride);
+        });
+    };
+    if (planes) return gather(k_interp<NT, false>, 1, G.zcls);
     if constexpr (D3 && NT <= 8) {
         // A tile costs a block and its whole region whatever it holds, and one
         // or two segments hide little of its loads: where such a batch has more
@@ -1808,21 +1801,18 @@ void interp_dispatch(const pg::Gnufft& G, const float2* grids, int nc, int L, co
         if (G.n_iitems3 > 0 && !sparse && g.G() * 8 < (1LL << 31)) {
             const int per = (G.n_iitems3 + 7) / 8;
             auto launch = [&](auto kern) {
-                const int cpl = std::max(1, max_blocks(8 * kI3Chunk) / (8 * per));  // coils a launch
-                for (int c = 0; c < nc; c += cpl)
-                    hipLaunchKernelGGL(kern, dim3((unsigned)(8 * per * std::min(cpl, nc - c))),
-                                       dim3(8 * kI3Chunk), 0, s, G.iitems3, G.n_iitems3, G.irec3,
-                                       G.wpad3, G.itx, G.ity, G.ipadl, grids + (long long)c * L * g.G(),
-                                       g.G(), g.Gx, g.Gy, g.Gz, nc, L, AA, AAi, G.M,
-                                       out + c * out_cstride, out_cstride, per);
+                pg::coil_runs(nc, 8 * per, 8 * kI3Chunk, [&](int c, int n) {
+                    hipLaunchKernelGGL(kern, dim3((unsigned)(8 * per * n)), dim3(8 * kI3Chunk), 0, s,
+                                       G.iitems3, G.n_iitems3, G.irec3, G.wpad3, G.itx, G.ity,
+                                       G.ipadl, grids + c * L * gsz, gsz, g.Gx, g.Gy, g.Gz, n, L, AA,
+                                       AAi, G.M, out + c * out_cstride, out_cstride, per);
+                });
             };
             AAi ? launch(k_interp3_lds<NT, true>) : launch(k_interp3_lds<NT, false>);
             return;
         }
     }
-    hipLaunchKernelGGL((k_interp<NT, D3>), dim3(nsb * nc), dim3(256), 0, s, G.lo, G.w, G.M, g.Gx,
-                       g.Gy, g.Gz, grids, g.G(), nc, L, AA, AAi, out, out_cstride, nsb, xmap,
-                       (const int*)nullptr, 0LL);
+    gather(k_interp<NT, D3>, g.Gz, nullptr);
 }
 
 template <int NT, bool D3>

@@ -1,6 +1,6 @@
-// pg_worklist.h -- the spread's work lists: how an item of the 3-D list is
-// packed, and whether a 2-D list takes every entry once.  Plain C++ besides
-// the device attributes.
+// pg_worklist.h -- the gridding's work lists: how an item of the 3-D spread's
+// list is packed, whether a 2-D list takes every entry once, and how lists go
+// in launches.  Plain C++ besides the device attributes.
 #pragma once
 
 #include <cstddef>
@@ -67,6 +67,31 @@ bool spread_items_tile(const Item* items, size_t n, const std::vector<long long>
     for (char m : met)
         if (!m) return false;
     return true;
+}
+
+// blocks of `threads` threads that one launch can have (its threads in 32
+// bits: with more, a part of them runs and no error is given)
+constexpr int max_blocks(int threads) { return (int)(((1LL << 32) - 1) / threads); }
+
+// launch(first, count) over a work list of n blocks (a multiple of 8), each
+// `times` times, in runs that one launch can have; every run a multiple of 8
+// blocks, one for each XCD
+template <class F>
+void block_runs(int n, int times, int threads, F launch)
+{
+    const int fit = max_blocks(threads) / times / 8 * 8;
+    const int run = fit > 8 ? fit : 8;
+    for (int o = 0; o < n; o += run) launch(o, n - o < run ? n - o : run);
+}
+
+// the same over nc coils of `blocks` blocks each; a multiple of 8 coils at a
+// time, which keep their XCDs, where that many fit
+template <class F>
+void coil_runs(int nc, long long blocks, int threads, F launch)
+{
+    const long long fit = max_blocks(threads) / blocks;
+    const int run = fit >= nc ? nc : fit >= 8 ? (int)(fit / 8 * 8) : fit > 1 ? (int)fit : 1;
+    for (int c = 0; c < nc; c += run) launch(c, nc - c < run ? nc - c : run);
 }
 
 }  // namespace pg

@@ -1,6 +1,6 @@
 // The spread's work lists (pg_worklist.h) on the CPU: the packing of 3-D items
-// over the whole range of entries, the bound on the partial slots, and the
-// check of a 2-D list against lists that are wrong.
+// over the whole range of entries, the bound on the partial slots, the check
+// of a 2-D list against lists that are wrong, and the runs of launches.
 #include "../../powergrid_amd/csrc/pg_worklist.h"
 
 #include <cstdio>
@@ -59,6 +59,30 @@ int main()
     CHECK(!ok(with(3, {-1, 0, 0, -1})));     // an empty patch without an item
     CHECK(!ok(with(4, {2, 5, 70, -1})));     // longer than an item may be
     CHECK(!ok(with(4, {3, 5, 69, -1})));     // no such patch
+    // runs of at most 2^32 - 1 threads that take every block once, in order
+    for (int threads : {256, 512})
+        for (int times : {1, 7, 96, 1 << 20})
+            for (int n : {8, 4096, 1 << 20, (1 << 24) + 8}) {
+                long long next = 0;
+                bool good = true;
+                block_runs(n, times, threads, [&](int o, int k) {
+                    good = good && o == next && k > 0 && k % 8 == 0 &&
+                           ((long long)k * times * threads < 1LL << 32 || k == 8);
+                    next = o + k;
+                });
+                CHECK(good && next == n);
+            }
+    for (int threads : {256, 512})
+        for (long long blocks : {1LL, 35000LL, 300000LL, 1LL << 22})
+            for (int nc : {1, 3, 8, 37, 512, 100000}) {
+                long long next = 0;
+                bool good = true;
+                coil_runs(nc, blocks, threads, [&](int c, int k) {
+                    good = good && c == next && k > 0 && k * blocks * threads < 1LL << 32;
+                    next = c + k;
+                });
+                CHECK(good && next == nc);
+            }
     std::printf("ok\n");
     return 0;
 }

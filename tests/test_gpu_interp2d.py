@@ -149,3 +149,31 @@ def test_rule(N, M, nc, L, interp, patches):
     assert not np.array_equal(y[3], y[2])
     assert np.array_equal(y[1], y[3 if patches else 2])
     assert np.linalg.norm(y[3] - y[2]) / np.linalg.norm(y[2]) < TOL
+
+
+@pytest.mark.parametrize("L", [1, 2, 4])
+def test_many_blocks(L):
+    """more (block of samples, coil) blocks than one launch can have: the
+    gather, and tiles of all and of four segments"""
+    import ctypes as C
+
+    import powergrid_amd as P
+    from powergrid_amd._lib import check, lib
+    rng = np.random.default_rng(17)
+    N, M, nc = 8, 2_200_000, 512
+    n = N * N
+    kx, ky = (rng.uniform(-N / 2, N / 2, M).astype(np.float32) for _ in range(2))
+    G = P.Gnufft(M, 2.0, N, N, 1, kx, ky, np.zeros(M, np.float32))
+    if L > 1:
+        t = np.linspace(1e-3, 9e-3, M).astype(np.float32)
+        G = P.TimeSegmentation(G, rng.uniform(-700, 700, n).astype(np.float32), t, M, n, L)
+    maps, x = _complex(rng, 4, n), _complex(rng, n)
+    ref = (P.SENSE(G, maps, M, n, 4) * x).reshape(4, M)
+    out = P.DeviceArray(nc * M)
+    A = P.SENSE(G, np.tile(maps, (nc // 4, 1)), M, n, nc)
+    A.forward(P.DeviceArray.from_host(x), out=out)
+    y = np.empty(M, np.complex64)
+    for c in (0, 1, 250, 490, 510, 511):
+        check(lib().pg_memcpy_dtoh(y.ctypes.data_as(C.c_void_p),
+                                   C.c_void_p(out.ptr.value + 8 * M * c), 8 * M, None))
+        assert np.array_equal(y, ref[c % 4])

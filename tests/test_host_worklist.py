@@ -1,7 +1,7 @@
-"""The host-side work lists of the spread (powergrid_amd/csrc/pg_worklist.h),
+"""The host-side work lists of the gridding (powergrid_amd/csrc/pg_worklist.h),
 compiled with g++: plans of more than 2^31 (sample, patch) entries keep their
-items, the partial slots are bounded, and a list that misses or repeats an
-entry is noticed.  CPU only."""
+items, the partial slots are bounded, a list that misses or repeats an entry
+is noticed, and no launch has 2^32 threads.  CPU only."""
 import os
 import subprocess
 
